@@ -92,6 +92,14 @@ struct DevModel {
     const double* hcoef;
     int32_t hadj_beg[2], hadj_end[2], hfeat_beg[2], hfeat_end[2];
     int lmaxh, n_lmhh;
+    // merged rows of the linear order-5/6 families per centre species: rows
+    // hrow[hrow_beg[t] .. hrow_end[t]), term codes from hrterm + hrt_off[t]
+    // (hrt_num[t] of them), coefficients hrcoef[hrc_off[t] + n hrt_num[t] + term]
+    const HiRow* hrow;
+    const int32_t* hrterm;
+    const double* hrcoef;
+    int32_t hrow_beg[2], hrow_end[2], hrt_off[2], hrt_num[2], hrc_off[2];
+    int hi_split;           // 1: rows scaled by 1 / order (the per-atom energy split)
 };
 
 // order-1/2 adjoint row L runs inside the order-3/4 kernel

@@ -284,6 +284,27 @@ bool upload_model(mlip_ctx* c) {
         dm.hvis = c->d_hvis.p;
         dm.hterm = c->d_hterm.p;
         dm.hcoef = c->d_hcoef.p;
+        std::vector<HiRow> hr;
+        std::vector<int32_t> hrt;
+        std::vector<double> hrc;
+        for (int t = 0; t < m.n_type && t < 2; ++t) {
+            const TypeTables& tt = m.types[t];
+            dm.hrow_beg[t] = static_cast<int32_t>(hr.size());
+            hr.insert(hr.end(), tt.hi_rows.begin(), tt.hi_rows.end());
+            dm.hrow_end[t] = static_cast<int32_t>(hr.size());
+            dm.hrt_off[t] = static_cast<int32_t>(hrt.size());
+            dm.hrt_num[t] = static_cast<int32_t>(tt.hi_rterm.size());
+            hrt.insert(hrt.end(), tt.hi_rterm.begin(), tt.hi_rterm.end());
+            dm.hrc_off[t] = static_cast<int32_t>(hrc.size());
+            hrc.insert(hrc.end(), tt.hi_rcoef.begin(), tt.hi_rcoef.end());
+        }
+        if (!upload(c, c->d_hrow, hr.data(), hr.size(), "order-5/6 rows") ||
+            !upload(c, c->d_hrterm, hrt.data(), hrt.size(), "order-5/6 row terms") ||
+            !upload(c, c->d_hrcoef, hrc.data(), hrc.size(), "order-5/6 row coefficients"))
+            return false;
+        dm.hrow = c->d_hrow.p;
+        dm.hrterm = c->d_hrterm.p;
+        dm.hrcoef = c->d_hrcoef.p;
         dm.lmaxh = m.lmaxh;
         dm.n_lmhh = n_lmh_of(m.lmaxh);
     } else {
@@ -706,6 +727,7 @@ bool run_atom_split(mlip_ctx* c, double* epv, double* evat) {
         run("pair_model_energy", launch_pair_model_energy(me, se, epv, st));
     } else {
         me.weight = c->d_weight_e.p;
+        me.hi_split = 1;
         se.H = se.Hq;
         if (me.n_p > 0) run("poly_split", launch_poly_split(me, se, st));
         if (ok) run("q12_split", launch_q12(me, se, false, st));
@@ -1013,6 +1035,9 @@ void mlip_destroy(mlip_ctx* c) {
     c->d_hvis.release();
     c->d_hterm.release();
     c->d_hcoef.release();
+    c->d_hrow.release();
+    c->d_hrterm.release();
+    c->d_hrcoef.release();
     drop_graph(c);
     pool_free(c);
     nb_free(c);
@@ -1626,6 +1651,7 @@ int mlip_flops(const mlip_ctx* c, double* out7) {
         };
         out7[2] += na * hi_terms(tt.hi_feat, false);
         out7[3] += na * hi_terms(tt.hi_adj, true);
+        for (const HiRow& r : tt.hi_rows) out7[3] += na * ((r.tend - r.tbeg) * (6.0 * (r.order - 2) + 4.0) + 10.0);
         const double np = m.n_p, w = static_cast<double>(m.prange[t][1] - m.prange[t][0]) * m.n_fn;
         out7[4] += static_cast<double>(c->owners_per_type[t]) * (np > 0 ? 2.0 * w * w + 6.0 * w + 12.0 * m.c3_w.size() / np : 0.0);
     }

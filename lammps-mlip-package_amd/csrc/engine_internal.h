@@ -69,8 +69,9 @@ struct mlip_ctx {
     mlip::DBuf<int32_t> d_phoff, d_zlist;
     mlip::DBuf<mlip::PairHEntry> d_phent;
     mlip::DBuf<mlip::VisitHi> d_hvis;
-    mlip::DBuf<int32_t> d_hterm;
-    mlip::DBuf<double> d_hcoef;
+    mlip::DBuf<int32_t> d_hterm, d_hrterm;
+    mlip::DBuf<double> d_hcoef, d_hrcoef;
+    mlip::DBuf<mlip::HiRow> d_hrow;
     mlip::DevModel dm{};
     // structure buffers
     mlip::DBuf<double> x, pshift, A, G, D, Hq, H, Ep, Eq12, Eq34, gpair, vown, f, e_slot, red, out;

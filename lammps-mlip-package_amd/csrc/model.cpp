@@ -515,6 +515,8 @@ void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<i
     std::vector<std::vector<VisitQ12>> by_l(m.maxl + 1);
     using Pending = PlanVisit;
     std::vector<Pending> adj, feat;
+    // merged order-5/6 rows: (S, L, k, order) -> product -> coefficient per n
+    std::map<std::array<int, 4>, std::map<std::vector<int>, std::vector<double>>> hi_merge;
     auto push_coef = [&](double v) { m.coef.push_back(v); };
     for (int i = 0; i < m.n_gtinv; ++i) {
         const Itc& it = m.itcs[i];
@@ -603,6 +605,22 @@ void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<i
                     w.tend = static_cast<int32_t>(m.hi_term.size());
                     return w;
                 };
+                if (pslot < 0) {
+                    // linear family: its weights are the same for every
+                    // centre, so its terms join the merged rows
+                    const int nl = (m.lmaxh + 1) * (m.lmaxh + 1);
+                    for (size_t ti = 0; ti < ir.m.size(); ++ti) {
+                        const std::vector<int>& mt = ir.m[ti];
+                        if (mt[p] > 0) continue;  // outputs m <= 0 only
+                        std::vector<int> prod;
+                        for (int k : oth) prod.push_back(sp[k] * nl + ir.l[k] * ir.l[k] + ir.l[k] + mt[k]);
+                        std::sort(prod.begin(), prod.end());
+                        std::vector<double>& w = hi_merge[{v.S, v.L, -mt[p], q}][prod];
+                        w.resize(m.n_fn, 0.0);
+                        for (int n = 0; n < m.n_fn; ++n) w[n] += m.weight[n * m.n_gtinv + i] * ir.c[ti];
+                    }
+                    continue;
+                }
                 tt.hi_adj.push_back(emit_terms(false));
                 if (p == 0 && pslot >= 0) tt.hi_feat.push_back(emit_terms(true));
             }
@@ -691,6 +709,26 @@ void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<i
                 feat.push_back({sp[p], L, f, cost, static_cast<int>(m.coef.size()) - f.coef});
             }
         }
+    }
+    {
+        std::vector<const std::vector<double>*> cols;
+        for (const auto& row : hi_merge) {
+            HiRow r{row.first[0], row.first[1], row.first[2], row.first[3], static_cast<int32_t>(cols.size()), 0, 0};
+            if (!tt.hi_rows.empty()) {
+                const HiRow& q = tt.hi_rows.back();
+                r.out = q.out + (q.S == r.S && q.L == r.L && q.k == r.k ? 0 : 1);
+            }
+            for (const auto& term : row.second) {
+                int32_t code = 0;
+                for (size_t k = 0; k < term.first.size(); ++k) code |= term.first[k] << (6 * k);
+                tt.hi_rterm.push_back(code);
+                cols.push_back(&term.second);
+            }
+            r.tend = static_cast<int32_t>(cols.size());
+            tt.hi_rows.push_back(r);
+        }
+        for (int n = 0; n < m.n_fn; ++n)
+            for (const std::vector<double>* c : cols) tt.hi_rcoef.push_back((*c)[n]);
     }
     tt.q12_off.assign(m.maxl + 2, 0);
     for (int L = 0; L <= m.maxl; ++L) {

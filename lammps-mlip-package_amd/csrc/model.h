@@ -140,6 +140,19 @@ struct VisitHi {
     int32_t tbeg, tend;         // term range
 };
 
+// Merged order-5/6 adjoint row of the linear families: all terms of one
+// (output S, L, m = -k; family order), over every family and factor position
+// that adds to it.  The table's order-5/6 factors are few (l <= 1: eight a per
+// centre), so thousands of (family, position) terms share a few hundred
+// products; a term lists its product once, with one coefficient per radial
+// index, sum over families of weight x C.  Term codes hold order - 1 factor
+// indices of 6 bits each, s (lmaxh + 1)^2 + l^2 + l + m.
+struct HiRow {
+    int32_t S, L, k, order;
+    int32_t tbeg, tend;                 // within the centre species' terms
+    int32_t out;                        // index of (S, L, k): rows of one output share a wave
+};
+
 // Radial-only model (des_type pair): one entry of the per-feature
 // derivative lists, H_a = w_a + sum_entries w prod(d_b, d_c) (b, c = -1 for
 // absent factors); ew = w / order is the Euler energy share of the term.
@@ -168,6 +181,11 @@ struct TypeTables {
     std::vector<VisitQ34> visits_adj, visits_feat;
     // orders 5/6: adjoint and polynomial-feature visits
     std::vector<VisitHi> hi_adj, hi_feat;
+    // linear families of orders 5/6, merged: rows, term codes, coefficients
+    // [radial index][term]
+    std::vector<HiRow> hi_rows;
+    std::vector<int32_t> hi_rterm;
+    std::vector<double> hi_rcoef;
     // order 3/4 visits before grouping (plan_q34 groups them)
     std::vector<PlanVisit> plan_adj, plan_feat;
 };

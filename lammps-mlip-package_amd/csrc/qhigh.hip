@@ -9,10 +9,11 @@
 // Workgroup = one wave on (block of 64 same-species centres, radial index n),
 // lane = centre.  The centre's a_{s,l<=lmaxh,m<=0} is staged in LDS (each
 // lane reads only its own entries); a visit is one (family, factor position)
-// with its terms listed: G_{S,L,-k} += H sum_terms C prod(other factors),
-// and for linear families the energy share (1/q) sum_k w_k Re(G_k a_{S,L,-k})
-// (Euler's theorem summed over the q factor positions), added to the
-// order-3/4 energy slot 0 of the centre after the order-3/4 kernel.
+// with its terms listed: G_{S,L,-k} += H sum_terms C prod(other factors).
+// Families outside the polynomial have the same weights for every centre and
+// run merged (k_qhigh_rows), with their energy (1/q) sum_k w_k
+// Re(G_k a_{S,L,-k}) (Euler's theorem summed over the q factor positions)
+// added to the order-3/4 energy slot 0 of the centre after that kernel.
 #include <hip/hip_runtime.h>
 
 #include "device_api.h"
@@ -58,11 +59,10 @@ __global__ __launch_bounds__(64) void k_qhigh(DevModel M, DevSystem S) {
     cptr<VisitHi> vis = as_const(M.hvis);
     cptr<int32_t> term = as_const(M.hterm);
     cptr<double> coef = as_const(M.hcoef);
-    double eacc = 0.0;
     for (int vi = vb; vi < ve; ++vi) {
         const VisitHi v = vis[vi];
-        const int L = uniform(v.L), Sx = uniform(v.S), q = uniform(v.order), pslot = uniform(v.pslot);
-        const int no = q - 1;
+        const int L = uniform(v.L), Sx = uniform(v.S), pslot = uniform(v.pslot);
+        const int no = uniform(v.order) - 1;
         double gr[kMaxLHi + 1], gi[kMaxLHi + 1];
 #pragma unroll
         for (int k = 0; k <= kMaxLHi; ++k) gr[k] = gi[k] = 0.0;
@@ -98,22 +98,104 @@ __global__ __launch_bounds__(64) void k_qhigh(DevModel M, DevSystem S) {
             S.D[prow + pslot] = d;
             continue;
         }
-        const double H = pslot >= 0 ? S.H[prow + pslot] : as_const(M.weight)[n * M.n_gtinv + uniform(v.itc)];
-        double dot = 0.0;
+        const double H = S.H[prow + pslot];
 #pragma unroll
         for (int k = 0; k <= kMaxLHi; ++k) {
             if (k > L) break;
-            const double hr = H * gr[k], hi = H * gi[k];
             double* g = S.G + a_index(M, blk, n, Sx, lmh(L, -k), 0, lane);
-            g[0] += hr;
-            g[kBlock] += hi;  // imaginary part: next component, same lane
-            double ar, ai;
-            T.get(Sx, L, -k, ar, ai);
-            dot = fma(k == 0 ? 1.0 : 2.0, hr * ar - hi * ai, dot);
+            g[0] += H * gr[k];
+            g[kBlock] += H * gi[k];  // imaginary part: next component, same lane
         }
-        if (pslot < 0) eacc = fma(1.0 / q, dot, eacc);
     }
-    if (!FEAT) S.Eq34[((size_t)slot * M.n_fn + n) * kWavesPerWg] += eacc;
+}
+
+// Merged rows of the linear families (HiRow): the workgroup's four waves share
+// the tile of a (block of centres, radial index), every m stored so that a
+// factor is one LDS read; a row's terms are dealt over the waves (term ti to
+// wave ti mod 4) and the four partial rows summed in wave order through LDS,
+// kHiRows rows at a time.  G_{S,L,-k} += scale sum_terms coef prod, energy
+// (1/q) w_k Re(G a) per row (Euler).  Bound: LDS reads and FP64 products of
+// the terms (the table's order-5/6 invariants: 61,036 terms of 1,090 visits
+// per species become the distinct products of 12 rows).  499 atoms of the
+// order-6, l <= 20 model: orders 5/6 49.3 ms as one visit per (family, factor
+// position) on one wave per (block, n), the evaluation 53.0 -> 3.1 ms.
+constexpr int kHiWaves = 4;
+constexpr int kHiRows = 8;
+
+__global__ __launch_bounds__(64 * kHiWaves) void k_qhigh_rows(DevModel M, DevSystem S) {
+    extern __shared__ double2 hi_tile[];
+    const int blk = blockIdx.x, n = blockIdx.y, lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+    const int t = uniform(S.block_type[blk]);
+    const int nh = M.n_lmhh, nl = (M.lmaxh + 1) * (M.lmaxh + 1);
+    double2* part = hi_tile + M.n_type * nl * kBlock;  // [row of the group][wave][lane]
+    for (int e = wave; e < M.n_type * nh; e += kHiWaves) {
+        const int s = e / nh, lm = e % nh;
+        int l = 0;
+        while ((l + 1) * (l + 2) / 2 <= lm) ++l;
+        const int m = l * (l + 1) / 2 + l - lm;  // entry of a_{l,-m}
+        const double re = S.A[a_index(M, blk, n, s, lm, 0, lane)], im = S.A[a_index(M, blk, n, s, lm, 1, lane)];
+        double2* row = hi_tile + (s * nl + l * l + l) * kBlock + lane;
+        row[-m * kBlock] = double2{re, im};
+        if (m > 0) row[m * kBlock] = (m & 1) ? double2{-re, im} : double2{re, -im};
+    }
+    __syncthreads();
+    cptr<HiRow> rows = as_const(M.hrow);
+    cptr<int32_t> term = as_const(M.hrterm) + uniform(M.hrt_off[t]);
+    cptr<double> coef = as_const(M.hrcoef) + uniform(M.hrc_off[t] + n * M.hrt_num[t]);
+    const double2* tile = hi_tile + lane;
+    double eacc = 0.0;
+    const int rb = uniform(M.hrow_beg[t]), re = uniform(M.hrow_end[t]);
+    for (int r0 = rb; r0 < re; r0 += kHiRows) {
+        const int rn = min(kHiRows, re - r0);
+        for (int r = 0; r < rn; ++r) {
+            const HiRow R = rows[r0 + r];
+            const int no = uniform(R.order) - 1;
+            double gr = 0.0, gi = 0.0;
+            for (int ti = uniform(R.tbeg) + wave; ti < uniform(R.tend); ti += kHiWaves) {
+                const int code = term[ti];
+                const double c = coef[ti];
+                double2 p = tile[(code & 63) * kBlock];
+                for (int o = 1; o < no; ++o) {
+                    const double2 y = tile[((code >> (6 * o)) & 63) * kBlock];
+                    p = double2{p.x * y.x - p.y * y.y, p.x * y.y + p.y * y.x};
+                }
+                gr = fma(c, p.x, gr);
+                gi = fma(c, p.y, gi);
+            }
+            part[(r * kHiWaves + wave) * kBlock + lane] = double2{gr, gi};
+        }
+        __syncthreads();
+        for (int r = 0; r < rn; ++r) {
+            const HiRow R = rows[r0 + r];
+            // the rows of one output (orders 5 and 6) add to the same G entry
+            if (uniform(R.out) % kHiWaves != wave) continue;
+            const int Sx = uniform(R.S), L = uniform(R.L), k = uniform(R.k);
+            const double iq = 1.0 / uniform(R.order), scale = M.hi_split ? iq : 1.0;
+            double gr = 0.0, gi = 0.0;
+#pragma unroll
+            for (int w = 0; w < kHiWaves; ++w) {
+                const double2 v = part[(r * kHiWaves + w) * kBlock + lane];
+                gr += v.x;
+                gi += v.y;
+            }
+            gr *= scale;
+            gi *= scale;
+            double* g = S.G + a_index(M, blk, n, Sx, lmh(L, -k), 0, lane);
+            g[0] += gr;
+            g[kBlock] += gi;
+            const double2 a = tile[(Sx * nl + L * L + L - k) * kBlock];
+            eacc = fma((k == 0 ? 1.0 : 2.0) * iq, gr * a.x - gi * a.y, eacc);
+        }
+        __syncthreads();
+    }
+    part[wave * kBlock + lane].x = eacc;
+    __syncthreads();
+    if (wave == 0) {
+        double e = 0.0;
+#pragma unroll
+        for (int w = 0; w < kHiWaves; ++w) e += part[w * kBlock + lane].x;
+        S.Eq34[((size_t)(blk * kBlock + lane) * M.n_fn + n) * kWavesPerWg] += e;
+    }
 }
 
 }  // namespace
@@ -124,9 +206,18 @@ hipError_t launch_qhigh(const DevModel& m, const DevSystem& s, bool feat, hipStr
     if (lds > lds_limit()) return hipErrorInvalidConfiguration;
     if (feat)
         hipLaunchKernelGGL(k_qhigh<true>, dim3(s.nblocks, m.n_fn), dim3(64), lds, st, m, s);
-    else
+    else if (m.hadj_end[0] > m.hadj_beg[0] || m.hadj_end[1] > m.hadj_beg[1])
         hipLaunchKernelGGL(k_qhigh<false>, dim3(s.nblocks, m.n_fn), dim3(64), lds, st, m, s);
-    return launched(lds);
+    hipError_t e = launched(lds);
+    if (feat || (m.hrow_end[0] == m.hrow_beg[0] && m.hrow_end[1] == m.hrow_beg[1])) return e;
+    const size_t rlds = sizeof(double2) * kBlock *
+                        (static_cast<size_t>(m.n_type) * (m.lmaxh + 1) * (m.lmaxh + 1) + kHiRows * kHiWaves);
+    if (rlds > lds_limit()) return hipErrorInvalidConfiguration;
+    const hipError_t ea = hipFuncSetAttribute(reinterpret_cast<const void*>(k_qhigh_rows),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(rlds));
+    if (ea != hipSuccess) return first_error(e, ea);
+    hipLaunchKernelGGL(k_qhigh_rows, dim3(s.nblocks, m.n_fn), dim3(64 * kHiWaves), rlds, st, m, s);
+    return first_error(e, launched(rlds));
 }
 
 }  // namespace mlip
