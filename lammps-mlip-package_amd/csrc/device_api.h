@@ -81,6 +81,9 @@ struct DevModel {
     const double* pair_w;   // linear weights, n_p (= n_des) entries
     const int32_t* ph_off;  // per-feature derivative lists
     const PairHEntry* ph_ent;
+    int pd_k2, pd_k3, pd_cols;  // dense derivative product (pd_cols = 0: none, see Model)
+    const int32_t* pd_bc;
+    const double* pd_w;     // [species][pd_k2 + pd_k3][pd_cols]
     int q34_red;            // doubles of LDS partial rows of split adjoint groups
     int q34_dyn_adj, q34_dyn_feat;  // visits for the general-loop order-3/4 kernel
     const YTab<double>* yt64;

@@ -266,6 +266,18 @@ bool upload_model(mlip_ctx* c) {
         dm.pair_w = c->d_pairw.p;
         dm.ph_off = c->d_phoff.p;
         dm.ph_ent = c->d_phent.p;
+        dm.pd_cols = m.pd_cols;
+        if (m.pd_cols > 0) {
+            std::vector<double> w;
+            for (int t = 0; t < m.n_type; ++t) w.insert(w.end(), m.pd_w[t].begin(), m.pd_w[t].end());
+            if (!upload(c, c->d_pdbc, m.pd_bc.data(), m.pd_bc.size(), "pair product rows") ||
+                !upload(c, c->d_pdw, w.data(), w.size(), "pair product weights"))
+                return false;
+            dm.pd_k2 = m.pd_k2;
+            dm.pd_k3 = m.pd_k3;
+            dm.pd_bc = c->d_pdbc.p;
+            dm.pd_w = c->d_pdw.p;
+        }
     }
     if (m.has_hi) {
         std::vector<VisitHi> hv;
@@ -1032,6 +1044,8 @@ void mlip_destroy(mlip_ctx* c) {
     c->d_pairw.release();
     c->d_phoff.release();
     c->d_phent.release();
+    c->d_pdbc.release();
+    c->d_pdw.release();
     c->d_hvis.release();
     c->d_hterm.release();
     c->d_hcoef.release();

@@ -65,8 +65,8 @@ struct mlip_ctx {
     mlip::DBuf<mlip::GroupQ34> d_gadj, d_gfeat;
     mlip::DBuf<mlip::YTab<double>> d_yt64;
     mlip::DBuf<mlip::YTab<float>> d_yt32;
-    mlip::DBuf<double> d_pairw;
-    mlip::DBuf<int32_t> d_phoff, d_zlist;
+    mlip::DBuf<double> d_pairw, d_pdw;
+    mlip::DBuf<int32_t> d_phoff, d_pdbc, d_zlist;
     mlip::DBuf<mlip::PairHEntry> d_phent;
     mlip::DBuf<mlip::VisitHi> d_hvis;
     mlip::DBuf<int32_t> d_hterm, d_hrterm;

@@ -913,6 +913,55 @@ bool load_pair_model(std::istream& in, Model& m, std::string& err, bool strict_c
         m.ph_ent.insert(m.ph_ent.end(), lists[a].begin(), lists[a].end());
         m.ph_off[a + 1] = static_cast<int32_t>(m.ph_ent.size());
     }
+    // dense form: every product row of the seen features; taken when the
+    // lists fill at least an eighth of it (model_type 2 fills it, model_type
+    // 1 has one entry per column)
+    {
+        const int nf = m.n_type * m.n_fn;
+        std::vector<int32_t> bc;
+        std::vector<int> row2(nf), row3(static_cast<size_t>(nf) * nf, -1);
+        auto pad = [&] {
+            while (bc.size() % 4) bc.push_back(nf | nf << 16);
+        };
+        for (int b = 0; b < nf; ++b) {
+            row2[b] = static_cast<int>(bc.size());
+            bc.push_back(b | nf << 16);
+        }
+        pad();
+        m.pd_k2 = static_cast<int>(bc.size());
+        if (!m.comb3.empty())
+            for (int b = 0; b < nf; ++b)
+                for (int c = b; c < nf; ++c) {
+                    row3[b * nf + c] = static_cast<int>(bc.size());
+                    bc.push_back(b | c << 16);
+                }
+        pad();
+        m.pd_k3 = static_cast<int>(bc.size()) - m.pd_k2;
+        m.pd_cols = (nf + 15) / 16 * 16;
+        size_t filled = 0;
+        for (int t = 0; t < m.n_type; ++t) {
+            std::vector<int> local(m.n_des, -1);
+            for (int s = 0; s < m.n_type; ++s)
+                for (int n = 0; n < m.n_fn; ++n) local[m.pair_tc[t][s] * m.n_fn + n] = s * m.n_fn + n;
+            std::vector<double>& w = m.pd_w[t];
+            w.assign(bc.size() * m.pd_cols, 0.0);
+            for (int a = 0; a < m.n_des; ++a)
+                for (int k = m.ph_off[a]; k < m.ph_off[a + 1] && local[a] >= 0; ++k) {
+                    const PairHEntry& q = m.ph_ent[k];
+                    const int b = local[q.b], c = q.c < 0 ? nf : local[q.c];
+                    if (b < 0 || c < 0) continue;  // a factor this species does not see is zero
+                    const int row = q.c < 0 ? row2[b] : row3[std::min(b, c) * nf + std::max(b, c)];
+                    w[static_cast<size_t>(row) * m.pd_cols + local[a]] += q.w;
+                    ++filled;
+                }
+        }
+        m.pd_bc = std::move(bc);
+        if (filled * 8 < m.pd_bc.size() * static_cast<size_t>(nf) * m.n_type) {
+            m.pd_cols = 0;
+            m.pd_bc.clear();
+            for (auto& w : m.pd_w) w.clear();
+        }
+    }
     // device layout: the feature rows reuse the polynomial-feature buffers
     m.n_p = m.n_des;
     m.maxl = 0;

@@ -235,6 +235,15 @@ struct Model {
     std::array<std::array<int, 2>, 2> pair_tc{};   // [centre type][neighbor type] -> tc
     std::vector<int32_t> ph_off;                   // n_des + 1
     std::vector<PairHEntry> ph_ent;
+    // the same derivatives as one dense product per centre species t where
+    // the lists fill it: columns a = s n_fn + n (its features by neighbor
+    // species s, nf = n_type n_fn of them, padded to 16), rows = the factors
+    // d_b (kd2 rows, the quadratic terms), then the products d_b d_c, b <= c
+    // (the cubic ones), each part padded to 4 rows; pd_bc holds b | c << 16
+    // per row (index nf: the factor 1)
+    int pd_k2 = 0, pd_k3 = 0, pd_cols = 0;         // pd_cols = 0: lists only
+    std::vector<int32_t> pd_bc;
+    std::vector<double> pd_w[2];                   // [row][pd_cols]
     int q34_red = 0;           // doubles of LDS partial rows (adjoint pass), max over types
     // orders 5/6: term codes and coefficients of every VisitHi, tile l_max
     std::vector<int32_t> hi_term;
