@@ -14,6 +14,9 @@ namespace mlip {
 constexpr int kBlock = kBlockLanes;  // atoms per slot block (one wavefront of lanes)
 
 
+// doubles of DevSystem::red: partial energies, then partial virials
+constexpr int kRedDoubles = 4096;
+
 enum Precision : int { kFP64 = 0, kMixed = 1 };
 
 // Constants of the normalised Legendre recursion (see pair_kernels.hip).
@@ -132,8 +135,8 @@ struct DevSystem {
     double* Hq;      // quadratic-form product [slot][n_p]
     double* H;       // polynomial adjoint [slot][n_p]
     double* Ep;      // [slot]
-    double* Eq12;    // [slot][n_fn]
-    double* Eq34;    // [slot][n_fn][kWavesPerWg]
+    double* Eq12;    // [blk][n_fn][64]
+    double* Eq34;    // [blk][n_fn][kWavesPerWg][64]
     double* gpair;   // [npairs][3] dE_centre/d(del)
     double* vown;    // [nown][6]
     const int32_t* goff;   // [nall] force gather lists: begin

@@ -398,7 +398,7 @@ bool setup_layout(mlip_ctx* c, int nall, int nown, int64_t npairs, const std::ve
         !c->H.ensure(z.psz) || !c->Ep.ensure(z.nslot) || !c->Eq12.ensure(z.nslot * m.n_fn) ||
         !c->Eq34.ensure(z.nslot * m.n_fn * kWavesPerWg) || !c->gpair.ensure(static_cast<size_t>(npairs) * 3) ||
         !c->vown.ensure(static_cast<size_t>(nown) * 6) || !c->f.ensure(static_cast<size_t>(nall) * 3) ||
-        !c->e_slot.ensure(z.nslot) || !c->red.ensure(7 * 128) || !c->out.ensure(8)) {
+        !c->e_slot.ensure(z.nslot) || !c->red.ensure(kRedDoubles) || !c->out.ensure(8)) {
         c->err = "device allocation failed for structure buffers";
         return false;
     }

@@ -11,7 +11,7 @@
 //   k_poly   E_i polynomial part and H = dE_i/dd                 (:321-343,481-521)
 //   k_force  per-pair dE_i/d(del) from G and dphi/d(del)          (:161-256, pair_kernels.hip)
 //   k_gather atomics-free per-position force sums, deterministic
-//   k_energy per-centre energies and virial, fixed-order reductions
+//   k_energy, k_totals  per-centre energies and virial, fixed-order reductions
 //
 // Conventions shared with the reference CPU style: del = x_centre - x_neighbor,
 // a_nlm uses Y_lm(del) without conjugation, pairs with r < cutoff (strict).
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64) void k_q12(DevModel M, DevSystem S, int stage) 
     }
     Q12Levels<0, kMaxLQ12, FEAT>::run(M, S, blk, n, lane, t, e, tile);
     for (int L = kMaxLQ12 + 1; L <= M.maxl; ++L) q12_level_dyn<FEAT>(M, S, blk, n, lane, t, L, e, tile);
-    if (!FEAT) S.Eq12[(size_t)(blk * kBlock + lane) * M.n_fn + n] = e;
+    if (!FEAT) S.Eq12[((size_t)blk * M.n_fn + n) * kBlock + lane] = e;
     if (FEAT && tile && w > 0) {
         __syncthreads();
         // segment of slot j: w doubles from column n * w of its row
@@ -318,33 +318,41 @@ __global__ __launch_bounds__(256) void k_atom_ev(DevSystem S, const double* __re
 }
 
 // ---------------------------------------------------------------- gather
+// kGatherLanes lanes per position: lane u takes entries u, u + 16, ... of the
+// position's list, four at a time (their pair forces loaded together), and
+// the lanes' sums go through a fixed butterfly, so the order of a position's
+// sum depends on its own list alone.  Bound: the latency of the scattered
+// pair-force reads (~270 entries per position at 137 neighbors).  One lane per
+// position, eight entries at a time, walked ~34 such round trips in a row:
+// 3,991 atoms 123 us, 2,048 atoms with 440 neighbors 322 us, 256k atoms 1.01 ms.
+constexpr int kGatherLanes = 16;
+
 __global__ __launch_bounds__(256) void k_gather(DevSystem S) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= S.nall) return;
+    const int u = threadIdx.x % kGatherLanes;
+    const int k = static_cast<int>((blockIdx.x * 256LL + threadIdx.x) / kGatherLanes);
+    if (k >= S.nall) return;  // whole groups of lanes leave together
     double fx = 0.0, fy = 0.0, fz = 0.0;
     const int e1 = S.gend[k];
-    int e = S.goff[k];
-    // eight entries per step: their pair forces are loaded together, then
-    // added in list order (the same sums as one entry at a time)
-    for (; e + 8 <= e1; e += 8) {
-        double v[8][3], sg[8];
+    int e = S.goff[k] + u;
+    for (; e + 3 * kGatherLanes < e1; e += 4 * kGatherLanes) {
+        double v[4][3], sg[4];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int code = S.gent[e + u];
+        for (int q = 0; q < 4; ++q) {
+            const int code = S.gent[e + q * kGatherLanes];
             const int64_t p = code > 0 ? code - 1 : -code - 1;
-            sg[u] = code > 0 ? 1.0 : -1.0;
-            v[u][0] = S.gpair[3 * p];
-            v[u][1] = S.gpair[3 * p + 1];
-            v[u][2] = S.gpair[3 * p + 2];
+            sg[q] = code > 0 ? 1.0 : -1.0;
+            v[q][0] = S.gpair[3 * p];
+            v[q][1] = S.gpair[3 * p + 1];
+            v[q][2] = S.gpair[3 * p + 2];
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            fx = fma(sg[u], v[u][0], fx);
-            fy = fma(sg[u], v[u][1], fy);
-            fz = fma(sg[u], v[u][2], fz);
+        for (int q = 0; q < 4; ++q) {
+            fx = fma(sg[q], v[q][0], fx);
+            fy = fma(sg[q], v[q][1], fy);
+            fz = fma(sg[q], v[q][2], fz);
         }
     }
-    for (; e < e1; ++e) {
+    for (; e < e1; e += kGatherLanes) {
         const int code = S.gent[e];
         const int64_t p = code > 0 ? code - 1 : -code - 1;
         const double sg = code > 0 ? 1.0 : -1.0;
@@ -352,86 +360,116 @@ __global__ __launch_bounds__(256) void k_gather(DevSystem S) {
         fy = fma(sg, S.gpair[3 * p + 1], fy);
         fz = fma(sg, S.gpair[3 * p + 2], fz);
     }
-    S.f[3 * k] = fx;
-    S.f[3 * k + 1] = fy;
-    S.f[3 * k + 2] = fz;
+#pragma unroll
+    for (int off = kGatherLanes / 2; off > 0; off >>= 1) {
+        fx += __shfl_xor(fx, off);
+        fy += __shfl_xor(fy, off);
+        fz += __shfl_xor(fz, off);
+    }
+    if (u < 3) S.f[3 * (size_t)k + u] = u == 0 ? fx : u == 1 ? fy : fz;
 }
 
 // ---------------------------------------------------------------- energy / virial
-__global__ __launch_bounds__(256) void k_energy_slot(DevModel M, DevSystem S) {
-    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= S.nblocks * kBlock) return;
-    double e = 0.0;
-    if (S.atom_of_slot[slot] >= 0 && M.pair_model) {
-        e = S.Ep[slot];
-    } else if (S.atom_of_slot[slot] >= 0) {
-        e = M.n_p > 0 ? S.Ep[slot] : 0.0;
-        for (int n = 0; n < M.n_fn; ++n) {
-            if (M.q12_adj_levels) e += S.Eq12[(size_t)slot * M.n_fn + n];
-            if (M.has_q34)
-                for (int w = 0; w < kWavesPerWg; ++w) e += S.Eq34[((size_t)slot * M.n_fn + n) * kWavesPerWg + w];
+// Workgroups below `eparts`: energies of the slot blocks blockIdx, blockIdx +
+// eparts, ... (four waves, wave w the radial indices w, w + 4, ...; reads are
+// whole lines, lane = slot), and the sum over them in red[blockIdx].  The
+// next vparts workgroups (totals only): partial virials over the owned
+// atoms, kVirRows at a time.  k_totals adds the parts, all in fixed order.  (Two launches; one
+// per-slot kernel and two reductions of two levels each took five.)
+constexpr int kEnergyThreads = 256;
+constexpr int kVirRows = 42;  // atoms per pass of a workgroup: 252 threads read whole runs of vown
+
+__global__ __launch_bounds__(kEnergyThreads) void k_energy(DevModel M, DevSystem S, int eparts, int vparts) {
+    __shared__ double sh[kEnergyThreads];
+    const int tid = threadIdx.x;
+    if (static_cast<int>(blockIdx.x) < eparts) {
+        const int lane = tid & 63, w = tid >> 6;
+        double total = 0.0;
+        for (int blk = blockIdx.x; blk < S.nblocks; blk += eparts) {
+            double e = 0.0;
+            if (!M.pair_model)
+                for (int n = w; n < M.n_fn; n += kEnergyThreads / 64) {
+                    const size_t row = static_cast<size_t>(blk) * M.n_fn + n;
+                    if (M.q12_adj_levels) e += S.Eq12[row * kBlock + lane];
+                    if (M.has_q34)
+#pragma unroll
+                        for (int q = 0; q < kWavesPerWg; ++q) e += S.Eq34[(row * kWavesPerWg + q) * kBlock + lane];
+                }
+            sh[tid] = e;
+            __syncthreads();
+            if (w == 0) {
+                const int slot = blk * kBlock + lane;
+                double v = M.pair_model || M.n_p > 0 ? S.Ep[slot] : 0.0;
+#pragma unroll
+                for (int q = 0; q < kEnergyThreads / 64; ++q) v += sh[q * 64 + lane];
+                if (S.atom_of_slot[slot] < 0) v = 0.0;
+                S.e_slot[slot] = v;
+                total += v;
+            }
+            __syncthreads();
         }
+        if (w == 0) {
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
+            if (lane == 0) S.red[blockIdx.x] = total;
+        }
+        return;
     }
-    S.e_slot[slot] = e;
+    // virial: component tid % 6 of atoms part * kVirRows + tid / 6, ...
+    const int part = blockIdx.x - eparts;
+    double v = 0.0;
+    if (tid < 6 * kVirRows)
+        for (int64_t i = static_cast<int64_t>(part) * kVirRows + tid / 6; i < S.nown;
+             i += static_cast<int64_t>(vparts) * kVirRows)
+            v += S.vown[6 * i + tid % 6];
+    sh[tid] = v;
+    __syncthreads();
+    if (tid < 6) {
+        double s = 0.0;
+        for (int k = 0; k < kVirRows; ++k) s += sh[6 * k + tid];
+        S.red[kRedDoubles / 2 + part * 6 + tid] = s;
+    }
+}
+
+__global__ __launch_bounds__(64 * 7) void k_totals(DevSystem S, int eparts, int vparts) {
+    // wave 0: energy; wave 1 + c: virial component c
+    const int c = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    double s = 0.0;
+    if (c == 0) {
+        for (int i = lane; i < eparts; i += 64) s += S.red[i];
+    } else {
+        for (int i = lane; i < vparts; i += 64) s += S.red[kRedDoubles / 2 + i * 6 + c - 1];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if (lane == 0) S.out[c] = s;
 }
 
 // Per-structure energy and virial of a batch: one workgroup per structure,
-// fixed-order tree over its (contiguous) atoms.
+// its (contiguous) atoms over the threads, the seven sums by wave butterflies
+// and over the waves in order.
 __global__ __launch_bounds__(256) void k_struct_reduce(DevSystem S, const int32_t* sbeg, const int32_t* send,
                                                        double* out) {
-    __shared__ double sh[256];
+    __shared__ double sh[7][4];
     const int st = blockIdx.x;
     const int a0 = sbeg[st], a1 = send[st];
-    for (int c = 0; c < 7; ++c) {
-        double v = 0.0;
-        for (int i = a0 + threadIdx.x; i < a1; i += 256)
-            v += c == 0 ? S.e_slot[S.slot_of_atom[i]] : S.vown[6 * (size_t)i + (c - 1)];
-        sh[threadIdx.x] = v;
-        __syncthreads();
-        for (int w = 128; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) out[7 * st + c] = sh[0];
-        __syncthreads();
+    double v[7] = {0, 0, 0, 0, 0, 0, 0};
+    for (int i = a0 + threadIdx.x; i < a1; i += 256) {
+        v[0] += S.e_slot[S.slot_of_atom[i]];
+#pragma unroll
+        for (int c = 0; c < 6; ++c) v[1 + c] += S.vown[6 * (size_t)i + c];
     }
-}
-
-// Fixed-order two-level reduction: k_reduce1 sums contiguous chunks per
-// workgroup, k_reduce2 sums the partials in one workgroup.
-constexpr int kRedThreads = 256;
-
-__global__ __launch_bounds__(kRedThreads) void k_reduce1(const double* in, int n, int stride, int ncomp,
-                                                         double* part) {
-    __shared__ double sh[kRedThreads];
-    for (int c = 0; c < ncomp; ++c) {
-        double s = 0.0;
-        for (int i = blockIdx.x * kRedThreads + threadIdx.x; i < n; i += gridDim.x * kRedThreads)
-            s += in[(size_t)i * stride + c];
-        sh[threadIdx.x] = s;
-        __syncthreads();
-        for (int w = kRedThreads / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) part[c * gridDim.x + blockIdx.x] = sh[0];
-        __syncthreads();
-    }
-}
-
-__global__ __launch_bounds__(kRedThreads) void k_reduce2(const double* part, int nparts, int ncomp, double* out) {
-    __shared__ double sh[kRedThreads];
-    for (int c = 0; c < ncomp; ++c) {
-        double s = 0.0;
-        for (int i = threadIdx.x; i < nparts; i += kRedThreads) s += part[c * nparts + i];
-        sh[threadIdx.x] = s;
-        __syncthreads();
-        for (int w = kRedThreads / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) out[c] = sh[0];
-        __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 7; ++c)
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v[c] += __shfl_xor(v[c], off);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int c = 0; c < 7; ++c) sh[c][threadIdx.x >> 6] = v[c];
+    __syncthreads();
+    if (threadIdx.x < 7) {
+        const double* q = sh[threadIdx.x];
+        out[7 * st + threadIdx.x] = ((q[0] + q[1]) + q[2]) + q[3];
     }
 }
 
@@ -509,7 +547,8 @@ hipError_t launch_atom_ev(const DevSystem& s, const double* epv, double* evat, h
 
 hipError_t launch_gather(const DevModel&, const DevSystem& s, hipStream_t st) {
     if (s.nall == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_gather, dim3((s.nall + 255) / 256), dim3(256), 0, st, s);
+    const int64_t threads = static_cast<int64_t>(s.nall) * kGatherLanes;
+    hipLaunchKernelGGL(k_gather, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, st, s);
     return launched();
 }
 
@@ -536,18 +575,13 @@ hipError_t launch_struct_reduce(const DevSystem& s, const int32_t* sbeg, const i
 }
 
 hipError_t launch_energy_virial(const DevModel& m, const DevSystem& s, bool totals, hipStream_t st) {
-    const int nslot = s.nblocks * kBlock;
-    if (nslot > 0) hipLaunchKernelGGL(k_energy_slot, dim3((nslot + 255) / 256), dim3(256), 0, st, m, s);
-    hipError_t e = launched();
+    const int eparts = std::min(s.nblocks, kRedDoubles / 2);
+    const int vparts = totals ? std::min(kRedDoubles / 2 / 6, (s.nown + kVirRows - 1) / kVirRows) : 0;
+    if (eparts + vparts > 0)
+        hipLaunchKernelGGL(k_energy, dim3(eparts + vparts), dim3(kEnergyThreads), 0, st, m, s, eparts, vparts);
+    const hipError_t e = launched();
     if (!totals) return e;
-    const int parts = 120;
-    hipLaunchKernelGGL(k_reduce1, dim3(parts), dim3(kRedThreads), 0, st, s.e_slot, nslot, 1, 1, s.red);
-    e = first_error(e, launched());
-    hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kRedThreads), 0, st, s.red, parts, 1, s.out);
-    e = first_error(e, launched());
-    hipLaunchKernelGGL(k_reduce1, dim3(parts), dim3(kRedThreads), 0, st, s.vown, s.nown, 6, 6, s.red + parts);
-    e = first_error(e, launched());
-    hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kRedThreads), 0, st, s.red + parts, parts, 6, s.out + 1);
+    hipLaunchKernelGGL(k_totals, dim3(1), dim3(64 * 7), 0, st, s, eparts, vparts);
     return first_error(e, launched());
 }
 

@@ -77,7 +77,7 @@ void carve(Carver& cv, const Model& m, const LammpsLists& L, int inum, const Wor
     b.vown = cv.take<double>(6 * static_cast<size_t>(inum));
     b.f = cv.take<double>(3 * na);
     b.e_slot = cv.take<double>(z.nslot);
-    b.red = cv.take<double>(7 * 128);
+    b.red = cv.take<double>(kRedDoubles);
     b.out = cv.take<double>(8);
     if (split) {
         P.epv = cv.take<double>(7 * np);

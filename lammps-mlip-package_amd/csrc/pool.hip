@@ -486,7 +486,7 @@ int mlip_pool_init(mlip_ctx* c, int64_t max_atoms, int64_t max_pairs, int max_re
                     p->A.ensure(asz) && p->G.ensure(asz) && p->D.ensure(ns * np) && p->Hq.ensure(ns * np) &&
                     p->H.ensure(ns * np) && p->Ep.ensure(ns) && p->Eq12.ensure(ns * m.n_fn) &&
                     p->Eq34.ensure(ns * m.n_fn * kWavesPerWg) && p->e_slot.ensure(ns) &&
-                    p->atom_of_slot.ensure(ns) && p->block_type.ensure(ns / kBlock + 1) && p->red.ensure(7 * 128) &&
+                    p->atom_of_slot.ensure(ns) && p->block_type.ensure(ns / kBlock + 1) && p->red.ensure(kRedDoubles) &&
                     p->out.ensure(8) && p->sout.ensure(7 * nr) && p->ke.ensure(6 * nr) && p->sbeg.ensure(nr) &&
                     p->send.ensure(nr) && p->first.ensure(nr) && p->final_.ensure(nr) && p->disp.ensure(nr) &&
                     p->dnext.ensure(nr) && p->xref.ensure(3 * na) && p->mass.ensure(static_cast<size_t>(m.n_type));

@@ -863,7 +863,7 @@ __global__ __launch_bounds__(kQ34Threads) void k_q34(DevModel M, DevSystem S) {
                 q34_combine(M, S, g, blk, n, T.lane, red, DYN);
             }
         }
-        double* e = &S.Eq34[((size_t)(blk * kBlock + T.lane) * M.n_fn + n) * kWavesPerWg + wave];
+        double* e = &S.Eq34[(((size_t)blk * M.n_fn + n) * kWavesPerWg + wave) * kBlock + T.lane];
         if (DYN)
             *e += eacc;
         else

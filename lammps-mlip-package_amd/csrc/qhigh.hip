@@ -194,7 +194,7 @@ __global__ __launch_bounds__(64 * kHiWaves) void k_qhigh_rows(DevModel M, DevSys
         double e = 0.0;
 #pragma unroll
         for (int w = 0; w < kHiWaves; ++w) e += part[w * kBlock + lane].x;
-        S.Eq34[((size_t)(blk * kBlock + lane) * M.n_fn + n) * kWavesPerWg] += e;
+        S.Eq34[((size_t)blk * M.n_fn + n) * kWavesPerWg * kBlock + lane] += e;
     }
 }
 
