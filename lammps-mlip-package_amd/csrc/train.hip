@@ -10,14 +10,11 @@
 // is the virial.
 //
 // Kernels (a_nlm from k_anlm in FP64 first):
-//   k_tr_feat    thread per (slot lane, feature): CG terms over the lane's
-//                a_nlm rows (lane-contiguous, coalesced)
-//   k_tr_poly    thread per (atom, coefficient)
-//   k_tr_dirj    workgroup per centre: its a_nlm in LDS; per chunk of its
-//                pairs the geometry, g_n, g'_n and Y_lm, grad Y_lm in LDS;
-//                then thread per (pair, itc, n): dirj = d d_f^(i)/d del_q
+//   k_tr_dirj    workgroup per (centre, group of features): the features, and
+//                dirj = d d_f^(i)/d del_q for every pair q of the centre
 //                (mlipkk.cpp:992-1157 restated for a full list: each
 //                directed pair carries its own centre's derivative)
+//   k_tr_poly    thread per (atom, coefficient)
 //   k_tr_force   thread per (atom, coefficient): the atom's gather list in
 //                pair order, g_qp = sum_nu prod_{nu' != nu} X[cen][f_nu'] dirj[q][f_nu],
 //                -g on the centre, +g on the neighbor (fixed order)
@@ -26,6 +23,7 @@
 // All FP64.  Work and memory scale with pairs x n_des (dirj) and atoms x
 // n_coeff (force features): a training-sized structure or batch, not the
 // 256k-atom evaluation workload.
+#include <algorithm>
 #include <climits>
 #include <cstring>
 
@@ -73,10 +71,10 @@ namespace {
 using namespace dev;
 
 constexpr int kTrThreads = 256;
-constexpr int kTrPairs = 8;     // pairs per chunk of k_tr_dirj
-constexpr int kTrMaxFn = 16;    // radial functions of the training path (kTrPairs * kTrMaxFn threads fill g_n)
-constexpr int kTrFeatY = 16;    // features per workgroup of k_tr_feat
-constexpr int kTrMaxL = 12;     // angular momenta of the training path (kTrPairs * (kTrMaxL + 1) <= 128 threads)
+constexpr int kTrPairs = 16;    // pairs per chunk of k_tr_dirj (at most)
+constexpr int kTrMaxF = 128;    // features per workgroup of k_tr_dirj (at most)
+constexpr int kTrMaxFn = 16;    // radial functions of the training path
+constexpr int kTrMaxL = 12;     // angular momenta of the training path (2 n_lmh / 4 <= 64 depth steps)
 constexpr int kTrL1 = kTrMaxL + 1;
 
 struct TrArgs {
@@ -103,40 +101,6 @@ __device__ __forceinline__ void fac(int code, double& re, double& im) {
     }
 }
 
-__global__ __launch_bounds__(64) void k_tr_feat(DevModel M, DevSystem S, TrArgs T) {
-    const int blk = blockIdx.x;
-    const int lane = threadIdx.x;
-    const int slot = blk * kBlock + lane;
-    const int atom = S.atom_of_slot[slot];
-    const int t = S.block_type[blk];
-    const int f1 = min(T.n_des, (int)(blockIdx.y + 1) * kTrFeatY);
-    for (int f = blockIdx.y * kTrFeatY; f < f1; ++f) {
-        const int itc = f % T.n_gtinv, n = f / T.n_gtinv;
-        const TrItc& I = T.itc[itc];
-        bool seen = true;
-        for (int mu = 0; mu < I.order; ++mu) seen = seen && I.spec[t][mu] >= 0;
-        double d = 0.0;
-        if (seen) {
-            for (int k = I.tbeg; k < I.tend; ++k) {
-                const TrTerm& tm = T.term[k];
-                double pr = tm.c, pi = 0.0;
-                for (int mu = 0; mu < I.order; ++mu) {
-                    const int code = tm.code[mu];
-                    const int lm = code & 0xffff;
-                    double ar = S.A[a_index(M, blk, n, I.spec[t][mu], lm, 0, lane)];
-                    double ai = S.A[a_index(M, blk, n, I.spec[t][mu], lm, 1, lane)];
-                    fac(code, ar, ai);
-                    const double nr = pr * ar - pi * ai;
-                    pi = pr * ai + pi * ar;
-                    pr = nr;
-                }
-                d += pr;
-            }
-        }
-        if (atom >= 0) T.X[(size_t)atom * T.n_des + f] = d;
-    }
-}
-
 __global__ __launch_bounds__(kTrThreads) void k_tr_poly(int natoms, TrArgs T) {
     const int64_t w = (int64_t)blockIdx.x * kTrThreads + threadIdx.x;
     if (w >= (int64_t)natoms * T.n_coeff) return;
@@ -155,36 +119,66 @@ __global__ __launch_bounds__(kTrThreads) void k_tr_pcen(DevSystem S, int32_t* pc
     for (int q = S.poff[a]; q < S.pend[a]; ++q) pcen[q] = a;
 }
 
+// Shape of a k_tr_dirj launch: F features and `pairs` pairs at a time per
+// workgroup, kp = 2 n_lmh rounded up to the matrix instruction's depth of 4,
+// and the rows of radial indices F consecutive features can span.
+struct TrShape {
+    int F, pairs, kp, nrow;
+    __host__ __device__ int ypitch() const { return kp + 2; }
+};
+
 struct TrLds {
     double yt_diag[kTrL1 + 1];
     double yt_alm[kTrL1][kTrL1];
     double yt_ainv[kTrL1][kTrL1];
     double yt_grad[kTrL1][kTrL1];
-    double ux[kTrPairs], uy[kTrPairs], uz[kTrPairs], rr[kTrPairs];
-    int spec[kTrPairs], valid[kTrPairs];
+    double ux[kTrPairs], uy[kTrPairs], uz[kTrPairs], rr[kTrPairs], fc[kTrPairs], fcd[kTrPairs];
+    int spec[kTrPairs];
     double gn[kTrPairs][kTrMaxFn], gd[kTrPairs][kTrMaxFn];
+    unsigned long long steps[kTrMaxF / 16][2];
 };
 
-// dynamic LDS: a of the centre [n][s][lm] (re, im), then per chunk pair
-// Y_{l,-m} and grad Y_{l,-m} [pair][lm][4] (re, im)
-__global__ __launch_bounds__(kTrThreads) void k_tr_dirj(DevModel M, DevSystem S, TrArgs T) {
+// Structural features and their derivatives along every pair of the centre.
+// Workgroup = (centre, F consecutive features).
+//  1. Thread per feature: d_f and, since d d_f / d a_{s,n,lm} does not depend
+//     on the pair, its partials B_f[s][(lm, re/im)] over all terms and factors
+//     into the thread's own LDS column (m > 0 folded onto m <= 0).
+//  2. Per tile of pairs: Y_lm and grad Y_lm of each pair into LDS, then
+//     [(pair, Y / x / y / z)][(lm, c)] x B[(lm, c)][f] on the matrix cores
+//     (v_mfma_f64_16x16x4f64, lanes as in k_anlm_mfma): 4 pairs x 16 features
+//     per instruction tile; rows of pairs of the other species are masked, and
+//     the depth steps no feature of the tile uses are skipped.  Row i = pair
+//     i % 4, quantity i / 4, so a lane ends with the four sums of one pair and
+//     feature.
+// Bound: the products of step 1 and the matrix steps.  Forming each pair's
+// derivative from all terms took one product chain per (pair, term, factor):
+// 12 random cells of 8-32 atoms (gtinv-820, ~1,900 features, ~70 pairs per
+// atom) 51.0 ms, now 2.3 ms.
+__global__ __launch_bounds__(kTrThreads) void k_tr_dirj(DevModel M, DevSystem S, TrArgs T, TrShape H, int grad) {
     extern __shared__ double tr_dyn[];
     __shared__ TrLds C;
+    typedef double dbl4 __attribute__((ext_vector_type(4)));
     const int atom = blockIdx.x;
-    if (atom >= S.nown) return;
     const int tid = threadIdx.x;
     const int nfn = M.n_fn, ns = M.n_type, nlmh = M.n_lmh, maxl = M.maxl;
     const int slot = S.slot_of_atom[atom];
-    const int blk = slot / kBlock, lane = slot % kBlock;
+    const int blk = slot / kBlock, slane = slot % kBlock;
     const int tcen = S.elem[atom];
-    double* aL = tr_dyn;                                  // 2 * nfn * ns * nlmh
-    double* yL = tr_dyn + (size_t)2 * nfn * ns * nlmh;    // kTrPairs * nlmh * 8
-    for (int k = tid; k < nfn * ns * nlmh; k += kTrThreads) {
-        const int lm = k % nlmh, s = (k / nlmh) % ns, n = k / (nlmh * ns);
-        aL[2 * k] = S.A[a_index(M, blk, n, s, lm, 0, lane)];
-        aL[2 * k + 1] = S.A[a_index(M, blk, n, s, lm, 1, lane)];
+    const int f0 = blockIdx.y * H.F, f1 = min(f0 + H.F, T.n_des);
+    const int nlo = f0 / T.n_gtinv, nhi = (f1 - 1) / T.n_gtinv;
+    double* aL = tr_dyn;                                          // [n - nlo][s][lm] (re, im)
+    double* bL = aL + static_cast<size_t>(2) * H.nrow * ns * nlmh;  // [s][kp][F]
+    double* yL = bL + static_cast<size_t>(ns) * H.kp * H.F;       // [pair][quantity][ypitch]
+    const int yp = H.ypitch();
+    for (int k = tid; k < (nhi - nlo + 1) * ns * nlmh; k += kTrThreads) {
+        const int lm = k % nlmh, s = (k / nlmh) % ns, n = nlo + k / (nlmh * ns);
+        aL[2 * k] = S.A[a_index(M, blk, n, s, lm, 0, slane)];
+        aL[2 * k + 1] = S.A[a_index(M, blk, n, s, lm, 1, slane)];
     }
-    {
+    if (grad) {
+        for (int k = tid; k < ns * H.kp * H.F; k += kTrThreads) bL[k] = 0.0;
+        for (int k = tid; k < H.pairs * 4 * yp; k += kTrThreads) yL[k] = 0.0;
+        if (tid < 2 * (kTrMaxF / 16)) C.steps[tid / 2][tid % 2] = 0;
         const YTab<double>* yt = M.yt64;
         for (int k = tid; k < kTrL1 * kTrL1; k += kTrThreads) {
             const int l = k / kTrL1, mm = k % kTrL1;
@@ -194,15 +188,71 @@ __global__ __launch_bounds__(kTrThreads) void k_tr_dirj(DevModel M, DevSystem S,
         }
         if (tid <= kTrL1) C.yt_diag[tid] = yt->diag[tid];
     }
+    __syncthreads();
+    if (f0 + tid < f1) {
+        const int f = f0 + tid, itc = f % T.n_gtinv, n = f / T.n_gtinv;
+        const TrItc& I = T.itc[itc];
+        bool seen = true;
+        for (int mu = 0; mu < I.order; ++mu) seen = seen && I.spec[tcen][mu] >= 0;
+        double d = 0.0;
+        if (seen) {
+            const double* ar = aL + static_cast<size_t>(2) * (n - nlo) * ns * nlmh;
+            unsigned long long used[2] = {0, 0};
+            for (int k = I.tbeg; k < I.tend; ++k) {
+                const TrTerm& tm = T.term[k];
+                double vr[4], vi[4];
+                double pr = tm.c, pi = 0.0;
+#pragma unroll
+                for (int mu = 0; mu < 4; ++mu) {
+                    if (mu >= I.order) break;
+                    const double* av = ar + 2 * (I.spec[tcen][mu] * nlmh + (tm.code[mu] & 0xffff));
+                    vr[mu] = av[0];
+                    vi[mu] = av[1];
+                    fac(tm.code[mu], vr[mu], vi[mu]);
+                    const double nr = pr * vr[mu] - pi * vi[mu];
+                    pi = pr * vi[mu] + pi * vr[mu];
+                    pr = nr;
+                }
+                d += pr;
+                if (!grad) continue;
+#pragma unroll
+                for (int mu = 0; mu < 4; ++mu) {
+                    if (mu >= I.order) break;
+                    double qr = tm.c, qi = 0.0;
+#pragma unroll
+                    for (int m2 = 0; m2 < 4; ++m2) {
+                        if (m2 >= I.order || m2 == mu) continue;
+                        const double nr = qr * vr[m2] - qi * vi[m2];
+                        qi = qr * vi[m2] + qi * vr[m2];
+                        qr = nr;
+                    }
+                    // Re(q Y_m) with Y_m = (-1)^m conj(Y_{-m}) for m > 0 is
+                    // Re((-1)^m conj(q) Y_{-m})
+                    const int code = tm.code[mu], kk = 2 * (code & 0xffff), s = I.spec[tcen][mu];
+                    fac(code, qr, qi);
+                    double* col = bL + (static_cast<size_t>(s) * H.kp + kk) * H.F + tid;
+                    col[0] += qr;
+                    col[H.F] += qi;
+                    used[s] |= 1ull << (kk >> 2);
+                }
+            }
+            if (grad)
+                for (int s = 0; s < ns; ++s) atomicOr(&C.steps[tid / 16][s], used[s]);
+        }
+        T.X[static_cast<size_t>(atom) * T.n_des + f] = d;
+    }
+    if (!grad) return;
     const int p0 = S.poff[atom], p1 = S.pend[atom];
     const double pir = 3.141592653589793 / M.cutoff;
-    const int items = kTrPairs * T.n_gtinv * nfn;
-    for (int pc = p0; pc < p1; pc += kTrPairs) {
+    const int wave = uniform(tid >> 6), lane = tid & 63;
+    const int ftiles = (f1 - f0 + 15) / 16;
+    for (int pc = p0; pc < p1; pc += H.pairs) {
+        const int np = min(H.pairs, p1 - pc);
         __syncthreads();
-        if (tid < kTrPairs) {
+        if (tid < H.pairs) {
             const int q = pc + tid;
-            int ok = 0;
-            if (q < p1) {
+            int spec = -1;
+            if (tid < np) {
                 const int nb = S.pnbr[q];
                 double dx = S.x[3 * atom] - S.x[3 * nb], dy = S.x[3 * atom + 1] - S.x[3 * nb + 1],
                        dz = S.x[3 * atom + 2] - S.x[3 * nb + 2];
@@ -212,153 +262,151 @@ __global__ __launch_bounds__(kTrThreads) void k_tr_dirj(DevModel M, DevSystem S,
                     dz += S.pshift[3 * q + 2];
                 }
                 const double r = sqrt(dx * dx + dy * dy + dz * dz);
-                ok = (r < M.cutoff) && (r > 0.0);
-                if (ok) {
+                if ((r < M.cutoff) && (r > 0.0)) {
+                    spec = S.elem[nb];
                     C.ux[tid] = dx / r;
                     C.uy[tid] = dy / r;
                     C.uz[tid] = dz / r;
                     C.rr[tid] = r;
-                    C.spec[tid] = S.elem[nb];
+                    double sa, ca;
+                    sincos(pir * r, &sa, &ca);
+                    C.fc[tid] = 0.5 * (ca + 1.0);
+                    C.fcd[tid] = -0.5 * pir * sa;
                 }
             }
-            C.valid[tid] = ok;
+            C.spec[tid] = spec;
         }
         __syncthreads();
-        if (tid < kTrPairs * kTrL1) {
-            // column m of pair j: Y_{l,-m} and grad Y_{l,-m} for l = m..maxl
-            const int j = tid / kTrL1, m = tid % kTrL1;
-            if (m <= maxl && C.valid[j]) {
-                const double x = C.ux[j], y = C.uy[j], z = C.uz[j], ir = 1.0 / C.rr[j];
-                double cr = 1.0, ci = 0.0;  // conj(u)^m
-                for (int k = 0; k < m; ++k) {
-                    const double nr = cr * x + ci * y;
-                    ci = ci * x - cr * y;
-                    cr = nr;
-                }
-                double mr = 0.0, mi = 0.0;  // conj(u)^(m-1)
-                if (m > 0) {
-                    mr = 1.0;
-                    for (int k = 0; k < m - 1; ++k) {
-                        const double nr = mr * x + mi * y;
-                        mi = mi * x - mr * y;
-                        mr = nr;
-                    }
-                }
-                const double pr = cr * x + ci * y, pi = ci * x - cr * y;  // conj(u)^(m+1)
-                const double sg = (m & 1) ? -1.0 : 1.0, zz = 1.0 - z * z, fm = (double)m;
-                double a1 = 0.0, a2 = 0.0, b1 = 0.0, b2 = 0.0;
-                for (int l = m; l <= maxl; ++l) {
-                    const double q = (l == m) ? C.yt_diag[m] : C.yt_alm[l][m] * (z * a1 - C.yt_ainv[l][m] * a2);
-                    a2 = a1;
-                    a1 = q;
-                    double qp = 0.0;
-                    if (l == m + 1)
-                        qp = C.yt_diag[m + 1];
-                    else if (l > m + 1)
-                        qp = C.yt_alm[l][m + 1] * (z * b1 - C.yt_ainv[l][m + 1] * b2);
-                    b2 = b1;
-                    b1 = qp;
-                    double gxr, gxi, gyr, gyi, gzr, gzi;
-                    if (m == 0) {
-                        const double c = C.yt_grad[l][0] * qp;
-                        gxr = c * z * x;
-                        gxi = 0.0;
-                        gyr = c * z * y;
-                        gyi = 0.0;
-                        gzr = -c * zz;
-                        gzi = 0.0;
-                    } else {
-                        const double c = C.yt_grad[l][m];
-                        const double A = fm * z * q + zz * c * qp;
-                        const double B = fm * q - z * c * qp;
-                        const double E = fm * (1.0 + z * z) * q + z * zz * c * qp;
-                        gxr = 0.5 * (-B * pr + E * mr);
-                        gxi = 0.5 * (-B * pi + E * mi);
-                        const double zr = B * pr + E * mr, zi = B * pi + E * mi;
-                        gyr = 0.5 * zi;
-                        gyi = -0.5 * zr;
-                        gzr = -A * cr;
-                        gzi = -A * ci;
-                    }
-                    double* o = yL + ((size_t)j * nlmh + (l * (l + 1) / 2 + l - m)) * 8;
-                    o[0] = sg * q * cr;
-                    o[1] = sg * q * ci;
-                    o[2] = sg * gxr * ir;
-                    o[3] = sg * gxi * ir;
-                    o[4] = sg * gyr * ir;
-                    o[5] = sg * gyi * ir;
-                    o[6] = sg * gzr * ir;
-                    o[7] = sg * gzi * ir;
-                }
+        for (int it = tid; it < np * (maxl + 1); it += kTrThreads) {
+            // column m of pair j: Y_{l,-m} and grad Y_{l,-m} for l = m..maxl,
+            // imaginary parts negated (Re(B Y) = Br Yr + Bi (-Yi))
+            const int j = it % np, m = it / np;
+            if (C.spec[j] < 0) continue;
+            const double x = C.ux[j], y = C.uy[j], z = C.uz[j], ir = 1.0 / C.rr[j];
+            double cr = 1.0, ci = 0.0;  // conj(u)^m
+            double mr = 0.0, mi = 0.0;  // conj(u)^(m-1)
+            for (int k = 0; k < m; ++k) {
+                mr = cr;
+                mi = ci;
+                const double nr = cr * x + ci * y;
+                ci = ci * x - cr * y;
+                cr = nr;
             }
-        } else if (tid >= 128 && tid < 128 + kTrPairs * kTrMaxFn) {
-            const int j = (tid - 128) / kTrMaxFn, n = (tid - 128) % kTrMaxFn;
-            if (n < nfn && C.valid[j]) {
-                const double r = C.rr[j];
-                double sa, ca;
-                sincos(pir * r, &sa, &ca);
-                const double fc = 0.5 * (ca + 1.0), fcd = -0.5 * pir * sa;
-                const double dd = r - M.mu[n], be = M.beta[n];
-                const double b = exp(-be * (dd * dd));
-                C.gn[j][n] = b * fc;
-                C.gd[j][n] = b * (fcd - 2.0 * be * dd * fc);
+            const double pr = cr * x + ci * y, pi = ci * x - cr * y;  // conj(u)^(m+1)
+            const double sg = (m & 1) ? -1.0 : 1.0, zz = 1.0 - z * z, fm = (double)m;
+            double a1 = 0.0, a2 = 0.0, b1 = 0.0, b2 = 0.0;
+            for (int l = m; l <= maxl; ++l) {
+                const double q = (l == m) ? C.yt_diag[m] : C.yt_alm[l][m] * (z * a1 - C.yt_ainv[l][m] * a2);
+                a2 = a1;
+                a1 = q;
+                double qp = 0.0;
+                if (l == m + 1)
+                    qp = C.yt_diag[m + 1];
+                else if (l > m + 1)
+                    qp = C.yt_alm[l][m + 1] * (z * b1 - C.yt_ainv[l][m + 1] * b2);
+                b2 = b1;
+                b1 = qp;
+                double gxr, gxi, gyr, gyi, gzr, gzi;
+                if (m == 0) {
+                    const double c = C.yt_grad[l][0] * qp;
+                    gxr = c * z * x;
+                    gxi = 0.0;
+                    gyr = c * z * y;
+                    gyi = 0.0;
+                    gzr = -c * zz;
+                    gzi = 0.0;
+                } else {
+                    const double c = C.yt_grad[l][m];
+                    const double A = fm * z * q + zz * c * qp;
+                    const double B = fm * q - z * c * qp;
+                    const double E = fm * (1.0 + z * z) * q + z * zz * c * qp;
+                    gxr = 0.5 * (-B * pr + E * mr);
+                    gxi = 0.5 * (-B * pi + E * mi);
+                    const double zr = B * pr + E * mr, zi = B * pi + E * mi;
+                    gyr = 0.5 * zi;
+                    gyi = -0.5 * zr;
+                    gzr = -A * cr;
+                    gzi = -A * ci;
+                }
+                double* o = yL + static_cast<size_t>(4 * j) * yp + 2 * (l * (l + 1) / 2 + l - m);
+                o[0] = sg * q * cr;
+                o[1] = -sg * q * ci;
+                o[yp] = sg * gxr * ir;
+                o[yp + 1] = -sg * gxi * ir;
+                o[2 * yp] = sg * gyr * ir;
+                o[2 * yp + 1] = -sg * gyi * ir;
+                o[3 * yp] = sg * gzr * ir;
+                o[3 * yp + 1] = -sg * gzi * ir;
             }
+        }
+        for (int it = tid; it < np * nfn; it += kTrThreads) {
+            const int j = it / nfn, n = it % nfn;
+            if (C.spec[j] < 0) continue;
+            const double dd = C.rr[j] - M.mu[n], be = M.beta[n];
+            const double b = exp(-be * (dd * dd));
+            C.gn[j][n] = b * C.fc[j];
+            C.gd[j][n] = b * (C.fcd[j] - 2.0 * be * dd * C.fc[j]);
         }
         __syncthreads();
-        for (int w = tid; w < items; w += kTrThreads) {
-            const int n = w % nfn;
-            const int itc = (w / nfn) % T.n_gtinv;
-            const int j = w / (nfn * T.n_gtinv);
-            const int q = pc + j;
-            if (q >= p1) continue;
-            const int f = n * T.n_gtinv + itc;
-            double* out = T.dirj + ((size_t)q * T.n_des + f) * 3;
-            double sy = 0.0, sx = 0.0, syy = 0.0, sz = 0.0;
-            const TrItc& I = T.itc[itc];
-            bool seen = C.valid[j] != 0;
-            for (int mu = 0; mu < I.order; ++mu) seen = seen && I.spec[tcen][mu] >= 0;
-            if (seen) {
-                const int sj = C.spec[j];
-                const double* ar = aL + (size_t)2 * n * ns * nlmh;
-                const double* yj = yL + (size_t)j * nlmh * 8;
-                for (int k = I.tbeg; k < I.tend; ++k) {
-                    const TrTerm& tm = T.term[k];
-                    for (int mu = 0; mu < I.order; ++mu) {
-                        if (I.spec[tcen][mu] != sj) continue;
-                        double pr = tm.c, pi = 0.0;
-                        for (int mu2 = 0; mu2 < I.order; ++mu2) {
-                            if (mu2 == mu) continue;
-                            const int code = tm.code[mu2];
-                            const double* av = ar + 2 * ((size_t)I.spec[tcen][mu2] * nlmh + (code & 0xffff));
-                            double vr = av[0], vi = av[1];
-                            fac(code, vr, vi);
-                            const double nr = pr * vr - pi * vi;
-                            pi = pr * vi + pi * vr;
-                            pr = nr;
-                        }
-                        const int code = tm.code[mu];
-                        const double* yv = yj + (size_t)(code & 0xffff) * 8;
-                        double v[8];
-                        for (int e = 0; e < 8; ++e) v[e] = yv[e];
-                        for (int e = 0; e < 4; ++e) fac(code, v[2 * e], v[2 * e + 1]);
-                        sy += pr * v[0] - pi * v[1];
-                        sx += pr * v[2] - pi * v[3];
-                        syy += pr * v[4] - pi * v[5];
-                        sz += pr * v[6] - pi * v[7];
-                    }
+        const int ptiles = (np + 3) / 4;
+        for (int task = wave; task < ptiles * ftiles; task += kTrThreads / 64) {
+            const int ft = task % ftiles, pt = task / ftiles;
+            // A[i][k] from lane 16 k + i, B[k][j] from lane 16 k + j
+            const int ja = 4 * pt + (lane & 3), quant = (lane >> 2) & 3, kl = lane >> 4;
+            const int sa = ja < np ? C.spec[ja] : -1;
+            const double* ya = yL + static_cast<size_t>(4 * ja + quant) * yp + kl;
+            const double* bb = bL + static_cast<size_t>(kl) * H.F + 16 * ft + (lane & 15);
+            dbl4 acc = {0.0, 0.0, 0.0, 0.0};
+            for (int s = 0; s < ns; ++s) {
+                if (__ballot(sa == s) == 0) continue;
+                unsigned long long left = C.steps[ft][s];
+                while (left) {
+                    const int k = 4 * __builtin_ctzll(left);
+                    left &= left - 1;
+                    const double a = sa == s ? ya[k] : 0.0;
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        a, bb[(static_cast<size_t>(s) * H.kp + k) * H.F], acc, 0, 0, 0);
                 }
             }
-            if (seen) {
-                const double gd = C.gd[j][n], gn = C.gn[j][n];
-                out[0] = gd * C.ux[j] * sy + gn * sx;
-                out[1] = gd * C.uy[j] * sy + gn * syy;
-                out[2] = gd * C.uz[j] * sy + gn * sz;
-            } else {
-                out[0] = 0.0;
-                out[1] = 0.0;
-                out[2] = 0.0;
+            // lane: D[i = lane / 16 + 4 r][lane % 16] = quantity r of pair lane / 16
+            const int j = 4 * pt + (lane >> 4), f = f0 + 16 * ft + (lane & 15);
+            if (j < np && f < f1) {
+                double* out = T.dirj + (static_cast<size_t>(pc + j) * T.n_des + f) * 3;
+                double gd = 0.0, gn = 0.0, ux = 0.0, uy = 0.0, uz = 0.0;
+                if (C.spec[j] >= 0) {
+                    const int n = f / T.n_gtinv;
+                    gd = C.gd[j][n];
+                    gn = C.gn[j][n];
+                    ux = C.ux[j];
+                    uy = C.uy[j];
+                    uz = C.uz[j];
+                }
+                out[0] = gd * ux * acc[0] + gn * acc[1];
+                out[1] = gd * uy * acc[0] + gn * acc[2];
+                out[2] = gd * uz * acc[0] + gn * acc[3];
             }
         }
+    }
+}
+
+// LDS bytes of a launch shape, and the shape for a model: 128 features and 16
+// pairs per workgroup where the tables leave two workgroups per CU, fewer as
+// l_max grows (B takes n_type kp 8 bytes per feature, a pair 32 kp).
+size_t tr_lds(const DevModel& m, const TrShape& h) {
+    return sizeof(double) * (static_cast<size_t>(2) * h.nrow * m.n_type * m.n_lmh +
+                             static_cast<size_t>(m.n_type) * h.kp * h.F + static_cast<size_t>(h.pairs) * 4 * h.ypitch());
+}
+
+TrShape tr_shape(const DevModel& m, int n_gtinv) {
+    TrShape h{kTrMaxF, kTrPairs, (2 * m.n_lmh + 3) / 4 * 4, 0};
+    for (;;) {
+        h.nrow = std::min(m.n_fn, (h.F - 1) / n_gtinv + 2);
+        if (tr_lds(m, h) + sizeof(TrLds) <= 80 * 1024 || (h.F == 16 && h.pairs == 4)) return h;
+        // the larger of the two tables first
+        if (h.F > 16 && (h.pairs == 4 || m.n_type * h.F >= 4 * h.pairs))
+            h.F /= 2;
+        else
+            h.pairs /= 2;
     }
 }
 
@@ -517,8 +565,8 @@ int train_features(mlip_ctx* c, double* X, double* P, double* FF, double* SF) {
         c->err = "training features are defined for the gtinv descriptor";
         return MLIP_ERR_MODEL;
     }
-    static_assert(128 + kTrPairs * kTrMaxFn <= kTrThreads, "g_n threads of k_tr_dirj");
-    static_assert(kTrPairs * kTrL1 <= 128, "Y_lm threads of k_tr_dirj");
+    static_assert((kTrL1 * (kTrL1 + 1) + 3) / 4 <= 64, "depth steps of k_tr_dirj in one mask");
+    static_assert(kTrMaxF <= kTrThreads, "a thread per feature in k_tr_dirj");
     if (m.maxl > kTrMaxL) {
         c->err = "training features support max_l up to 12";
         return MLIP_ERR_MODEL;
@@ -573,23 +621,11 @@ int train_features(mlip_ctx* c, double* X, double* P, double* FF, double* SF) {
     TrArgs a{w.itc.p, w.term.p, w.rows.p, m.n_des, m.n_coeff, m.n_gtinv, w.X.p, w.P.p, w.FF.p, w.SF.p, w.dirj.p,
              w.pcen.p};
     if (!hip_ok(c, launch_anlm(c->dm, s, kFP64, st), "a_nlm launch")) return MLIP_ERR_DEVICE;
-    if (s.nblocks > 0) {
-        hipLaunchKernelGGL(k_tr_feat, dim3(s.nblocks, (m.n_des + kTrFeatY - 1) / kTrFeatY), dim3(64), 0, st, c->dm,
-                           s, a);
-        if (!hip_ok(c, launched(), "training feature launch")) return MLIP_ERR_DEVICE;
-    }
-    const int64_t npw = static_cast<int64_t>(n) * m.n_coeff;
-    if (npw > 0) {
-        hipLaunchKernelGGL(k_tr_poly, dim3(static_cast<unsigned>((npw + kTrThreads - 1) / kTrThreads)),
-                           dim3(kTrThreads), 0, st, n, a);
-        if (!hip_ok(c, launched(), "polynomial feature launch")) return MLIP_ERR_DEVICE;
-    }
-    if (n > 0 && np > 0 && (FF || SF)) {
-        hipLaunchKernelGGL(k_tr_pcen, dim3((n + kTrThreads - 1) / kTrThreads), dim3(kTrThreads), 0, st, s, w.pcen.p);
-        if (!hip_ok(c, launched(), "pair centre launch")) return MLIP_ERR_DEVICE;
-        const size_t lds = sizeof(double) * (2 * static_cast<size_t>(m.n_fn) * m.n_type * m.n_lmh +
-                                             static_cast<size_t>(kTrPairs) * m.n_lmh * 8);
-        if (lds > lds_limit()) {
+    const bool grad = n > 0 && np > 0 && (FF || SF);
+    if (n > 0) {
+        const TrShape h = tr_shape(c->dm, m.n_gtinv);
+        const size_t lds = tr_lds(c->dm, h);
+        if (lds + sizeof(TrLds) > lds_limit()) {
             c->err = "training features: the model's per-centre LDS tile exceeds the device limit";
             return MLIP_ERR_MODEL;
         }
@@ -597,8 +633,19 @@ int train_features(mlip_ctx* c, double* X, double* P, double* FF, double* SF) {
                                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
                     "training LDS"))
             return MLIP_ERR_DEVICE;
-        hipLaunchKernelGGL(k_tr_dirj, dim3(n), dim3(kTrThreads), lds, st, c->dm, s, a);
+        hipLaunchKernelGGL(k_tr_dirj, dim3(n, (m.n_des + h.F - 1) / h.F), dim3(kTrThreads), lds, st, c->dm, s, a, h,
+                           grad ? 1 : 0);
         if (!hip_ok(c, launched(), "feature derivative launch")) return MLIP_ERR_DEVICE;
+    }
+    const int64_t npw = static_cast<int64_t>(n) * m.n_coeff;
+    if (npw > 0) {
+        hipLaunchKernelGGL(k_tr_poly, dim3(static_cast<unsigned>((npw + kTrThreads - 1) / kTrThreads)),
+                           dim3(kTrThreads), 0, st, n, a);
+        if (!hip_ok(c, launched(), "polynomial feature launch")) return MLIP_ERR_DEVICE;
+    }
+    if (grad) {
+        hipLaunchKernelGGL(k_tr_pcen, dim3((n + kTrThreads - 1) / kTrThreads), dim3(kTrThreads), 0, st, s, w.pcen.p);
+        if (!hip_ok(c, launched(), "pair centre launch")) return MLIP_ERR_DEVICE;
         const int pchunks = (m.n_coeff + kTrThreads - 1) / kTrThreads;
         if (FF) {
             hipLaunchKernelGGL(k_tr_force, dim3(static_cast<unsigned>(static_cast<int64_t>(n) * pchunks)),
