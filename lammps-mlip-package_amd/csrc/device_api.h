@@ -29,7 +29,8 @@ struct YTab {
 };
 
 struct DevModel {
-    int n_type, n_fn, n_gtinv, n_lmh, n_lmh3, maxl, lmax3, n_pitc, n_p;
+    int n_type, n_fn, n_gtinv, n_lmh, maxl, lmax3, n_pitc, n_p;
+    int lmax_t;             // largest l of the order-3/4 adjoint kernel's tile (lmax3: the feature kernel's)
     int has_q34;            // order-3/4 invariants present (k_q34 runs)
     int q12_fuse;           // order-1/2 adjoint rows L <= q12_fuse are the order-3/4 kernel's (-1: none)
     int q12_fuse_hi;        // ... and the rows lmax3 < L <= q12_fuse_hi (a_nlm from HBM)
@@ -44,6 +45,18 @@ struct DevModel {
     const VisitPack* vadj;
     const GroupQ34* gadj;
     int32_t gadj_beg[2], gadj_end[2];
+    // order-3 linear families by output m (q3.hip): tasks of species t and wave
+    // w are t3[t3_off[t][w] .. t3_off[t][w + 1]), weights from w3_off[t], w3_ent[t]
+    // entries of 8 per radial index
+    const Rec3* r3;
+    const Task3* t3;
+    const double* c3;
+    const double* w3;
+    int32_t t3_off[2][kWavesPerWg + 1], w3_off[2], w3_ent[2];
+    const double* c4;       // order-4 linear families ([species][n][q4_total]) or null
+    const int32_t* q12r;    // order-1/2 families of the rows ([species][S][kMaxLQ12 + 1][6], see TypeTables)
+    int lmaxq3;             // largest l of the order-3 families (-1: the kernel does not run)
+    int q3_rounds;
     const VisitPack* vfeat;
     const GroupQ34* gfeat;
     int32_t gfeat_beg[2], gfeat_end[2];
@@ -105,13 +118,16 @@ struct DevModel {
     const int32_t* hrterm;
     const double* hrcoef;
     int32_t hrow_beg[2], hrow_end[2], hrt_off[2], hrt_num[2], hrc_off[2];
-    int hi_split;           // 1: rows scaled by 1 / order (the per-atom energy split)
+    int split;              // 1: merged families scaled by 1 / order (the per-atom energy split)
 };
 
-// order-1/2 adjoint row L runs inside the order-3/4 kernel
+// order-1/2 adjoint row L runs inside the order-3 kernel, which then writes every
+// row L <= kMaxLQ12, or inside the order-3/4 kernel (else the order-1/2 kernel's)
 __host__ __device__ inline bool q12_fused(const DevModel& m, int L) {
-    return L <= m.q12_fuse || (L > m.lmax3 && L <= m.q12_fuse_hi);
+    return (m.lmaxq3 >= 0 && L <= kMaxLQ12) || L <= m.q12_fuse || (L > m.lmax_t && L <= m.q12_fuse_hi);
 }
+// the order-3/4 kernel writes the row (otherwise one before it did)
+__host__ __device__ inline bool q34_writes(const DevModel& m, int L) { return m.lmaxq3 < 0 && q12_fused(m, L); }
 
 struct DevSystem {
     int nall;      // positions (owned atoms first; ghosts / images after)
@@ -174,6 +190,9 @@ hipError_t launch_anlm(const DevModel& m, const DevSystem& s, int precision, hip
 bool anlm_has_mfma(const DevModel& m);
 bool anlm_forms_features(const DevModel& m, int precision, int kind);
 hipError_t launch_q12(const DevModel& m, const DevSystem& s, bool feat, hipStream_t st);
+// order-3 linear families, G rows l <= lmaxq3 and the first order-3/4 energies
+// (called by launch_q34_adj); no-op for models without them
+hipError_t launch_q3(const DevModel& m, const DevSystem& s, hipStream_t st);
 hipError_t launch_q34_adj(const DevModel& m, const DevSystem& s, hipStream_t st);
 hipError_t launch_q34_feat(const DevModel& m, const DevSystem& s, hipStream_t st);
 // general-loop passes for visits outside the unrolled signatures (launched

@@ -17,6 +17,7 @@
 
 #include "engine_internal.h"
 #include "neighbor.h"
+#include "q4_terms.h"
 #include "workload.h"
 
 using namespace mlip;
@@ -114,9 +115,11 @@ bool upload_model(mlip_ctx* c) {
     dm.n_fn = m.n_fn;
     dm.n_gtinv = m.n_gtinv;
     dm.n_lmh = m.n_lmh;
-    dm.n_lmh3 = m.n_lmh3;
     dm.maxl = m.maxl;
     dm.lmax3 = m.lmax3;
+    dm.lmax_t = m.lmax_t;
+    dm.lmaxq3 = m.lmaxq3;
+    dm.q3_rounds = m.q3_rounds;
     dm.n_pitc = m.n_pitc;
     dm.n_p = m.n_p;
     for (int t = 0; t < 2; ++t)
@@ -278,6 +281,46 @@ bool upload_model(mlip_ctx* c) {
             dm.pd_bc = c->d_pdbc.p;
             dm.pd_w = c->d_pdw.p;
         }
+    }
+    if (m.lmaxq3 >= 0) {
+        std::vector<Rec3> r3;
+        std::vector<Task3> t3;
+        std::vector<double> w3, c4;
+        std::vector<int32_t> q12r;
+        const bool order4 = !m.types[0].c4.empty() || (m.n_type > 1 && !m.types[1].c4.empty());
+        for (int t = 0; t < m.n_type && t < 2; ++t) {
+            const TypeTables& tt = m.types[t];
+            const int rb = static_cast<int>(r3.size()), tb = static_cast<int>(t3.size());
+            for (int w = 0; w <= kWavesPerWg; ++w) dm.t3_off[t][w] = tb + tt.t3_off[w];
+            for (Task3 k : tt.task3) {
+                k.rbeg += rb;
+                k.rend += rb;
+                t3.push_back(k);
+            }
+            r3.insert(r3.end(), tt.rec3.begin(), tt.rec3.end());
+            dm.w3_off[t] = static_cast<int32_t>(w3.size());
+            dm.w3_ent[t] = tt.w3_ent;
+            w3.insert(w3.end(), tt.w3.begin(), tt.w3.end());
+            q12r.insert(q12r.end(), tt.q12r.begin(), tt.q12r.end());
+            // a species without order-4 families has zero coefficients
+            if (order4) {
+                c4.insert(c4.end(), tt.c4.begin(), tt.c4.end());
+                c4.resize(static_cast<size_t>(t + 1) * m.n_fn * q4_total(m.n_type), 0.0);
+            }
+        }
+        if (!upload(c, c->d_r3, r3.data(), r3.size(), "order-3 records") ||
+            !upload(c, c->d_t3, t3.data(), t3.size(), "order-3 tasks") ||
+            !upload(c, c->d_c3q, m.c3q.data(), m.c3q.size(), "order-3 coefficients") ||
+            !upload(c, c->d_w3, w3.data(), w3.size(), "order-3 weights") ||
+            !upload(c, c->d_q12r, q12r.data(), q12r.size(), "order-1/2 rows") ||
+            (order4 && !upload(c, c->d_c4, c4.data(), c4.size(), "order-4 products")))
+            return false;
+        dm.q12r = c->d_q12r.p;
+        dm.c4 = order4 ? c->d_c4.p : nullptr;
+        dm.r3 = c->d_r3.p;
+        dm.t3 = c->d_t3.p;
+        dm.c3 = c->d_c3q.p;
+        dm.w3 = c->d_w3.p;
     }
     if (m.has_hi) {
         std::vector<VisitHi> hv;
@@ -739,7 +782,7 @@ bool run_atom_split(mlip_ctx* c, double* epv, double* evat) {
         run("pair_model_energy", launch_pair_model_energy(me, se, epv, st));
     } else {
         me.weight = c->d_weight_e.p;
-        me.hi_split = 1;
+        me.split = 1;
         se.H = se.Hq;
         if (me.n_p > 0) run("poly_split", launch_poly_split(me, se, st));
         if (ok) run("q12_split", launch_q12(me, se, false, st));
@@ -1050,6 +1093,12 @@ void mlip_destroy(mlip_ctx* c) {
     c->d_hterm.release();
     c->d_hcoef.release();
     c->d_hrow.release();
+    c->d_r3.release();
+    c->d_t3.release();
+    c->d_c3q.release();
+    c->d_w3.release();
+    c->d_c4.release();
+    c->d_q12r.release();
     c->d_hrterm.release();
     c->d_hrcoef.release();
     drop_graph(c);
@@ -1653,6 +1702,11 @@ int mlip_flops(const mlip_ctx* c, double* out7) {
         };
         out7[2] += na * terms(tt.groups_feat, tt.visits_feat, false);
         out7[3] += na * terms(tt.groups_adj, tt.visits_adj, true);
+        // order-3 kernel: its records, the order-1/2 rows (5 per entry and
+        // factor species), order-4 products (6 each, then 4 per output)
+        out7[3] += na * tt.q3_flops;
+        if (!tt.q12r.empty()) out7[3] += na * 5.0 * m.n_type * m.n_type * n_lmh_of(std::min(m.maxl, kMaxLQ12));
+        if (!tt.c4.empty()) out7[3] += na * (m.n_type == 1 ? 31 * 6.0 + 69 * 6.0 + 87 * 4.0 : 137 * 6.0 + 484 * 6.0 + 1208 * 4.0);
         // orders 5/6: per term the product of the other factors (6 per
         // complex product after the first), then 4 (adjoint: one complex
         // FMA pair into G) or 5 (features); per visit the G update and the

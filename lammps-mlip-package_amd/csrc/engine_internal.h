@@ -72,6 +72,10 @@ struct mlip_ctx {
     mlip::DBuf<int32_t> d_hterm, d_hrterm;
     mlip::DBuf<double> d_hcoef, d_hrcoef;
     mlip::DBuf<mlip::HiRow> d_hrow;
+    mlip::DBuf<mlip::Rec3> d_r3;
+    mlip::DBuf<mlip::Task3> d_t3;
+    mlip::DBuf<double> d_c3q, d_w3, d_c4;
+    mlip::DBuf<int32_t> d_q12r;
     mlip::DevModel dm{};
     // structure buffers
     mlip::DBuf<double> x, pshift, A, G, D, Hq, H, Ep, Eq12, Eq34, gpair, vown, f, e_slot, red, out;

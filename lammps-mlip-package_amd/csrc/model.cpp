@@ -2,6 +2,8 @@
 // See model.h for the reference functions each part corresponds to.
 #include "model.h"
 
+#include "q4_terms.h"
+
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -242,7 +244,8 @@ void pair_rows(const Model& m, std::vector<PlanVisit>& pend) {
     auto cls = [](const VisitQ34& v) { return v.pslot >= 0 ? 4 : std::max(v.order - 1, 0); };
     std::vector<PlanVisit> out;
     std::vector<bool> taken(pend.size(), false);
-    for (int L = 0; L <= std::min(kPairMaxL, m.plan_pair); ++L) {
+    // (rows above the kernel's LDS tile have a path of their own)
+    for (int L = 0; L <= std::min({kPairMaxL, m.plan_pair, m.lmax_t}); ++L) {
         std::vector<size_t> r0, r1;
         bool all_fast = true;
         for (size_t k = 0; k < pend.size(); ++k) {
@@ -352,7 +355,7 @@ void make_groups(const Model& m, std::vector<PlanVisit> pend, std::vector<GroupQ
     }
     // LDS available for the partial rows of split rows (adjoint only):
     // what the workgroup's 160 KB leave beside the a_nlm tile
-    const long tile = static_cast<long>(m.n_type) * n_lmh_of(m.lmax3) * 2 * kBlockLanes;
+    const long tile = static_cast<long>(m.n_type) * n_lmh_of(m.lmax_t) * 2 * kBlockLanes;
     const long budget = adjoint ? std::max(0L, 160L * 1024 / 8 - tile) : 1L << 40;
     // a paired row keeps two partial rows per part
     auto row_red = [](int L, int np, int S) {
@@ -509,8 +512,260 @@ void make_groups(const Model& m, std::vector<PlanVisit> pend, std::vector<GroupQ
     red_total = std::max(red_total, red);
 }
 
+// Moves the order-3 visits of families outside the polynomial from `adj` into
+// m.types' by-output-m form (built by plan_order3): entry (la, lb, L) of one
+// irrep with its coefficient block and, per output species and species
+// combination, the families' weights.  An entry's visits must have coefficient
+// blocks proportional to one another (within the table's printed digits);
+// visits of an entry that has not stay in `adj`.
+struct Entry3 {
+    int la, lb, L;
+    std::vector<double> block;   // [ma + la][k], k <-> m_out = -k
+    // (output species, combination, family, factor)
+    std::vector<std::tuple<int, int, int, double>> use;
+};
+
+void extract_order3(const Model& m, std::vector<PlanVisit>& adj, std::vector<Entry3>& out) {
+    constexpr int kMaxL3 = 10;
+    std::map<std::array<int, 5>, std::vector<size_t>> groups;  // parity, la, lb, L, irrep
+    for (size_t i = 0; i < adj.size(); ++i) {
+        const VisitQ34& v = adj[i].v;
+        if (v.order != 3 || v.pslot >= 0 || std::max(adj[i].L, v.lb) > kMaxL3) continue;
+        groups[{(v.la + v.lb + adj[i].L) & 1, v.la, v.lb, adj[i].L, m.itcs[v.itc].irrep}].push_back(i);
+    }
+    std::vector<char> taken(adj.size(), 0);
+    for (const auto& gr : groups) {
+        const int la = gr.first[1], lb = gr.first[2], L = gr.first[3];
+        Entry3 en{la, lb, L, {}, {}};
+        bool ok = true;
+        for (size_t i : gr.second) {
+            const VisitQ34& v = adj[i].v;
+            // unrolled visits keep the valid terms only, the others a dense block
+            std::vector<double> b(static_cast<size_t>(2 * la + 1) * (L + 1), 0.0);
+            int at = v.coef;
+            for (int ia = 0; ia <= 2 * la; ++ia)
+                for (int k = 0; k <= L; ++k) {
+                    const bool valid = std::abs(k - (ia - la)) <= lb;
+                    if (valid) b[ia * (L + 1) + k] = m.coef[at];
+                    if (valid || !(v.flags & 4)) ++at;
+                }
+            int combo = m.n_type == 1 ? 0 : la < lb ? 2 * v.sa + v.sb : v.sa + v.sb;
+            if (la == lb && v.sa > v.sb) {
+                // (1, 0) as (0, 1): the factors' m exchanged
+                std::vector<double> x(b.size(), 0.0);
+                for (int ia = 0; ia <= 2 * la; ++ia)
+                    for (int k = 0; k <= L; ++k) {
+                        const int mb = k - (ia - la);
+                        if (std::abs(mb) <= lb) x[(mb + la) * (L + 1) + k] = b[ia * (L + 1) + k];
+                    }
+                b.swap(x);
+            }
+            if (en.block.empty()) en.block = b;
+            size_t big = 0;
+            for (size_t k = 0; k < b.size(); ++k)
+                if (std::abs(en.block[k]) > std::abs(en.block[big])) big = k;
+            const double rho = en.block[big] != 0.0 ? b[big] / en.block[big] : 0.0;
+            double worst = 0.0, top = 0.0;
+            for (size_t k = 0; k < b.size(); ++k) {
+                worst = std::max(worst, std::abs(b[k] - rho * en.block[k]));
+                top = std::max(top, std::abs(b[k]));
+            }
+            if (worst > 1e-13 * top) ok = false;
+            en.use.emplace_back(adj[i].S, combo, v.itc, rho);
+        }
+        if (!ok) continue;
+        for (size_t i : gr.second) taken[i] = 1;
+        out.push_back(std::move(en));
+    }
+    std::vector<PlanVisit> rest;
+    for (size_t i = 0; i < adj.size(); ++i)
+        if (!taken[i]) rest.push_back(adj[i]);
+    adj.swap(rest);
+}
+
+// Records and tasks of the order-3 kernel for one centre type from its entries
+// (grouped by la, lb with ascending L).
+void plan_order3(Model& m, TypeTables& tt, const std::vector<Entry3>& en) {
+    tt.w3_ent = static_cast<int>(en.size());
+    tt.w3.assign(static_cast<size_t>(m.n_fn) * en.size() * 8, 0.0);
+    for (int n = 0; n < m.n_fn; ++n)
+        for (size_t e = 0; e < en.size(); ++e)
+            for (const auto& u : en[e].use)
+                tt.w3[((static_cast<size_t>(n) * en.size() + e) * 2 + std::get<0>(u)) * 4 + std::get<1>(u)] +=
+                    std::get<3>(u) * m.weight[n * m.n_gtinv + std::get<2>(u)];
+    // records from runs of entries with the same la, lb and L rising by 2
+    struct Seg {
+        int k, L0, nL;
+        size_t rb, re;
+    };
+    std::vector<Seg> segs;
+    std::vector<long> cost;  // per record, in VALU instructions
+    const int V = m.n_type == 1 ? 1 : 4;
+    for (int k = 0; k <= m.lmaxq3; ++k)
+        for (int par = 0; par < 2; ++par) {
+            const int L0 = k + ((k + par) & 1);
+            if (L0 > m.lmaxq3) continue;
+            Seg sg{k, L0, (m.lmaxq3 - L0) / 2 + 1, tt.rec3.size(), 0};
+            for (size_t e = 0; e < en.size();) {
+                size_t f = e + 1;
+                auto follows = [&](size_t x) {
+                    return en[x].la == en[e].la && en[x].lb == en[e].lb && en[x].L == en[x - 1].L + 2;
+                };
+                while (f < en.size() && follows(f)) ++f;
+                size_t b = e;
+                while (b < f && (en[b].L < k || ((en[b].L ^ par) & 1))) ++b;
+                const int la = en[e].la, lb = en[e].lb;
+                for (; b < f; b += kQ3N) {
+                    const int N = static_cast<int>(std::min<size_t>(kQ3N, f - b));
+                    Rec3 r{};
+                    r.sig = la | lb << 4 | (N | (m.n_type > 1 && la == lb ? 8 : 0)) << 8 | ((en[b].L - L0) / 2) << 12;
+                    r.coef = static_cast<int32_t>(m.c3q.size());
+                    r.went = static_cast<int32_t>(b);
+                    int nm = 0;
+                    // the kernel's order: ma <= 0, then 1..k, then above k, with
+                    // the sign of a_{l,m} = (-1)^m conj(a_{l,-m})
+                    for (int ma = -la; ma <= la; ++ma) {
+                        const int mb = k - ma;
+                        if (std::abs(mb) > lb) continue;
+                        const int odd = (ma > 0 ? ma : 0) + (mb > 0 ? mb : 0);
+                        for (int j = 0; j < N; ++j)
+                            m.c3q.push_back((odd & 1 ? -1.0 : 1.0) * en[b + j].block[(ma + la) * (en[b + j].L + 1) + k]);
+                        ++nm;
+                    }
+                    if (nm == 0) continue;
+                    const int v = V == 4 && la == lb ? 3 : V;
+                    tt.rec3.push_back(r);
+                    cost.push_back(nm * (4L * v + 2L * v * N + 6) + 4L * m.n_type * v * N + 70);
+                    tt.q3_flops += nm * (6.0 * v + 4.0 * v * N) + 4.0 * m.n_type * v * N;
+                }
+                e = f;
+            }
+            sg.re = tt.rec3.size();
+            segs.push_back(sg);
+        }
+    // cut the sequence of records into twelve ranges of equal cost
+    long total = 0;
+    for (long c : cost) total += c;
+    size_t s = 0, r = 0;
+    long done = 0;
+    std::vector<int> parts(segs.size(), 0);
+    std::vector<std::pair<size_t, size_t>> owner;  // (segment, task)
+    for (int w = 0; w < kWavesPerWg; ++w) {
+        tt.t3_off[w] = static_cast<int32_t>(tt.task3.size());
+        const long goal = total * (w + 1) / kWavesPerWg;
+        while (s < segs.size()) {
+            const Seg& sg = segs[s];
+            r = std::max(r, sg.rb);
+            const size_t b = r;
+            while (r < sg.re && (w + 1 == kWavesPerWg || done + cost[r] / 2 <= goal)) done += cost[r++];
+            if (r == b && r < sg.re) break;  // nothing of this segment fits here
+            owner.emplace_back(s, tt.task3.size());
+            tt.task3.push_back({sg.k, sg.L0, sg.nL, static_cast<int32_t>(b), static_cast<int32_t>(r), 0});
+            ++parts[s];
+            if (r < sg.re) break;
+            ++s;
+        }
+    }
+    tt.t3_off[kWavesPerWg] = static_cast<int32_t>(tt.task3.size());
+    // a divided segment: its last part writes, part i before it adds in round i + 1
+    std::vector<int> seen(segs.size(), 0);
+    for (const auto& o : owner) {
+        const int i = seen[o.first]++;
+        if (i + 1 == parts[o.first]) continue;
+        tt.task3[o.second].mode = i + 1;
+        m.q3_rounds = std::max(m.q3_rounds, i + 1);
+    }
+}
+
+// Moves the order-4 linear families of centre type t whose products the
+// order-4 kernel walks (q4_terms.h) from the visits into its coefficients.
+void extract_order4(Model& m, int t) {
+    TypeTables& tt = m.types[t];
+    const int nt = m.n_type, total = q4_total(nt);
+    // first coefficient of product (i, j, k): its outputs follow by L, then S
+    std::vector<int> at(static_cast<size_t>(729) * nt * nt * nt, -1);
+    auto idx = [&](int i, int j, int k) { return (static_cast<size_t>(i) * 9 * nt + j) * 9 * nt + k; };
+    for (int part = 0, next = 0; part < kQ4Parts; ++part) {
+        int pair = 0;
+        for (int i = 0; i < 9 * nt; ++i)
+            for (int j = i; j < 9 * nt; ++j) {
+                if (!q4_pair_used(nt, i, j) || pair++ % kQ4Parts != part) continue;
+                for (int k = j; k < 9 * nt; ++k)
+                    if (q4_used(i, j, k)) {
+                        at[idx(i, j, k)] = next;
+                        next += q4_outputs(i, j, k) * nt;
+                    }
+            }
+    }
+    std::set<int> moved;
+    for (int i = 0; i < m.n_gtinv; ++i) {
+        const Itc& it = m.itcs[i];
+        if (it.order != 4 || m.prank[i] >= 0 || !((it.type_mask >> t) & 1u)) continue;
+        const Irrep& ir = m.irreps[it.irrep];
+        if (ir.l.back() > 2) continue;
+        int sp[4];
+        for (int k = 0; k < 4; ++k) sp[k] = m.tcp_other[it.tc[k]][t];
+        std::vector<std::pair<int, double>> add;
+        bool ok = true;
+        for (size_t k = 0; k < ir.m.size() && ok; ++k)
+            for (int p = 0; p < 4 && ok; ++p) {
+                if (ir.m[k][p] > 0) continue;  // outputs m <= 0 only
+                int v[3], nv = 0;
+                for (int o = 0; o < 4; ++o)
+                    if (o != p) v[nv++] = sp[o] * 9 + ir.l[o] * (ir.l[o] + 1) + ir.m[k][o];
+                std::sort(v, v + 3);
+                // (the outputs of a product are L = L0, L0 + 2 of its parity)
+                const int M = q4_m(v[0]) + q4_m(v[1]) + q4_m(v[2]), par = (q4_l(v[0]) + q4_l(v[1]) + q4_l(v[2])) & 1;
+                const int L0 = M + ((M ^ par) & 1), f = at[idx(v[0], v[1], v[2])];
+                ok = f >= 0 && ir.l[p] >= L0 && ((ir.l[p] ^ par) & 1) == 0;
+                if (ok) add.emplace_back(f + (ir.l[p] - L0) / 2 * nt + sp[p], ir.c[k]);
+            }
+        if (!ok) continue;
+        if (tt.c4.empty()) tt.c4.assign(static_cast<size_t>(m.n_fn) * total, 0.0);
+        for (int n = 0; n < m.n_fn; ++n)
+            for (const auto& a : add)
+                tt.c4[static_cast<size_t>(n) * total + a.first] += m.weight[n * m.n_gtinv + i] * a.second;
+        moved.insert(i);
+    }
+    std::vector<PlanVisit> rest;
+    for (const PlanVisit& q : tt.plan_adj)
+        if (!(q.v.order == 4 && moved.count(q.v.itc))) rest.push_back(q);
+    tt.plan_adj.swap(rest);
+}
+
+// Order-1/2 families of centre type t by adjoint row (TypeTables::q12r).
+bool rows_order12(Model& m, int t, const std::vector<std::map<std::vector<int>, double>>& cmap) {
+    std::vector<int32_t>& r = m.types[t].q12r;
+    r.assign(2 * (kMaxLQ12 + 1) * 6, kNoSource);
+    for (int i = 0; i < m.n_gtinv; ++i) {
+        const Itc& it = m.itcs[i];
+        const int q = it.order, L = m.irreps[it.irrep].l[0];
+        if (q > 2 || L > kMaxLQ12 || !((it.type_mask >> t) & 1u)) continue;
+        const std::map<std::vector<int>, double>& cm = cmap[it.irrep];
+        const int src = m.prank[i] >= 0 ? m.prank[i] - m.prange[t][0] : -1 - i;
+        for (int p = 0; p < q; ++p) {
+            // dd/da_{sp[p],L,-k} = C a_{other,L,+k}, C = C(-k, k) (p = 0) or
+            // C(k, -k) (p = 1); order 1: C
+            const int S = m.tcp_other[it.tc[p]][t], other = q == 2 ? m.tcp_other[it.tc[1 - p]][t] : 2;
+            int32_t* e = &r[(S * (kMaxLQ12 + 1) + L) * 6 + 2 * other];
+            if (e[0] != kNoSource && e[0] != src) return false;
+            const bool fresh = e[0] == kNoSource;
+            if (fresh) {
+                e[0] = src;
+                e[1] = static_cast<int32_t>(m.coef.size());
+                m.coef.resize(m.coef.size() + L + 1, 0.0);
+            }
+            for (int k = 0; k <= L; ++k)
+                m.coef[e[1] + k] += q == 1 ? lookup(cm, {0})
+                                           : lookup(cm, p == 0 ? std::vector<int>{-k, k} : std::vector<int>{k, -k});
+        }
+    }
+    return true;
+}
+
 // Builds the flattened visit tables for centre type t.
-void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<int>, double>>& cmap) {
+void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<int>, double>>& cmap,
+                       std::vector<Entry3>& entries) {
     TypeTables tt;
     std::vector<std::vector<VisitQ12>> by_l(m.maxl + 1);
     using Pending = PlanVisit;
@@ -542,30 +797,6 @@ void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<i
                 for (int m0 = -L; m0 <= L; ++m0) push_coef(lookup(cm, {m0, -m0}));
             }
             by_l[L].push_back(v);
-            if (L <= m.q12_fuse || (L > m.lmax3 && L <= m.q12_fuse_hi)) {
-                // the same family's adjoint in the order-3/4 kernel, one visit
-                // per factor position p: dd/da_{sp[p],L,-k} = C a_{other,L,+k}
-                // with C = C(-k, k) (p = 0) or C(k, -k) (p = 1)
-                for (int pp = 0; pp < q; ++pp) {
-                    VisitQ34 f{};
-                    f.order = q;
-                    f.itc = i;
-                    f.la = q == 2 ? L : 0;
-                    f.sa = q == 2 ? sp[1 - pp] : 0;
-                    f.pslot = pslot;
-                    f.flags = 2 | 4;
-                    f.coef = static_cast<int>(m.coef.size());
-                    f.dcoef = -1;
-                    if (q == 1) {
-                        push_coef(lookup(cm, {0}));
-                    } else {
-                        for (int k = 0; k <= L; ++k) push_coef(lookup(cm, pp == 0 ? std::vector<int>{-k, k}
-                                                                                   : std::vector<int>{k, -k}));
-                    }
-                    const int nc = q == 1 ? 1 : L + 1;
-                    adj.push_back({sp[pp], L, f, nc, nc});
-                }
-            }
             continue;
         }
         if (q >= 5) {
@@ -757,14 +988,67 @@ void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<i
         }
         adj.swap(merged);
     }
+    extract_order3(m, adj, entries);
+    tt.plan_adj = std::move(adj);
+    tt.plan_feat = std::move(feat);
+    m.types[t] = std::move(tt);
+}
+
+// Fused order-1/2 adjoint visits and row markers of centre type t, once the
+// order-3/4 kernel's tile (lmax_t) is known.
+void add_fused_rows(Model& m, int t, const std::vector<std::map<std::vector<int>, double>>& cmap) {
+    std::vector<PlanVisit>& adj = m.types[t].plan_adj;
+    auto push_coef = [&](double v) { m.coef.push_back(v); };
+    std::map<std::array<int, 11>, size_t> first;
+    for (int i = 0; i < m.n_gtinv; ++i) {
+        const Itc& it = m.itcs[i];
+        const int q = it.order;
+        if (q > 2 || !((it.type_mask >> t) & 1u)) continue;
+        const Irrep& ir = m.irreps[it.irrep];
+        const std::map<std::vector<int>, double>& cm = cmap[it.irrep];
+        const int L = ir.l[0], pslot = m.prank[i];
+        if (!(L <= m.q12_fuse || (L > m.lmax_t && L <= m.q12_fuse_hi))) continue;
+        int sp[2] = {0, 0};
+        for (int k = 0; k < q; ++k) sp[k] = m.tcp_other[it.tc[k]][t];
+        // the family's adjoint in the order-3/4 kernel, one visit per factor
+        // position p: dd/da_{sp[p],L,-k} = C a_{other,L,+k} with C = C(-k, k)
+        // (p = 0) or C(k, -k) (p = 1); positions that add the same products
+        // into the same row become one visit
+        for (int pp = 0; pp < q; ++pp) {
+            VisitQ34 f{};
+            f.order = q;
+            f.itc = i;
+            f.la = q == 2 ? L : 0;
+            f.sa = q == 2 ? sp[1 - pp] : 0;
+            f.pslot = pslot;
+            f.flags = 2 | 4;
+            f.coef = static_cast<int>(m.coef.size());
+            f.dcoef = -1;
+            if (q == 1) {
+                push_coef(lookup(cm, {0}));
+            } else {
+                for (int k = 0; k <= L; ++k)
+                    push_coef(lookup(cm, pp == 0 ? std::vector<int>{-k, k} : std::vector<int>{k, -k}));
+            }
+            const int nc = q == 1 ? 1 : L + 1;
+            const std::array<int, 11> key{sp[pp], L, i, q, f.la, f.sa, 0, 0, 0, 0, f.flags};
+            auto at = first.find(key);
+            if (at == first.end()) {
+                first.emplace(key, adj.size());
+                adj.push_back({sp[pp], L, f, nc, nc});
+            } else {
+                for (int k = 0; k < nc; ++k) m.coef[adj[at->second].v.coef + k] += m.coef[f.coef + k];
+            }
+        }
+    }
     // every fused row is written by the order-3/4 kernel (the order-1/2
-    // kernel skips it): rows no family adds to get an empty marker visit,
-    // so their G is written as zero
+    // kernel skips it): rows no family adds to get an empty marker visit, so
+    // their G is written as zero
     for (int S = 0; S < m.n_type; ++S)
         for (int L = 0; L <= std::max(m.q12_fuse, m.q12_fuse_hi); ++L) {
-            if (!(L <= m.q12_fuse || (L > m.lmax3 && L <= m.q12_fuse_hi))) continue;
+            if (!(L <= m.q12_fuse || (L > m.lmax_t && L <= m.q12_fuse_hi))) continue;
             bool any = false;
-            for (const Pending& q : adj) any = any || (q.S == S && q.L == L);
+            for (const PlanVisit& q : adj) any = any || (q.S == S && q.L == L);
             if (!any) {
                 VisitQ34 z{};
                 z.order = 0;
@@ -774,9 +1058,6 @@ void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<i
                 adj.push_back({S, L, z, 0, 0});
             }
         }
-    tt.plan_adj = std::move(adj);
-    tt.plan_feat = std::move(feat);
-    m.types[t] = std::move(tt);
 }
 
 }  // namespace
@@ -966,7 +1247,6 @@ bool load_pair_model(std::istream& in, Model& m, std::string& err, bool strict_c
     m.n_p = m.n_des;
     m.maxl = 0;
     m.n_lmh = 1;
-    m.n_lmh3 = 1;
     m.lmax3 = 0;
     m.has_order34 = false;
     m.has_feat34 = false;
@@ -1179,12 +1459,6 @@ bool load_model(const std::string& path, const GtinvTable& table, Model& m, std:
             m.has_order34 = true;
             m.lmax3 = std::max(m.lmax3, ir.l.back());
         }
-    m.n_lmh3 = n_lmh_of(m.lmax3);
-    // order-1/2 adjoint rows inside the order-3/4 kernel: those within its
-    // LDS tile and unrolled signatures (l <= min(lmax3, 8)), and those above
-    // the tile up to kMaxLQ12 (a_nlm read from HBM)
-    m.q12_fuse = m.has_order34 ? std::min(m.lmax3, kUnrollCap3) : -1;
-    m.q12_fuse_hi = m.has_order34 ? std::min(m.maxl, kMaxLQ12) : -1;
     m.lmaxh = -1;
     for (const Irrep& ir : m.irreps)
         if (ir.l.size() >= 5) m.lmaxh = std::max(m.lmaxh, ir.l.back());
@@ -1196,7 +1470,35 @@ bool load_model(const std::string& path, const GtinvTable& table, Model& m, std:
         for (size_t t = 0; t < m.irreps[i].m.size(); ++t) cmap[i][m.irreps[i].m[t]] = m.irreps[i].c[t];
     m.coef.clear();
     m.types.assign(m.n_type, TypeTables());
-    for (int t = 0; t < m.n_type; ++t) build_type_tables(m, t, cmap);
+    m.c3q.clear();
+    std::vector<std::vector<Entry3>> entries(m.n_type);
+    for (int t = 0; t < m.n_type; ++t) build_type_tables(m, t, cmap, entries[t]);
+    m.lmaxq3 = -1;
+    for (int t = 0; t < m.n_type; ++t)
+        for (const Entry3& e : entries[t]) m.lmaxq3 = std::max({m.lmaxq3, e.L, e.lb});
+    m.q3_rounds = 0;
+    if (m.lmaxq3 >= 0)
+        for (int t = 0; t < m.n_type; ++t) {
+            plan_order3(m, m.types[t], entries[t]);
+            extract_order4(m, t);
+            if (!rows_order12(m, t, cmap)) {
+                err = "internal: two order-1/2 families of one species pair and l";
+                return false;
+            }
+        }
+    // tile of the order-3/4 adjoint kernel: the visits it keeps
+    m.lmax_t = 0;
+    for (int t = 0; t < m.n_type; ++t)
+        for (const PlanVisit& q : m.types[t].plan_adj)
+            m.lmax_t = std::max({m.lmax_t, q.L, q.v.la, q.v.lb, q.v.lc});
+    // without the order-3 kernel: order-1/2 adjoint rows inside the order-3/4
+    // kernel, those within its LDS tile and unrolled signatures (l <=
+    // min(lmax_t, 8)), and those above the tile up to kMaxLQ12 (a_nlm read
+    // from HBM)
+    const bool fuse = m.has_order34 && m.lmaxq3 < 0;
+    m.q12_fuse = fuse ? std::min(m.lmax_t, kUnrollCap3) : -1;
+    m.q12_fuse_hi = fuse ? std::min(m.maxl, kMaxLQ12) : -1;
+    for (int t = 0; t < m.n_type; ++t) add_fused_rows(m, t, cmap);
     plan_q34(m, m.plan_region, m.plan_visit, m.plan_pair);
     m.has_feat34 = false;
     for (const auto& tt : m.types)

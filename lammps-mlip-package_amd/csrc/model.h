@@ -140,6 +140,22 @@ struct VisitHi {
     int32_t tbeg, tend;         // term range
 };
 
+// Order-3 linear families in the by-output-m kernel (q3.hip): a record is one
+// (la, lb) and up to kQ3N output L = L0 + 2 (i0 + j) of a segment; sig packs
+// la, lb, N (| 8 where la = lb) and i0 in 4 bits each; coefficients [ma][j] in the
+// kernel's order of ma with the conjugation signs; went: first of its entries
+// in the weight table [n][entry][S][species combination].
+constexpr int kQ3N = 4;
+struct Rec3 {
+    int32_t sig, coef, went;
+};
+// A wave's part of segment (output m = -k, L = L0, L0 + 2, .. of nL): mode 0
+// writes the rows, mode r adds them in round r.
+constexpr int kNoSource = INT32_MIN;
+struct Task3 {
+    int32_t k, L0, nL, rbeg, rend, mode;
+};
+
 // Merged order-5/6 adjoint row of the linear families: all terms of one
 // (output S, L, m = -k; family order), over every family and factor position
 // that adds to it.  The table's order-5/6 factors are few (l <= 1: eight a per
@@ -186,6 +202,22 @@ struct TypeTables {
     std::vector<HiRow> hi_rows;
     std::vector<int32_t> hi_rterm;
     std::vector<double> hi_rcoef;
+    // order-3 linear families by output m (Rec3, Task3): tasks of wave w are
+    // t3_off[w] .. t3_off[w + 1], weights [n][w3_ent][2][4]
+    std::vector<Rec3> rec3;
+    std::vector<Task3> task3;
+    std::array<int32_t, kWavesPerWg + 1> t3_off{};
+    std::vector<double> w3;
+    int w3_ent = 0;
+    double q3_flops = 0.0;             // operations per (centre, radial index)
+    // order-4 linear families as products of three variables (q4_terms.h):
+    // [n][q4_total] coefficients; empty: none
+    std::vector<double> c4;
+    // order-1/2 families of each adjoint row for the order-3 kernel: [S][L <=
+    // kMaxLQ12][6] = H source and coefficient offset of factor species 0, of 1,
+    // and of the order-1 family (L = 0); a source is the polynomial rank from
+    // the species' first, -1 - family for a linear weight, or kNoSource
+    std::vector<int32_t> q12r;
     // order 3/4 visits before grouping (plan_q34 groups them)
     std::vector<PlanVisit> plan_adj, plan_feat;
 };
@@ -211,7 +243,13 @@ struct Model {
     // GPU-side layout
     int lmax3 = 0;             // largest l among order>=3 irreps (LDS tile)
     int n_lmh = 0;             // (maxl+1)(maxl+2)/2, m<=0 entries of a_nlm
-    int n_lmh3 = 0;            // same for lmax3
+    int lmax_t = 0;            // largest l of the visits left to the order-3/4 adjoint kernel (its LDS tile)
+    // largest l of the order-3 linear families; >= 0: the order-3 kernel (q3.hip)
+    // runs and writes every adjoint row up to min(maxl, kMaxLQ12), order-1/2
+    // families included; -1: none, the order-3/4 and order-1/2 kernels do
+    int lmaxq3 = -1;
+    std::vector<double> c3q;   // their coefficients, all types
+    int q3_rounds = 0;
     int n_pitc = 0;            // itcs whose features enter polynomial products
     std::vector<int> prank;    // itc -> rank among polynomial itcs or -1
     int n_p = 0;               // n_fn * n_pitc; feature (n, rank) = n * n_pitc + rank
@@ -224,10 +262,10 @@ struct Model {
     std::vector<TypeTables> types;
     bool has_order34 = false;
     bool has_feat34 = false;
-    // order-1/2 adjoint rows L <= q12_fuse run inside the order-3/4 adjoint
+    // order-1/2 adjoint rows L <= q12_fuse (within lmax_t) run inside the order-3/4 adjoint
     // kernel, on its LDS tile (-1: none; the order-1/2 kernel takes the rest)
     int q12_fuse = -1;
-    // ... and so do the rows above the order-3/4 tile, lmax3 < L <= q12_fuse_hi
+    // ... and so do the rows above its tile, lmax_t < L <= q12_fuse_hi
     // (their a_nlm read from HBM)
     int q12_fuse_hi = -1;
     // radial-only style (des_type pair): features f = tc * n_fn + n
@@ -269,6 +307,6 @@ bool load_model(const std::string& path, const GtinvTable& table, Model& m, std:
                 bool strict_count = true);
 
 inline int lmh_index(int l, int m) { return l * (l + 1) / 2 + l + m; }  // m <= 0
-inline int n_lmh_of(int lmax) { return (lmax + 1) * (lmax + 2) / 2; }
+constexpr int n_lmh_of(int lmax) { return (lmax + 1) * (lmax + 2) / 2; }
 
 }  // namespace mlip

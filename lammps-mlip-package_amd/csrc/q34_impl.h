@@ -30,12 +30,12 @@ constexpr int kQ34Threads = 64 * kWavesPerWg;
 
 struct Tile {
     const double2* As;  // [s][lm][lane] (re, im): one 16-byte LDS read per entry
-    int nlmh3;
+    int nlmh3;          // entries per species in the tile
     int lane;
     const double* Ag;   // a_nlm of the (block, n) in HBM: [s][lm][re, im][lane]
     int nlmh;
     // the row (s, l) of a level above the LDS tile (fused order-1/2 rows
-    // l > lmax3) in HBM: entry m <= 0 at (l - |m|) 2 kBlock from the
+    // l > lmax_t) in HBM: entry m <= 0 at (l - |m|) 2 kBlock from the
     // returned base.  The base is opaque, so a visit keeps one pointer rather
     // than every entry's address hoisted out of the visit loop.
     __device__ __forceinline__ const double* rowg(int s, int l) const {
@@ -500,8 +500,8 @@ __device__ __forceinline__ void q34_group_pair(const Tile& T, const DevModel& M,
     close0(cls0);
     close1(cls1);
     if (uniform(g.nparts) == 1) {
-        // a fused row (L <= q12_fuse) is written, any other added to
-        const bool first = L <= M.q12_fuse;
+        // a fused row no kernel wrote before is written, any other added to
+        const bool first = q34_writes(M, L);
         double* G0 = g_row_base(M, S, blk, n, T.lane);
         double* G1 = G0 + static_cast<size_t>(M.n_lmh) * 2 * kBlock;
 #pragma unroll
@@ -630,8 +630,8 @@ __device__ __forceinline__ void q34_group(const Tile& T, const DevModel& M, cons
     if (!FEAT) {
         close_class(cls_cur);
         if (uniform(g.nparts) == 1) {
-            // fused rows are this kernel's alone: the first kernel writes them
-            const bool first = !DYN && L <= M.q12_fuse;
+            // fused rows no kernel wrote before are written
+            const bool first = !DYN && q34_writes(M, L);
 #pragma unroll
             for (int k = 0; k <= L; ++k) {
                 const size_t ir = a_index(M, blk, n, Sx, lmh(L, -k), 0, T.lane);
@@ -655,7 +655,7 @@ __device__ __forceinline__ void q34_group(const Tile& T, const DevModel& M, cons
     }
 }
 
-// A fused order-1/2 row above the LDS tile (lmax3 < L <= q12_fuse_hi): its
+// A fused order-1/2 row above the LDS tile (lmax_t < L <= q12_fuse_hi): its
 // visits are order 1/2 only and read a_{s_a,L,+k} from HBM (each a 64-lane
 // coalesced line); energies by the same Euler classes, G written like the
 // other fused rows (first write, or a partial row of a split row).  One
@@ -725,11 +725,13 @@ __device__ __forceinline__ void q34_group_glob(const Tile& T, const DevModel& M,
     if (uniform(g.nparts) == 1) {
         double* Gs = g_row_base(M, S, blk, n, T.lane) + static_cast<size_t>(Sx) * M.n_lmh * 2 * kBlock +
                      static_cast<size_t>(L * (L + 1) / 2) * 2 * kBlock;
+        const bool first = q34_writes(M, L);
 #pragma unroll
         for (int k = 0; k <= LM; ++k) {
             if (k <= L) {
-                Gs[(2 * (L - k)) * kBlock] = gr[k];  // lmh(L, -k) = L (L + 1) / 2 + L - k
-                Gs[(2 * (L - k) + 1) * kBlock] = gi[k];
+                double* g = Gs + (2 * (L - k)) * kBlock;  // lmh(L, -k) = L (L + 1) / 2 + L - k
+                g[0] = first ? gr[k] : g[0] + gr[k];
+                g[kBlock] = first ? gi[k] : g[kBlock] + gi[k];
             }
         }
     } else {
@@ -748,7 +750,7 @@ __device__ __forceinline__ void q34_group_glob(const Tile& T, const DevModel& M,
 __device__ __forceinline__ void q34_combine(const DevModel& M, const DevSystem& S, const GroupQ34& g, int blk, int n,
                                             int lane, const double* red, bool dyn) {
     const int L = uniform(g.L), Sx = uniform(g.S), np = uniform(g.nparts);
-    const bool first = !dyn && q12_fused(M, L);  // a fused row: written, not added to
+    const bool first = !dyn && q34_writes(M, L);  // written, not added to
     // a species-paired group keeps rows 0 and 1 one after the other per part
     const int nrows = Sx == kPairedRows ? 2 : 1;
     const int rowlen = (L + 1) * 2 * kBlock;
@@ -784,7 +786,8 @@ __global__ __launch_bounds__(kQ34Threads) void k_q34(DevModel M, DevSystem S) {
     extern __shared__ __attribute__((aligned(16))) double As[];
     const int blk = blockIdx.x, n = blockIdx.y;
     const int t = S.block_type[blk];
-    const int per_s = M.n_lmh3 * kBlock;  // entries (re, im) per species
+    const int ltile = FEAT ? M.lmax3 : M.lmax_t;  // largest l of the tile
+    const int per_s = n_lmh_of(ltile) * kBlock;   // entries (re, im) per species
     double2* As2 = reinterpret_cast<double2*>(As);
     for (int s = 0; s < M.n_type; ++s) {
         // global [lm][re,im][lane] -> LDS [lm][lane](re, im)
@@ -797,7 +800,7 @@ __global__ __launch_bounds__(kQ34Threads) void k_q34(DevModel M, DevSystem S) {
     double* red = As + 2 * M.n_type * per_s;  // partial rows of split groups
     __syncthreads();
     const int wave = uniform(threadIdx.x >> 6);
-    Tile T{As2, M.n_lmh3, static_cast<int>(threadIdx.x & 63), S.A + a_index(M, blk, n, 0, 0, 0, 0), M.n_lmh};
+    Tile T{As2, n_lmh_of(ltile), static_cast<int>(threadIdx.x & 63), S.A + a_index(M, blk, n, 0, 0, 0, 0), M.n_lmh};
     cptr<GroupQ34> groups = as_const(FEAT ? M.gfeat : M.gadj);
     const int gb = FEAT ? M.gfeat_beg[t] : M.gadj_beg[t];
     const int ge = FEAT ? M.gfeat_end[t] : M.gadj_end[t];
@@ -808,8 +811,8 @@ __global__ __launch_bounds__(kQ34Threads) void k_q34(DevModel M, DevSystem S) {
         const int L = uniform(g.L);
         // above the unrolled signatures the first kernel has only fused
         // order-1/2 rows (adjoint)
-        if (!DYN && L > kMaxLUnrolled && (FEAT || L <= M.lmax3)) continue;
-        if (!FEAT && L > M.lmax3) {
+        if (!DYN && L > kMaxLUnrolled && (FEAT || L <= ltile)) continue;
+        if (!FEAT && L > ltile) {
             // fused order-1/2 row above the tile: the first kernel's
             if constexpr (!FEAT && !DYN) q34_group_glob<kMaxLQ12>(T, M, S, g, blk, n, red, eacc);
             continue;
@@ -857,14 +860,14 @@ __global__ __launch_bounds__(kQ34Threads) void k_q34(DevModel M, DevSystem S) {
             for (int gi = gb; gi < ge; ++gi) {
                 const GroupQ34 g = groups[gi];
                 if (uniform(g.wave) != wave || uniform(g.nparts) == 1 || uniform(g.part) != 0) continue;
-                if (!DYN && uniform(g.L) > kMaxLUnrolled && uniform(g.L) <= M.lmax3) continue;
-                if (DYN && uniform(g.L) > M.lmax3) continue;  // the first kernel's
+                if (!DYN && uniform(g.L) > kMaxLUnrolled && uniform(g.L) <= ltile) continue;
+                if (DYN && uniform(g.L) > ltile) continue;  // the first kernel's
                 if (DYN && uniform(g.S) == kPairedRows) continue;  // the unrolled kernel's
                 q34_combine(M, S, g, blk, n, T.lane, red, DYN);
             }
         }
         double* e = &S.Eq34[(((size_t)blk * M.n_fn + n) * kWavesPerWg + wave) * kBlock + T.lane];
-        if (DYN)
+        if (DYN || M.lmaxq3 >= 0)
             *e += eacc;
         else
             *e = eacc;
@@ -873,7 +876,7 @@ __global__ __launch_bounds__(kQ34Threads) void k_q34(DevModel M, DevSystem S) {
 
 template <bool FEAT, bool DYN>
 hipError_t launch(const DevModel& m, const DevSystem& s, hipStream_t st) {
-    const size_t lds = sizeof(double) * (static_cast<size_t>(m.n_type) * m.n_lmh3 * 2 * kBlock + (FEAT ? 0 : m.q34_red));
+    const size_t lds = sizeof(double) * (static_cast<size_t>(m.n_type) * n_lmh_of(FEAT ? m.lmax3 : m.lmax_t) * 2 * kBlock + (FEAT ? 0 : m.q34_red));
     if (lds > lds_limit()) return hipErrorInvalidConfiguration;
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_q34<FEAT, DYN>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(64 * kHiWaves) void k_qhigh_rows(DevModel M, DevSys
             // the rows of one output (orders 5 and 6) add to the same G entry
             if (uniform(R.out) % kHiWaves != wave) continue;
             const int Sx = uniform(R.S), L = uniform(R.L), k = uniform(R.k);
-            const double iq = 1.0 / uniform(R.order), scale = M.hi_split ? iq : 1.0;
+            const double iq = 1.0 / uniform(R.order), scale = M.split ? iq : 1.0;
             double gr = 0.0, gi = 0.0;
 #pragma unroll
             for (int w = 0; w < kHiWaves; ++w) {
