@@ -90,6 +90,8 @@ struct DevModel {
     const double* weight_e;
     const int32_t* pdeg;
     const double* wmat;
+    const double* wmat_e;   // poly_fused models: W_ab / (q_a + q_b) and lin_a / q_a
+    const double* lin_e;
     int32_t wofs[2], wdim[2];
     // radial-only style
     int pair_model;         // 1: features sum_j g_n(r) per type combination

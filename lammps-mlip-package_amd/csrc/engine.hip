@@ -244,7 +244,23 @@ bool upload_model(mlip_ctx* c) {
     if (!m.pair_model)
         for (int f = 0; f < m.n_des && f < static_cast<int>(wsplit.size()); ++f)
             wsplit[f] /= m.itcs[f % m.n_gtinv].order;
+    // ... and of the quadratic polynomial: W_ab / (q_a + q_b), lin_a / q_a
+    std::vector<double> we, line;
+    if (!m.pair_model && m.n_p > 0 && c3w.empty()) {
+        we = wc;
+        line = linc;
+        for (int t = 0; t < 2; ++t) {
+            const int32_t* q = pdeg.data() + static_cast<size_t>(t) * n_pr;
+            for (int a = 0; a < c->wdim[t]; ++a) {
+                line[static_cast<size_t>(t) * n_pr + a] /= q[a];
+                double* row = we.data() + c->wofs[t] + static_cast<size_t>(a) * c->wdim[t];
+                for (int b = 0; b < c->wdim[t]; ++b) row[b] /= q[a] + q[b];
+            }
+        }
+    }
     bool ok = upload(c, c->d_coef, m.coef.data(), m.coef.size(), "coefficients") &&
+              upload(c, c->d_wmat_e, we.data(), we.size(), "split quadratic form") &&
+              upload(c, c->d_line, line.data(), line.size(), "split linear poly weights") &&
               upload(c, c->d_weight_e, wsplit.data(), wsplit.size(), "split weights") &&
               upload(c, c->d_pdeg, pdeg.data(), pdeg.size(), "feature degrees") &&
               upload(c, c->d_weight, m.weight.data(), m.weight.size(), "weights") &&
@@ -387,6 +403,8 @@ bool upload_model(mlip_ctx* c) {
     dm.weight_e = c->d_weight_e.p;
     dm.pdeg = c->d_pdeg.p;
     dm.wmat = c->d_wmat.p;
+    dm.wmat_e = c->d_wmat_e.p;
+    dm.lin_e = c->d_line.p;
     for (int t = 0; t < 2; ++t) {
         dm.wofs[t] = static_cast<int32_t>(c->wofs[t]);
         dm.wdim[t] = c->wdim[t];
@@ -784,7 +802,20 @@ bool run_atom_split(mlip_ctx* c, double* epv, double* evat) {
         me.weight = c->d_weight_e.p;
         me.split = 1;
         se.H = se.Hq;
-        if (me.n_p > 0) run("poly_split", launch_poly_split(me, se, st));
+        if (me.poly_fused) {
+            // without cubic terms He = lin / q + D W' with W'_ab = W_ab / (q_a +
+            // q_b): the quadratic-form product with split weights (its energy
+            // partials go to the old H, which this pass no longer reads); one
+            // wave per centre over W took 982 us at 864 atoms of the order-4 model
+            DevModel mg = me;
+            DevSystem sg = c->ds;
+            mg.wmat = me.wmat_e;
+            mg.lin_p = me.lin_e;
+            std::swap(sg.H, sg.Hq);
+            run("poly_split", launch_poly_gemm(mg, sg, c->nblk_type, st));
+        } else if (me.n_p > 0) {
+            run("poly_split", launch_poly_split(me, se, st));
+        }
         if (ok) run("q12_split", launch_q12(me, se, false, st));
         if (ok && mm.has_order34) run("q34_split", launch_q34_adj(me, se, st));
         if (ok && mm.has_hi) run("qhigh_split", launch_qhigh(me, se, false, st));
@@ -1067,7 +1098,7 @@ void mlip_destroy(mlip_ctx* c) {
         (void)hipEventDestroy(e.a);
         (void)hipEventDestroy(e.b);
     }
-    DBuf<double>* dbs[] = {&c->d_coef, &c->d_weight, &c->d_weight_e, &c->d_wmat, &c->d_linp, &c->d_c3w, &c->x,
+    DBuf<double>* dbs[] = {&c->d_coef, &c->d_weight, &c->d_weight_e, &c->d_wmat_e, &c->d_line, &c->d_wmat, &c->d_linp, &c->d_c3w, &c->x,
                            &c->pshift, &c->epv, &c->evat,
                            &c->A, &c->G, &c->D, &c->Hq, &c->H, &c->Ep, &c->Eq12, &c->Eq34, &c->gpair,
                            &c->vown, &c->f, &c->e_slot, &c->red, &c->out, &c->sout};

@@ -57,7 +57,7 @@ struct mlip_ctx {
     hipStream_t stream = nullptr;
     int device = 0;
     // model tables
-    mlip::DBuf<double> d_coef, d_weight, d_wmat, d_linp, d_c3w, d_weight_e;
+    mlip::DBuf<double> d_coef, d_weight, d_wmat, d_linp, d_c3w, d_weight_e, d_wmat_e, d_line;
     mlip::DBuf<mlip::VisitQ12> d_q12;
     mlip::DBuf<mlip::FeatQ12> d_fq12;
     mlip::DBuf<int32_t> d_q12off, d_c3off, d_c3bc, d_pdeg;

@@ -301,22 +301,6 @@ __global__ __launch_bounds__(256) void k_poly_split(DevModel M, DevSystem S) {
     }
 }
 
-// Per position k: half the energy share and virial of every pair in its
-// gather list (centre or neighbor side), in list order.
-__global__ __launch_bounds__(256) void k_atom_ev(DevSystem S, const double* __restrict__ epv, double* evat) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= S.nall) return;
-    double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-    for (int e = S.goff[k]; e < S.gend[k]; ++e) {
-        const int code = S.gent[e];
-        const int64_t p = code > 0 ? code - 1 : -code - 1;
-#pragma unroll
-        for (int c = 0; c < 7; ++c) acc[c] += epv[7 * p + c];
-    }
-#pragma unroll
-    for (int c = 0; c < 7; ++c) evat[7 * (size_t)k + c] = 0.5 * acc[c];
-}
-
 // ---------------------------------------------------------------- gather
 // kGatherLanes lanes per position: lane u takes entries u, u + 16, ... of the
 // position's list, four at a time (their pair forces loaded together), and
@@ -367,6 +351,29 @@ __global__ __launch_bounds__(256) void k_gather(DevSystem S) {
         fz += __shfl_xor(fz, off);
     }
     if (u < 3) S.f[3 * (size_t)k + u] = u == 0 ? fx : u == 1 ? fy : fz;
+}
+
+// Per position: half the energy share and virial of every pair in its gather
+// list (centre or neighbor side), lanes and order as k_gather (one lane per
+// position: 200 us at 864 atoms and their ghosts).
+__global__ __launch_bounds__(256) void k_atom_ev(DevSystem S, const double* __restrict__ epv, double* evat) {
+    const int u = threadIdx.x % kGatherLanes;
+    const int k = static_cast<int>((blockIdx.x * 256LL + threadIdx.x) / kGatherLanes);
+    if (k >= S.nall) return;
+    double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 2
+    for (int e = S.goff[k] + u; e < S.gend[k]; e += kGatherLanes) {
+        const int code = S.gent[e];
+        const int64_t p = code > 0 ? code - 1 : -code - 1;
+#pragma unroll
+        for (int c = 0; c < 7; ++c) acc[c] += epv[7 * p + c];
+    }
+#pragma unroll
+    for (int c = 0; c < 7; ++c) {
+#pragma unroll
+        for (int off = kGatherLanes / 2; off > 0; off >>= 1) acc[c] += __shfl_xor(acc[c], off);
+        if (u == c) evat[7 * (size_t)k + c] = 0.5 * acc[c];
+    }
 }
 
 // ---------------------------------------------------------------- energy / virial
@@ -541,7 +548,8 @@ hipError_t launch_poly_split(const DevModel& m, const DevSystem& s, hipStream_t 
 
 hipError_t launch_atom_ev(const DevSystem& s, const double* epv, double* evat, hipStream_t st) {
     if (s.nall == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_atom_ev, dim3((s.nall + 255) / 256), dim3(256), 0, st, s, epv, evat);
+    const int64_t threads = static_cast<int64_t>(s.nall) * kGatherLanes;
+    hipLaunchKernelGGL(k_atom_ev, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, st, s, epv, evat);
     return launched();
 }
 

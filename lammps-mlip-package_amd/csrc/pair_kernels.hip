@@ -864,23 +864,39 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NF > 16 ? 1 
 }
 
 // ---------------------------------------------------------------- per-pair energy share
-// Thread per directed pair of the slot's centre (64 threads, FP64):
+// Workgroup per centre, thread per directed pair of it (FP64):
 //   e_p = sum_{n,l,m<=0} w_m Re(G_{s,n,l,m} g_n(r) Y_lm(del)),  w_0 = 1, w_{m<0} = 2
-// with G read from HBM (every lane of the workgroup reads the same entry),
 // plus the pair's virial del (x) (-g_p) from the force pass.  With G holding
 // the split adjoint, e_p + e_p' over the two directions of a pair is the
-// reference's pair energy evdwl (pair_mlip_gtinv.cpp:240-253).
-__global__ __launch_bounds__(64) void k_pair_energy(DevModel M, DevSystem S, double* __restrict__ epv) {
+// reference's pair energy evdwl (pair_mlip_gtinv.cpp:240-253).  The centre's G
+// is staged in LDS as [s][lm][n](re, im) and read as broadcasts (GL; models
+// whose tile does not fit read it from HBM).  Bound: those LDS reads, one per
+// two FMAs.  One wave per centre with every G entry from HBM took 999 us at
+// 864 atoms of the order-4 model.
+constexpr int kPairEnergyThreads = 192;
+
+template <int NF, bool GL>
+__global__ __launch_bounds__(kPairEnergyThreads) void k_pair_energy(DevModel M, DevSystem S, double* __restrict__ epv) {
+    extern __shared__ double2 pe_tile[];
     const int slot = xcd_slot(blockIdx.x, S.nblocks);
     if (slot < 0) return;
     const int atom = S.atom_of_slot[slot];
     if (atom < 0) return;
     const int blk = slot / kBlock, lane = slot % kBlock;
-    const int nfn = M.n_fn, maxl = M.maxl;
+    const int nfn = M.n_fn, maxl = M.maxl, nlmh = M.n_lmh;
+    if (GL) {
+#pragma unroll 4
+        for (int k = threadIdx.x; k < M.n_type * nlmh * NF; k += kPairEnergyThreads) {
+            const int n = k % NF, lm = (k / NF) % nlmh, s = k / (NF * nlmh), nr = n < nfn ? n : nfn - 1;
+            const double re = S.G[a_index(M, blk, nr, s, lm, 0, lane)], im = S.G[a_index(M, blk, nr, s, lm, 1, lane)];
+            pe_tile[k] = n < nfn ? double2{re, im} : double2{0.0, 0.0};
+        }
+        __syncthreads();
+    }
     const YTab<double>* yt = M.yt64;
     const double pir = kPiRef / M.cutoff;
     const int p0 = S.poff[atom], p1 = S.pend[atom];
-    for (int64_t p = p0 + threadIdx.x; p < p1; p += 64) {
+    for (int64_t p = p0 + threadIdx.x; p < p1; p += kPairEnergyThreads) {
         const PairDel pg = pair_del(M, S, atom, p);
         double e = 0.0;
         double v[6] = {0, 0, 0, 0, 0, 0};
@@ -889,11 +905,13 @@ __global__ __launch_bounds__(64) void k_pair_energy(DevModel M, DevSystem S, dou
             const double ir = 1.0 / pg.r;
             const double x = pg.dx * ir, y = pg.dy * ir, z = pg.dz * ir;
             const double fc = 0.5 * (cos(pir * pg.r) + 1.0);
-            double gn[kMaxFn];
-            for (int n = 0; n < kMaxFn; ++n) {
+            double gn[NF];
+#pragma unroll
+            for (int n = 0; n < NF; ++n) {
                 const double dd = pg.r - M.mu[n];
                 gn[n] = n < nfn ? exp(-M.beta[n] * (dd * dd)) * fc : 0.0;
             }
+            const double2* gs = pe_tile + static_cast<size_t>(spec) * nlmh * NF;
             double cr = 1.0, ci = 0.0;  // conj(u)^m
             for (int m = 0; m <= maxl; ++m) {
                 double q1 = 0.0, q2 = 0.0, sr = 0.0, si = 0.0;
@@ -903,9 +921,18 @@ __global__ __launch_bounds__(64) void k_pair_energy(DevModel M, DevSystem S, dou
                     q2 = q1;
                     q1 = q;
                     double gr = 0.0, gi = 0.0;
-                    for (int n = 0; n < nfn; ++n) {
-                        gr = fma(gn[n], S.G[a_index(M, blk, n, spec, lm, 0, lane)], gr);
-                        gi = fma(gn[n], S.G[a_index(M, blk, n, spec, lm, 1, lane)], gi);
+#pragma unroll
+                    for (int n = 0; n < NF; ++n) {
+                        double2 g;
+                        if (GL)
+                            g = gs[lm * NF + n];
+                        else if (n < nfn)
+                            g = double2{S.G[a_index(M, blk, n, spec, lm, 0, lane)],
+                                        S.G[a_index(M, blk, n, spec, lm, 1, lane)]};
+                        else
+                            g = double2{0.0, 0.0};
+                        gr = fma(gn[n], g.x, gr);
+                        gi = fma(gn[n], g.y, gi);
                     }
                     sr = fma(q, gr, sr);
                     si = fma(q, gi, si);
@@ -1126,10 +1153,30 @@ bool anlm_forms_features(const DevModel& m, int precision, int kind) {
     return true;
 }
 
+namespace {
+template <int NF>
+hipError_t launch_pair_energy_n(const DevModel& m, const DevSystem& s, double* epv, hipStream_t st) {
+    const dim3 grid(slot_grid(s)), block(kPairEnergyThreads);
+    const size_t lds = sizeof(double2) * m.n_type * m.n_lmh * NF;
+    if (lds > lds_limit()) {
+        hipLaunchKernelGGL((k_pair_energy<NF, false>), grid, block, 0, st, m, s, epv);
+        return launched();
+    }
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_pair_energy<NF, true>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_pair_energy<NF, true>), grid, block, lds, st, m, s, epv);
+    return launched(lds);
+}
+}  // namespace
+
 hipError_t launch_pair_energy(const DevModel& m, const DevSystem& s, double* epv, hipStream_t st) {
     if (s.nblocks == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_pair_energy, dim3(slot_grid(s)), dim3(64), 0, st, m, s, epv);
-    return launched();
+    if (m.n_fn <= 4) return launch_pair_energy_n<4>(m, s, epv, st);
+    if (m.n_fn <= 8) return launch_pair_energy_n<8>(m, s, epv, st);
+    if (m.n_fn <= 12) return launch_pair_energy_n<12>(m, s, epv, st);
+    if (m.n_fn <= 16) return launch_pair_energy_n<16>(m, s, epv, st);
+    return launch_pair_energy_n<32>(m, s, epv, st);
 }
 
 hipError_t launch_force(const DevModel& m, const DevSystem& s, int precision, int threads, hipStream_t st) {
