@@ -28,6 +28,20 @@ struct YTab {
     T grad[kMaxL + 1][kMaxL + 1];   // sqrt((l+m+1)(l-m))
 };
 
+// Tables of the column a_nlm kernel (anlm_cols.hip; l_max <= 12), per step and
+// product column: recursion constants (negative), target 2 lmh + (re/im) or -1,
+// norm.
+constexpr int kColsMaxL = 12;
+constexpr int kColsBuf = 1984;  // doubles of LDS per workgroup: a batch of 64 neighbors or an epilogue round
+struct ColsTab {
+    double c[kColsMaxL + 1][16];
+    double norm[kColsMaxL + 1][16];
+    int32_t lmc[kColsMaxL + 1][16];
+};
+// weights of an order-1/2 feature's terms m = 0 .. L (L <= 12): the coefficients
+// of +m and -m summed, with the sign (-1)^m
+constexpr int kQ12Weights = 14;
+
 struct DevModel {
     int n_type, n_fn, n_gtinv, n_lmh, maxl, lmax3, n_pitc, n_p;
     int lmax_t;             // largest l of the order-3/4 adjoint kernel's tile (lmax3: the feature kernel's)
@@ -67,6 +81,7 @@ struct DevModel {
     // order-1/2 polynomial features per centre species, fq12[fq12_off[t] ..
     // fq12_off[t+1]) (formed in the a_nlm kernel's epilogue)
     const FeatQ12* fq12;
+    const double* fq12w;    // [fq12][kQ12Weights] (null above l_max 12)
     int32_t fq12_off[3];
     // Polynomial features on the device are per species and compact: a
     // centre of species t keeps the ranks [lo, hi) = prange[t] it sees, as
@@ -106,6 +121,7 @@ struct DevModel {
     int q34_dyn_adj, q34_dyn_feat;  // visits for the general-loop order-3/4 kernel
     const YTab<double>* yt64;
     const YTab<float>* yt32;
+    const ColsTab* cols;    // null above l_max 12
     // orders 5/6: visits of every species (adjoint, then features), their
     // term codes and coefficients; tile of a_nlm up to l = lmaxh
     const VisitHi* hvis;
@@ -189,6 +205,11 @@ enum AnlmKind : int { kAnlmValu = 0, kAnlmMfma = 1 };
 // anlm_forms_features says the launch can
 hipError_t launch_anlm(const DevModel& m, const DevSystem& s, int precision, hipStream_t st, int kind = kAnlmValu,
                        bool feat = false);
+// the column kernel: matrix cores, up to 16 radial functions and l_max 12
+void build_cols_tables(int maxl, ColsTab& t);
+bool anlm_cols_fits(const DevModel& m);
+bool anlm_cols_features(const DevModel& m);
+hipError_t launch_anlm_cols(const DevModel& m, const DevSystem& s, int feat, int precision, hipStream_t st);
 bool anlm_has_mfma(const DevModel& m);
 bool anlm_forms_features(const DevModel& m, int precision, int kind);
 hipError_t launch_q12(const DevModel& m, const DevSystem& s, bool feat, hipStream_t st);

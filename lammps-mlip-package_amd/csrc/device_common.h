@@ -55,6 +55,36 @@ __device__ __forceinline__ int pcol(const DevModel& M, int t, int n, int rank) {
     return n * (M.prange[t][1] - M.prange[t][0]) + rank - M.prange[t][0];
 }
 
+struct PairDel {
+    double dx, dy, dz, r;
+    bool valid;
+};
+
+// del = x_centre - x_neighbor (+ image shift), strict r < cutoff.  Always
+// FP64: the difference of absolute positions and the cutoff test must not
+// depend on the precision mode.
+__device__ __forceinline__ PairDel pair_del(const DevModel& M, const DevSystem& S, int owner, int64_t p) {
+    PairDel g;
+    const int nb = S.pnbr[p];
+    const int c = S.pcen ? S.pcen[p] : owner;
+    g.dx = S.x[3 * c] - S.x[3 * nb];
+    g.dy = S.x[3 * c + 1] - S.x[3 * nb + 1];
+    g.dz = S.x[3 * c + 2] - S.x[3 * nb + 2];
+    if (S.pshift) {
+        g.dx += S.pshift[3 * p];
+        g.dy += S.pshift[3 * p + 1];
+        g.dz += S.pshift[3 * p + 2];
+    }
+    g.r = sqrt(g.dx * g.dx + g.dy * g.dy + g.dz * g.dz);
+    g.valid = (g.r < M.cutoff) && (g.r > 0.0);
+    return g;
+}
+
+// compile-time constants as arguments
+template <int N>
+struct Const {
+    static constexpr int value = N;
+};
 
 }  // namespace dev
 }  // namespace mlip

@@ -274,6 +274,23 @@ bool upload_model(mlip_ctx* c) {
               upload(c, c->d_fq12, fq12.data(), fq12.size(), "order-1/2 feature list") &&
               upload(c, c->d_zlist, zlist.data(), zlist.size(), "feature zero list");
     if (!ok) return false;
+    if (!m.pair_model && m.maxl <= kColsMaxL) {
+        ColsTab ct;
+        build_cols_tables(m.maxl, ct);
+        std::vector<double> w(std::max<size_t>(fq12.size(), 1) * kQ12Weights, 0.0);
+        for (size_t k = 0; k < fq12.size(); ++k) {
+            const FeatQ12& f = fq12[k];
+            const double* cp = m.coef.data() + f.coef;
+            double* wk = w.data() + k * kQ12Weights;
+            wk[0] = f.order == 1 ? cp[0] : cp[f.L];
+            for (int j = 1; f.order == 2 && j <= f.L; ++j) wk[j] = (j & 1 ? -1.0 : 1.0) * (cp[f.L - j] + cp[f.L + j]);
+        }
+        if (!upload(c, c->d_cols, &ct, 1, "a_nlm column table") ||
+            !upload(c, c->d_fq12w, w.data(), w.size(), "order-1/2 feature weights"))
+            return false;
+        dm.cols = c->d_cols.p;
+        dm.fq12w = c->d_fq12w.p;
+    }
     dm.poly_fused = (!m.pair_model && m.n_p > 0 && c3w.empty()) ? 1 : 0;
     dm.zlist = c->d_zlist.p;
     dm.fq12 = c->d_fq12.p;
@@ -1098,7 +1115,7 @@ void mlip_destroy(mlip_ctx* c) {
         (void)hipEventDestroy(e.a);
         (void)hipEventDestroy(e.b);
     }
-    DBuf<double>* dbs[] = {&c->d_coef, &c->d_weight, &c->d_weight_e, &c->d_wmat_e, &c->d_line, &c->d_wmat, &c->d_linp, &c->d_c3w, &c->x,
+    DBuf<double>* dbs[] = {&c->d_coef, &c->d_fq12w, &c->d_weight, &c->d_weight_e, &c->d_wmat_e, &c->d_line, &c->d_wmat, &c->d_linp, &c->d_c3w, &c->x,
                            &c->pshift, &c->epv, &c->evat,
                            &c->A, &c->G, &c->D, &c->Hq, &c->H, &c->Ep, &c->Eq12, &c->Eq34, &c->gpair,
                            &c->vown, &c->f, &c->e_slot, &c->red, &c->out, &c->sout};
@@ -1124,6 +1141,7 @@ void mlip_destroy(mlip_ctx* c) {
     c->d_hterm.release();
     c->d_hcoef.release();
     c->d_hrow.release();
+    c->d_cols.release();
     c->d_r3.release();
     c->d_t3.release();
     c->d_c3q.release();

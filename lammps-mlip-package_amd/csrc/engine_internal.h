@@ -72,6 +72,8 @@ struct mlip_ctx {
     mlip::DBuf<int32_t> d_hterm, d_hrterm;
     mlip::DBuf<double> d_hcoef, d_hrcoef;
     mlip::DBuf<mlip::HiRow> d_hrow;
+    mlip::DBuf<mlip::ColsTab> d_cols;
+    mlip::DBuf<double> d_fq12w;
     mlip::DBuf<mlip::Rec3> d_r3;
     mlip::DBuf<mlip::Task3> d_t3;
     mlip::DBuf<double> d_c3q, d_w3, d_c4;

@@ -97,31 +97,6 @@ __device__ __forceinline__ void sin_cos(double a, lds_cdouble* q, double* s, dou
     *c = up ? -ct : ct;
 }
 
-struct PairDel {
-    double dx, dy, dz, r;
-    bool valid;
-};
-
-// del = x_centre - x_neighbor (+ image shift), strict r < cutoff.  Always
-// FP64: the difference of absolute positions and the cutoff test must not
-// depend on the precision mode.
-__device__ __forceinline__ PairDel pair_del(const DevModel& M, const DevSystem& S, int owner, int64_t p) {
-    PairDel g;
-    const int nb = S.pnbr[p];
-    const int c = S.pcen ? S.pcen[p] : owner;
-    g.dx = S.x[3 * c] - S.x[3 * nb];
-    g.dy = S.x[3 * c + 1] - S.x[3 * nb + 1];
-    g.dz = S.x[3 * c + 2] - S.x[3 * nb + 2];
-    if (S.pshift) {
-        g.dx += S.pshift[3 * p];
-        g.dy += S.pshift[3 * p + 1];
-        g.dz += S.pshift[3 * p + 2];
-    }
-    g.r = sqrt(g.dx * g.dx + g.dy * g.dy + g.dz * g.dz);
-    g.valid = (g.r < M.cutoff) && (g.r > 0.0);
-    return g;
-}
-
 // ---------------------------------------------------------------- a_nlm
 // One workgroup of NTH threads per centre (192, or 256 when l_max > 18).
 // Neighbors are taken in blocks of NTH (geometry once per neighbor into
@@ -1001,9 +976,9 @@ hipError_t launch_anlm_mfma_k(const DevModel& m, const DevSystem& s, hipStream_t
     return launched();
 }
 
-// the matrix-core a_nlm kernel takes l_max <= 12, two species and up to 32
-// radial functions (MT = 1 or 2 tiles of 16), with at most three column
-// tiles per wave (2 n_lmh <= 192 columns)
+// this matrix-core a_nlm kernel takes l_max <= 12, two species and 17 to 32
+// radial functions (two tiles of 16; up to 16 are the column kernel's), with
+// at most three column tiles per wave (2 n_lmh <= 192 columns)
 bool anlm_mfma_fits(const DevModel& m) {
     const int nt = (2 * m.n_lmh + 15) / 16;
     return m.maxl < kSmallL1 && m.n_type <= 2 && m.n_fn <= 32 && (nt + 3) / 4 <= 3;
@@ -1011,12 +986,7 @@ bool anlm_mfma_fits(const DevModel& m) {
 
 template <typename T>
 hipError_t launch_anlm_mfma_t(const DevModel& m, const DevSystem& s, hipStream_t st) {
-    const int mt = (m.n_fn + 15) / 16, ntw = ((2 * m.n_lmh + 15) / 16 + 3) / 4;
-    if (mt == 1) {
-        if (ntw == 1) return launch_anlm_mfma_k<T, 1, 1>(m, s, st);
-        if (ntw == 2) return launch_anlm_mfma_k<T, 1, 2>(m, s, st);
-        return launch_anlm_mfma_k<T, 1, 3>(m, s, st);
-    }
+    const int ntw = ((2 * m.n_lmh + 15) / 16 + 3) / 4;
     if (ntw == 1) return launch_anlm_mfma_k<T, 2, 1>(m, s, st);
     if (ntw == 2) return launch_anlm_mfma_k<T, 2, 2>(m, s, st);
     return launch_anlm_mfma_k<T, 2, 3>(m, s, st);
@@ -1132,9 +1102,10 @@ void build_ylm_tables(YTab<double>& t64, YTab<float>& t32) {
 hipError_t launch_anlm(const DevModel& m, const DevSystem& s, int precision, hipStream_t st, int kind, bool feat) {
     if (s.nblocks == 0) return hipSuccess;
     if (feat && !anlm_forms_features(m, precision, kind)) return hipErrorInvalidValue;
+    const int f = feat ? 1 : 0;
+    if (kind == kAnlmMfma && anlm_cols_fits(m)) return launch_anlm_cols(m, s, f, precision, st);
     if (kind == kAnlmMfma && anlm_mfma_fits(m))
         return precision == kMixed ? launch_anlm_mfma_t<float>(m, s, st) : launch_anlm_mfma_t<double>(m, s, st);
-    const int f = feat ? 1 : 0;
     return precision == kMixed ? launch_anlm_t<float>(m, s, f, st) : launch_anlm_t<double>(m, s, f, st);
 }
 
@@ -1143,8 +1114,9 @@ bool anlm_has_mfma(const DevModel& m) { return anlm_mfma_fits(m); }
 // The register kernel forms the order-1/2 features when a round of at least
 // one radial index fits its chunk buffer for every species' row segment.
 bool anlm_forms_features(const DevModel& m, int precision, int kind) {
-    if (kind == kAnlmMfma && anlm_mfma_fits(m)) return false;
     if (m.pair_model || m.n_p <= 0) return false;
+    if (kind == kAnlmMfma && anlm_cols_fits(m)) return anlm_cols_features(m);
+    if (kind == kAnlmMfma && anlm_mfma_fits(m)) return false;
     // the smallest buffer either table size may use (T2 entries): a round
     // that fits it fits the compact tables' larger one too
     const int t2 = precision == kMixed ? 8 : 16;
