@@ -38,6 +38,15 @@ struct ColsTab {
     double norm[kColsMaxL + 1][16];
     int32_t lmc[kColsMaxL + 1][16];
 };
+// Tables of the matrix-core force kernel (force_cols.hip; l_max <= 12): per entry
+// and quarter the recursion constant (negative), per product tile and 4 quarter +
+// result the source row 2 lmh + (re/im) or -1 and its factor (norm, w_m).
+constexpr int kForceEntries = 28;
+struct ForceTab {
+    double c[kForceEntries][4];
+    double fac[(kForceEntries + 1) / 2][16];
+    int32_t row[(kForceEntries + 1) / 2][16];
+};
 // weights of an order-1/2 feature's terms m = 0 .. L (L <= 12): the coefficients
 // of +m and -m summed, with the sign (-1)^m
 constexpr int kQ12Weights = 14;
@@ -122,6 +131,7 @@ struct DevModel {
     const YTab<double>* yt64;
     const YTab<float>* yt32;
     const ColsTab* cols;    // null above l_max 12
+    const ForceTab* ftab;   // null above l_max 12
     // orders 5/6: visits of every species (adjoint, then features), their
     // term codes and coefficients; tile of a_nlm up to l = lmaxh
     const VisitHi* hvis;
@@ -207,6 +217,9 @@ hipError_t launch_anlm(const DevModel& m, const DevSystem& s, int precision, hip
                        bool feat = false);
 // the column kernel: matrix cores, up to 16 radial functions and l_max 12
 void build_cols_tables(int maxl, ColsTab& t);
+void build_force_tables(int maxl, ForceTab& t);
+bool force_cols_fits(const DevModel& m);
+hipError_t launch_force_cols(const DevModel& m, const DevSystem& s, int precision, int threads, hipStream_t st);
 bool anlm_cols_fits(const DevModel& m);
 bool anlm_cols_features(const DevModel& m);
 hipError_t launch_anlm_cols(const DevModel& m, const DevSystem& s, int feat, int precision, hipStream_t st);

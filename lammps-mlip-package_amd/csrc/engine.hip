@@ -288,7 +288,11 @@ bool upload_model(mlip_ctx* c) {
         if (!upload(c, c->d_cols, &ct, 1, "a_nlm column table") ||
             !upload(c, c->d_fq12w, w.data(), w.size(), "order-1/2 feature weights"))
             return false;
+        ForceTab ft;
+        build_force_tables(m.maxl, ft);
+        if (!upload(c, c->d_ftab, &ft, 1, "force table")) return false;
         dm.cols = c->d_cols.p;
+        dm.ftab = c->d_ftab.p;
         dm.fq12w = c->d_fq12w.p;
     }
     dm.poly_fused = (!m.pair_model && m.n_p > 0 && c3w.empty()) ? 1 : 0;
@@ -1142,6 +1146,7 @@ void mlip_destroy(mlip_ctx* c) {
     c->d_hcoef.release();
     c->d_hrow.release();
     c->d_cols.release();
+    c->d_ftab.release();
     c->d_r3.release();
     c->d_t3.release();
     c->d_c3q.release();

@@ -73,6 +73,7 @@ struct mlip_ctx {
     mlip::DBuf<double> d_hcoef, d_hrcoef;
     mlip::DBuf<mlip::HiRow> d_hrow;
     mlip::DBuf<mlip::ColsTab> d_cols;
+    mlip::DBuf<mlip::ForceTab> d_ftab;
     mlip::DBuf<double> d_fq12w;
     mlip::DBuf<mlip::Rec3> d_r3;
     mlip::DBuf<mlip::Task3> d_t3;
@@ -101,7 +102,7 @@ struct mlip_ctx {
     std::vector<int64_t> owners_per_type;
     int64_t npairs = 0;
     // launch shape chosen by mlip_autotune
-    int force_threads = 192;
+    int force_threads = 256;
     int anlm_kind = mlip::kAnlmMfma;  // a_nlm kernel (mlip_autotune keeps the faster one)
     int nblk_type[2] = {0, 0};  // slot blocks of each species (blocks are grouped by species)
     size_t wofs[2] = {0, 0};    // per-species quadratic form in d_wmat: offset and dimension

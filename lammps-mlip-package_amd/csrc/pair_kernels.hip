@@ -570,6 +570,8 @@ __global__ __launch_bounds__(kAmThreads) void k_anlm_mfma(DevModel M, DevSystem 
 //   A = m z Q + (1-z^2) c Q', B = m Q - z c Q', E = m (1+z^2) Q + z (1-z^2) c Q',
 //   Q = Qb_l^m, Q' = Qb_l^{m+1}, c = sqrt((l+m+1)(l-m)); for m = 0 the
 //   singular terms cancel to c Q' (z x, z y, -(1-z^2)).
+constexpr int kForceThreads = 128;
+
 template <typename T, int KL1>
 struct ForceLds {
     double beta[kMaxFn], mu[kMaxFn];
@@ -580,15 +582,13 @@ struct ForceLds {
     double trig[kTrigN + 1];  // sin / cos series coefficients, then pi / r_c
 };
 
-// Register budget for occupancy: FP64 at most 168 VGPRs (3 waves per SIMD;
-// unconstrained it takes 214 and runs 2 waves), FP32 at most 128 (4 waves).
-// The spills this costs are cheaper than the lost latency hiding: 28.0 ->
-// 19.6 ms (FP64) and 14.2 -> 12.9 ms (FP32) at 256k atoms with 192 threads,
-// where the workgroups' G tiles still fit the LDS.  Models whose G tile does
-// not fit (l_max and n_fn near their limits) read G from HBM instead (GL =
-// false; every thread of the workgroup reads the same entries, served by the
-// caches), and models with more than 16 radial functions keep the register
-// arrays they need (no occupancy cap).
+// For l_max above 12 or more than 16 radial functions (the matrix-core kernel
+// takes the others).  Register budget for occupancy: FP64 at most 168 VGPRs (3
+// waves per SIMD), FP32 at most 128 (4 waves); the spills this costs are cheaper
+// than the lost latency hiding.  Models whose G tile does not fit the LDS read G
+// from HBM instead (GL = false; every thread of the workgroup reads the same
+// entries, served by the caches), and models with more than 16 radial functions
+// keep the register arrays they need (no occupancy cap).
 template <int NF, int NT, typename T, bool GL, int KL1>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NF > 16 ? 1 : (sizeof(T) == 4 ? 4 : 3)))) void k_force(DevModel M, DevSystem S) {
     extern __shared__ __attribute__((aligned(16))) unsigned char force_dyn[];
@@ -1025,45 +1025,22 @@ bool force_tile_fits(const DevModel& m, int nf, int nt) {
     return lds + sizeof(ForceLds<T, KL1>) + sizeof(double) * 6 * (nt / 64) <= lds_limit();
 }
 
-template <int NT, typename T>
-hipError_t launch_force_nt(const DevModel& m, const DevSystem& s, hipStream_t st) {
-    const int nf = m.n_fn <= 4 ? 4 : m.n_fn <= 8 ? 8 : m.n_fn <= 12 ? 12 : m.n_fn <= 16 ? 16 : m.n_fn <= 24 ? 24 : 32;
-    if (m.maxl < kSmallL1 && nf <= 16 && force_tile_fits<T, kSmallL1>(m, nf, NT)) {
-        if (nf == 4) return launch_force_k<4, NT, T, true, kSmallL1>(m, s, st);
-        if (nf == 8) return launch_force_k<8, NT, T, true, kSmallL1>(m, s, st);
-        if (nf == 12) return launch_force_k<12, NT, T, true, kSmallL1>(m, s, st);
-        return launch_force_k<16, NT, T, true, kSmallL1>(m, s, st);
-    }
-    // large models (l_max above 12, more than 16 radial functions or a G
-    // tile beyond the LDS): one launch shape, full-size tables
-    if (force_tile_fits<T, kL1>(m, nf, 128)) {
-        switch (nf) {
-            case 4: return launch_force_k<4, 128, T, true, kL1>(m, s, st);
-            case 8: return launch_force_k<8, 128, T, true, kL1>(m, s, st);
-            case 12: return launch_force_k<12, 128, T, true, kL1>(m, s, st);
-            case 16: return launch_force_k<16, 128, T, true, kL1>(m, s, st);
-            case 24: return launch_force_k<24, 128, T, true, kL1>(m, s, st);
-            default: return launch_force_k<32, 128, T, true, kL1>(m, s, st);
-        }
-    }
-    switch (nf) {
-        case 4: return launch_force_k<4, 128, T, false, kL1>(m, s, st);
-        case 8: return launch_force_k<8, 128, T, false, kL1>(m, s, st);
-        case 12: return launch_force_k<12, 128, T, false, kL1>(m, s, st);
-        case 16: return launch_force_k<16, 128, T, false, kL1>(m, s, st);
-        case 24: return launch_force_k<24, 128, T, false, kL1>(m, s, st);
-        default: return launch_force_k<32, 128, T, false, kL1>(m, s, st);
-    }
+// G staged in LDS where it fits (GL)
+template <typename T, bool GL>
+hipError_t launch_force_gl(const DevModel& m, const DevSystem& s, hipStream_t st) {
+    if (m.n_fn <= 4) return launch_force_k<4, kForceThreads, T, GL, kL1>(m, s, st);
+    if (m.n_fn <= 8) return launch_force_k<8, kForceThreads, T, GL, kL1>(m, s, st);
+    if (m.n_fn <= 12) return launch_force_k<12, kForceThreads, T, GL, kL1>(m, s, st);
+    if (m.n_fn <= 16) return launch_force_k<16, kForceThreads, T, GL, kL1>(m, s, st);
+    if (m.n_fn <= 24) return launch_force_k<24, kForceThreads, T, GL, kL1>(m, s, st);
+    return launch_force_k<32, kForceThreads, T, GL, kL1>(m, s, st);
 }
 
 template <typename T>
-hipError_t launch_force_t(const DevModel& m, const DevSystem& s, int threads, hipStream_t st) {
-    switch (threads) {
-        case 64: return launch_force_nt<64, T>(m, s, st);
-        case 192: return launch_force_nt<192, T>(m, s, st);
-        case 256: return launch_force_nt<256, T>(m, s, st);
-        default: return launch_force_nt<128, T>(m, s, st);
-    }
+hipError_t launch_force_t(const DevModel& m, const DevSystem& s, hipStream_t st) {
+    const int nf = m.n_fn <= 16 ? (m.n_fn + 3) / 4 * 4 : m.n_fn <= 24 ? 24 : 32;
+    return force_tile_fits<T, kL1>(m, nf, kForceThreads) ? launch_force_gl<T, true>(m, s, st)
+                                                        : launch_force_gl<T, false>(m, s, st);
 }
 
 }  // namespace
@@ -1153,7 +1130,8 @@ hipError_t launch_pair_energy(const DevModel& m, const DevSystem& s, double* epv
 
 hipError_t launch_force(const DevModel& m, const DevSystem& s, int precision, int threads, hipStream_t st) {
     if (s.nblocks == 0) return hipSuccess;
-    return precision == kMixed ? launch_force_t<float>(m, s, threads, st) : launch_force_t<double>(m, s, threads, st);
+    if (force_cols_fits(m)) return launch_force_cols(m, s, precision, threads, st);
+    return precision == kMixed ? launch_force_t<float>(m, s, st) : launch_force_t<double>(m, s, st);
 }
 
 }  // namespace mlip
