@@ -19,10 +19,10 @@
 //   k_nb_bin     fractional coordinates, wrapped position, global bin key
 //   radix sort   (bin key, atom) -> bin members in atom order
 //   k_nb_heads   thread per bin: first member (binary search)
-//   k_nb_pairs   count pass, exclusive scan, fill pass
+//   k_nb_pairs   wave per atom: count pass, exclusive scan, fill pass
 //   radix sort   (neighbor, pair) -> incoming pairs of every position in
 //                pair order
-//   k_nb_gather  thread per position: merge its outgoing (-) and incoming
+//   k_nb_gather  wave per position: merge its outgoing (-) and incoming
 //                (+) pairs in pair order
 #include <hipcub/hipcub.hpp>
 
@@ -77,7 +77,16 @@ namespace {
 
 constexpr int kNbThreads = 256;
 
+// orders a wave's LDS accesses against one another for the compiler (the
+// hardware executes them in order)
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 inline unsigned grid_of(int64_t n) { return static_cast<unsigned>((n + kNbThreads - 1) / kNbThreads); }
+
+inline unsigned wave_grid(int64_t n) { return static_cast<unsigned>((n + kNbThreads / 64 - 1) / (kNbThreads / 64)); }
 
 __global__ __launch_bounds__(kNbThreads) void k_nb_bin(const NbCell* __restrict__ cells,
                                                        const int32_t* __restrict__ sid, int n,
@@ -122,8 +131,22 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_heads(const uint32_t* __restr
     head[b] = lo;
 }
 
-// Count (FILL = false) or write (FILL = true) atom a's neighbors: stencil
-// bins in (d0, d1, d2) order, members in atom order, 0 < r^2 < rc2.
+// Count (FILL = false) or write (FILL = true) the neighbors of an atom, a wave
+// each: stencil bins in (d0, d1, d2) order, members in atom order, 0 < r^2 < rc2.
+// 64 stencil bins at a time, a lane per bin, are laid out as one list of members
+// in LDS (in parts of kNbList where they hold more); the members are then taken
+// 64 at a time, and ballots keep their order.  Bound: latency, a chain of ~10
+// dependent reads per 64 bins.  A thread per atom walked ~400 members one after
+// the other: 226 + 457 us (count + fill) at 1,371 atoms; now 11 + 14 us.
+constexpr int kNbWaves = kNbThreads / 64;
+constexpr int kNbList = 512;
+
+struct NbWave {
+    double sv[3][64];          // lattice image of the stencil bin: the neighbor sits at x_j + S
+    int32_t member[kNbList];
+    uint8_t bin[kNbList];
+};
+
 template <bool FILL>
 __global__ __launch_bounds__(kNbThreads) void k_nb_pairs(const NbCell* __restrict__ cells,
                                                          const int32_t* __restrict__ sid, int n,
@@ -134,11 +157,17 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_pairs(const NbCell* __restric
                                                          const double* __restrict__ wrap,
                                                          int64_t* __restrict__ cnt, const int64_t* __restrict__ off,
                                                          int32_t* __restrict__ pnbr, double* __restrict__ pshift) {
-    const int a = blockIdx.x * kNbThreads + threadIdx.x;
-    if (a >= n) return;
+    __shared__ NbWave lds[kNbWaves];
+    const int lane = threadIdx.x & 63;
+    NbWave& W = lds[threadIdx.x >> 6];
+    const int a = blockIdx.x * kNbWaves + (threadIdx.x >> 6);
+    if (a >= n) return;  // whole waves leave, and no barrier follows
     const NbCell& C = cells[sid[a]];
     const double rc2 = C.rc2;
     const int nb0 = C.nb[0], nb1 = C.nb[1], nb2 = C.nb[2];
+    const int r0 = C.reach[0], r1 = C.reach[1], r2n = C.reach[2];
+    const int w1 = 2 * r1 + 1, w2 = 2 * r2n + 1;
+    const int64_t nst = static_cast<int64_t>(2 * r0 + 1) * w1 * w2;
     const int bl = static_cast<int>(key[a]) - C.bin0;
     const int b0 = bl / (nb1 * nb2), b1 = (bl / nb2) % nb1, b2 = bl % nb2;
     const double xi0 = xw[3 * a], xi1 = xw[3 * a + 1], xi2 = xw[3 * a + 2];
@@ -149,48 +178,70 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_pairs(const NbCell* __restric
         lim = off[a + 1] - o;
     }
     int64_t k = 0;
-    for (int d0 = -C.reach[0]; d0 <= C.reach[0]; ++d0) {
-        const int c0 = b0 + d0;
-        const int j0 = ((c0 % nb0) + nb0) % nb0, s0 = (c0 - j0) / nb0;
-        for (int d1 = -C.reach[1]; d1 <= C.reach[1]; ++d1) {
-            const int c1 = b1 + d1;
+    for (int64_t st = 0; st < nst; st += 64) {
+        int q0 = 0, count = 0;
+        if (st + lane < nst) {
+            const int64_t id = st + lane, row = id / w2;
+            const int c0 = b0 + static_cast<int>(row / w1) - r0, c1 = b1 + static_cast<int>(row % w1) - r1,
+                      c2 = b2 + static_cast<int>(id % w2) - r2n;
+            const int j0 = ((c0 % nb0) + nb0) % nb0, s0 = (c0 - j0) / nb0;
             const int j1 = ((c1 % nb1) + nb1) % nb1, s1 = (c1 - j1) / nb1;
-            for (int d2 = -C.reach[2]; d2 <= C.reach[2]; ++d2) {
-                const int c2 = b2 + d2;
-                const int j2 = ((c2 % nb2) + nb2) % nb2, s2 = (c2 - j2) / nb2;
-                const int bj = C.bin0 + (j0 * nb1 + j1) * nb2 + j2;
-                // lattice image of the stencil bin: the neighbor sits at x_j + S
-                const double sv0 = static_cast<double>(s0) * C.cell[0] + static_cast<double>(s1) * C.cell[3] +
-                                   static_cast<double>(s2) * C.cell[6];
-                const double sv1 = static_cast<double>(s0) * C.cell[1] + static_cast<double>(s1) * C.cell[4] +
-                                   static_cast<double>(s2) * C.cell[7];
-                const double sv2 = static_cast<double>(s0) * C.cell[2] + static_cast<double>(s1) * C.cell[5] +
-                                   static_cast<double>(s2) * C.cell[8];
-                const double ex = xi0 - sv0, ey = xi1 - sv1, ez = xi2 - sv2;
-                const double ox = -sv0 - wi0, oy = -sv1 - wi1, oz = -sv2 - wi2;
-                const int q1 = head[bj + 1];
-                for (int q = head[bj]; q < q1; ++q) {
-                    const int j = member[q];
+            const int j2 = ((c2 % nb2) + nb2) % nb2, s2 = (c2 - j2) / nb2;
+            const int bj = C.bin0 + (j0 * nb1 + j1) * nb2 + j2;
+            q0 = head[bj];
+            count = head[bj + 1] - q0;
+            for (int x = 0; x < 3; ++x)
+                W.sv[x][lane] = static_cast<double>(s0) * C.cell[x] + static_cast<double>(s1) * C.cell[3 + x] +
+                                static_cast<double>(s2) * C.cell[6 + x];
+        }
+        int before = count;  // inclusive, then exclusive prefix of the counts
+#pragma unroll
+        for (int s = 1; s < 64; s <<= 1) {
+            const int v = __shfl_up(before, s);
+            if (lane >= s) before += v;
+        }
+        const int total = __shfl(before, 63);
+        before -= count;
+        for (int base = 0; base < total; base += kNbList) {
+            const int e1 = min(count, base + kNbList - before);
+            for (int e = max(0, base - before); e < e1; ++e) {
+                W.member[before + e - base] = member[q0 + e];
+                W.bin[before + e - base] = static_cast<uint8_t>(lane);
+            }
+            wave_lds_fence();
+            const int nl = min(kNbList, total - base);
+            for (int i = 0; i < nl; i += 64) {
+                bool hit = false;
+                int j = 0, bin = 0;
+                if (i + lane < nl) {
+                    j = W.member[i + lane];
+                    bin = W.bin[i + lane];
+                    const double ex = xi0 - W.sv[0][bin], ey = xi1 - W.sv[1][bin], ez = xi2 - W.sv[2][bin];
                     const double dx = ex - xw[3 * j];
                     const double dy = ey - xw[3 * j + 1];
                     const double dz = ez - xw[3 * j + 2];
                     const double r2 = dx * dx + dy * dy + dz * dz;
-                    if (r2 < rc2 && r2 > 0.0) {
-                        if (FILL && k < lim) {
-                            // del = x_i - x_j + shift on the caller's positions
-                            const int64_t e = o + k;
-                            pnbr[e] = j;
-                            pshift[3 * e] = ox + wrap[3 * j];
-                            pshift[3 * e + 1] = oy + wrap[3 * j + 1];
-                            pshift[3 * e + 2] = oz + wrap[3 * j + 2];
-                        }
-                        ++k;
+                    hit = r2 < rc2 && r2 > 0.0;
+                }
+                const uint64_t mask = __ballot(hit);
+                if (FILL && hit) {
+                    const int64_t at = k + __popcll(mask & ((1ull << lane) - 1ull));
+                    if (at < lim) {
+                        // del = x_i - x_j + shift on the caller's positions
+                        const double ox = -W.sv[0][bin] - wi0, oy = -W.sv[1][bin] - wi1, oz = -W.sv[2][bin] - wi2;
+                        pnbr[o + at] = j;
+                        pshift[3 * (o + at)] = ox + wrap[3 * j];
+                        pshift[3 * (o + at) + 1] = oy + wrap[3 * j + 1];
+                        pshift[3 * (o + at) + 2] = oz + wrap[3 * j + 2];
                     }
                 }
+                k += __popcll(mask);
             }
+            wave_lds_fence();
         }
+        wave_lds_fence();
     }
-    if (!FILL) cnt[a] = k;
+    if (!FILL && lane == 0) cnt[a] = k;
 }
 
 __global__ __launch_bounds__(kNbThreads) void k_nb_off32(const int64_t* __restrict__ off, int n,
@@ -217,29 +268,36 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_struct_off(const int64_t* __r
 
 // Gather list of position k: its own pairs (centre k, entry -(p+1)) and the
 // pairs that have k as neighbor (entry p+1), in increasing p; for a
-// self-image pair (both), the centre entry first.
+// self-image pair (both), the centre entry first.  A wave per position, and each
+// entry finds its place by itself: an own pair after the incoming ones below it
+// (binary search), an incoming one after the own ones up to it (they are
+// consecutive).  A thread per position merging the two took 113 us at 1,371 atoms;
+// now 7.
 __global__ __launch_bounds__(kNbThreads) void k_nb_gather(const int32_t* __restrict__ poff,
                                                           const int32_t* __restrict__ ihead,
                                                           const int32_t* __restrict__ inc, int n,
                                                           int32_t* __restrict__ goff, int32_t* __restrict__ gent) {
-    const int k = blockIdx.x * kNbThreads + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int k = blockIdx.x * kNbWaves + (threadIdx.x >> 6);
     if (k > n) return;
     const int w0 = poff[k] + ihead[k];
-    goff[k] = w0;
+    if (lane == 0) goff[k] = w0;
     if (k == n) return;
-    int po = poff[k];
-    const int pe = poff[k + 1];
-    int q = ihead[k];
-    const int qe = ihead[k + 1];
-    int w = w0;
-    while (po < pe || q < qe) {
-        if (q >= qe || (po < pe && po <= inc[q])) {
-            gent[w++] = -(po + 1);
-            ++po;
-        } else {
-            gent[w++] = inc[q] + 1;
-            ++q;
+    const int po = poff[k], no = poff[k + 1] - po, qo = ihead[k], nq = ihead[k + 1] - qo;
+    for (int i = lane; i < no; i += 64) {
+        int lo = 0, hi = nq;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (inc[qo + mid] < po + i)
+                lo = mid + 1;
+            else
+                hi = mid;
         }
+        gent[w0 + i + lo] = -(po + i + 1);
+    }
+    for (int i = lane; i < nq; i += 64) {
+        const int p = inc[qo + i];
+        gent[w0 + i + max(0, min(no, p + 1 - po))] = p + 1;
     }
 }
 
@@ -348,7 +406,7 @@ bool device_lists_into(mlip_ctx* c, NbWork*& wp, hipStream_t st, int nstruct, co
                 "bin sort"))
         return false;
     k_nb_heads<<<grid_of(static_cast<int64_t>(nbins) + 1), kNbThreads, 0, st>>>(w.key2.p, n, nbins, w.head.p);
-    k_nb_pairs<false><<<grid_of(n), kNbThreads, 0, st>>>(w.cells.p, w.sid.p, n, w.key.p, w.head.p, w.val2.p, w.xw.p,
+    k_nb_pairs<false><<<wave_grid(n), kNbThreads, 0, st>>>(w.cells.p, w.sid.p, n, w.key.p, w.head.p, w.val2.p, w.xw.p,
                                                          w.wrap.p, w.cnt.p, nullptr, nullptr, nullptr);
     if (!hip_ok(c, hipMemsetAsync(w.cnt.p + n, 0, sizeof(int64_t), st), "neighbor counts")) return false;
     tb = w.tmp.cap;
@@ -375,7 +433,7 @@ bool device_lists_into(mlip_ctx* c, NbWork*& wp, hipStream_t st, int nstruct, co
         c->err = "device allocation failed for the neighbor list";
         return false;
     }
-    k_nb_pairs<true><<<grid_of(n), kNbThreads, 0, st>>>(w.cells.p, w.sid.p, n, w.key.p, w.head.p, w.val2.p, w.xw.p,
+    k_nb_pairs<true><<<wave_grid(n), kNbThreads, 0, st>>>(w.cells.p, w.sid.p, n, w.key.p, w.head.p, w.val2.p, w.xw.p,
                                                         w.wrap.p, nullptr, w.off.p, out.pnbr->p, out.pshift->p);
     k_nb_off32<<<grid_of(static_cast<int64_t>(n) + 1), kNbThreads, 0, st>>>(w.off.p, n, out.poff->p);
     if (np == 0) {
@@ -403,7 +461,7 @@ bool device_lists_into(mlip_ctx* c, NbWork*& wp, hipStream_t st, int nstruct, co
                 "pair sort"))
         return false;
     k_nb_heads<<<grid_of(static_cast<int64_t>(n) + 1), kNbThreads, 0, st>>>(w.pk2.p, np, n, w.ihead.p);
-    k_nb_gather<<<grid_of(static_cast<int64_t>(n) + 1), kNbThreads, 0, st>>>(out.poff->p, w.ihead.p, w.pv2.p, n,
+    k_nb_gather<<<wave_grid(static_cast<int64_t>(n) + 1), kNbThreads, 0, st>>>(out.poff->p, w.ihead.p, w.pv2.p, n,
                                                                              out.goff->p, out.gent->p);
     return hip_ok(c, hipGetLastError(), "neighbor build");
 }
