@@ -345,9 +345,12 @@ bool upload_model(mlip_ctx* c) {
                 c4.resize(static_cast<size_t>(t + 1) * m.n_fn * q4_total(m.n_type), 0.0);
             }
         }
+        // the kernel requests a step past a record's last
+        std::vector<double> c3q = m.c3q;
+        c3q.resize(c3q.size() + kQ3N + 1, 0.0);
         if (!upload(c, c->d_r3, r3.data(), r3.size(), "order-3 records") ||
             !upload(c, c->d_t3, t3.data(), t3.size(), "order-3 tasks") ||
-            !upload(c, c->d_c3q, m.c3q.data(), m.c3q.size(), "order-3 coefficients") ||
+            !upload(c, c->d_c3q, c3q.data(), c3q.size(), "order-3 coefficients") ||
             !upload(c, c->d_w3, w3.data(), w3.size(), "order-3 weights") ||
             !upload(c, c->d_q12r, q12r.data(), q12r.size(), "order-1/2 rows") ||
             (order4 && !upload(c, c->d_c4, c4.data(), c4.size(), "order-4 products")))

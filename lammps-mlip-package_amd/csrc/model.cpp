@@ -621,18 +621,26 @@ void plan_order3(Model& m, TypeTables& tt, const std::vector<Entry3>& en) {
                     r.sig = la | lb << 4 | (N | (m.n_type > 1 && la == lb ? 8 : 0)) << 8 | ((en[b].L - L0) / 2) << 12;
                     r.coef = static_cast<int32_t>(m.c3q.size());
                     r.went = static_cast<int32_t>(b);
-                    int nm = 0;
-                    // the kernel's order: ma <= 0, then 1..k, then above k, with
-                    // the sign of a_{l,m} = (-1)^m conj(a_{l,-m})
-                    for (int ma = -la; ma <= la; ++ma) {
-                        const int mb = k - ma;
-                        if (std::abs(mb) > lb) continue;
+                    const int first = std::max(-la, k - lb), last = std::min(la, k + lb), nm = last - first + 1;
+                    if (nm <= 0) continue;
+                    r.sig |= nm << 16;
+                    auto factor = [](int l, int mm) {
+                        const uint32_t at = static_cast<uint32_t>(l * (l + 1) / 2 + l - std::abs(mm));
+                        return at * kBlockLanes * 2 * static_cast<uint32_t>(sizeof(double)) | (mm > 0 ? kQ3Conj : 0u);
+                    };
+                    r.x = factor(la, first);
+                    r.y = factor(lb, k - first);
+                    for (int ma = first; ma <= last; ++ma) {
+                        const int mb = k - ma, m1 = std::min(ma + 1, last);
+                        const uint32_t next[2] = {factor(la, m1), factor(lb, k - m1)};
+                        double code;
+                        static_assert(sizeof code == sizeof next, "two words per descriptor");
+                        std::memcpy(&code, next, sizeof code);
+                        m.c3q.push_back(code);
                         const int odd = (ma > 0 ? ma : 0) + (mb > 0 ? mb : 0);
                         for (int j = 0; j < N; ++j)
                             m.c3q.push_back((odd & 1 ? -1.0 : 1.0) * en[b + j].block[(ma + la) * (en[b + j].L + 1) + k]);
-                        ++nm;
                     }
-                    if (nm == 0) continue;
                     const int v = V == 4 && la == lb ? 3 : V;
                     tt.rec3.push_back(r);
                     cost.push_back(nm * (4L * v + 2L * v * N + 6) + 4L * m.n_type * v * N + 70);
@@ -643,16 +651,24 @@ void plan_order3(Model& m, TypeTables& tt, const std::vector<Entry3>& en) {
             sg.re = tt.rec3.size();
             segs.push_back(sg);
         }
-    // cut the sequence of records into twelve ranges of equal cost
+    // Cut the sequence of records into twelve ranges.  The three waves of a SIMD
+    // issue oldest first, so with ranges of equal cost they end one after the other
+    // (119-132, 137-156 and 163-185 thousand cycles) and the last runs alone;
+    // shares of 112 : 104 : 84 took the order-3/4 pass of 256k atoms from 18.2 to
+    // 17.1 ms (115 : 100 : 85 the same, 125 : 100 : 75 18.3).
+    static_assert(kWavesPerWg == 12, "three waves a SIMD");
+    constexpr long kShare[3] = {112, 104, 84};
     long total = 0;
     for (long c : cost) total += c;
     size_t s = 0, r = 0;
     long done = 0;
     std::vector<int> parts(segs.size(), 0);
     std::vector<std::pair<size_t, size_t>> owner;  // (segment, task)
+    long upto = 0;
     for (int w = 0; w < kWavesPerWg; ++w) {
         tt.t3_off[w] = static_cast<int32_t>(tt.task3.size());
-        const long goal = total * (w + 1) / kWavesPerWg;
+        upto += kShare[w / 4];
+        const long goal = total * upto / (4 * (kShare[0] + kShare[1] + kShare[2]));
         while (s < segs.size()) {
             const Seg& sg = segs[s];
             r = std::max(r, sg.rb);

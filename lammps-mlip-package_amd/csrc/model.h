@@ -142,12 +142,18 @@ struct VisitHi {
 
 // Order-3 linear families in the by-output-m kernel (q3.hip): a record is one
 // (la, lb) and up to kQ3N output L = L0 + 2 (i0 + j) of a segment; sig packs
-// la, lb, N (| 8 where la = lb) and i0 in 4 bits each; coefficients [ma][j] in the
-// kernel's order of ma with the conjugation signs; went: first of its entries
-// in the weight table [n][entry][S][species combination].
+// la, lb, N (| 8 where la = lb) and i0 in 4 bits each and the number of steps
+// (values of ma) above; coef: its first step in the stream; went: first of its
+// entries in the weight table [n][entry][S][species combination]; x, y: the first
+// step's factors.  A step of the stream is the next one's factors (two 32-bit
+// words in the place of a double), then N coefficients with the signs of
+// a_{l,m} = (-1)^m conj(a_{l,-m}); a factor is its byte offset in the kernel's tile,
+// with kQ3Conj where it is conjugated.
 constexpr int kQ3N = 4;
+constexpr uint32_t kQ3Conj = 0x80000000u;
 struct Rec3 {
     int32_t sig, coef, went;
+    uint32_t x, y;
 };
 // A wave's part of segment (output m = -k, L = L0, L0 + 2, .. of nL): mode 0
 // writes the rows, mode r adds them in round r.

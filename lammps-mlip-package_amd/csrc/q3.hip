@@ -14,20 +14,25 @@
 // the a_nlm tile l <= lmaxq3, m <= 0, both species, in LDS.  A wave walks records
 // (la, lb, up to kQ3N consecutive L of one parity) of one (k, parity of L) at a
 // time, G_{S,L,-k} of that segment in registers.  The records of all segments
-// in a row are cut into twelve ranges of equal modelled cost (model.cpp); a
-// segment that a cut divides is written by the wave that holds its end and
-// the other parts are added after a barrier, in order.
+// in a row are cut into twelve ranges by modelled cost (model.cpp); a segment
+// that a cut divides is written by the wave that holds its end and the other
+// parts are added after a barrier, in order.  A step's factors come as tile
+// offsets in the coefficient stream (Rec3), one step ahead.
 //
 // The waves also add the order-1/2 families to the rows they write (H of the
 // block's centres staged in LDS) and form the rows above the tile.
 //
 // Bound: FP64 VALU with one 16-byte LDS read per product, latency at 3 waves
-// per SIMD (161 VGPRs).  Per (atom, radial index) of the order-4 benchmark model
-// (l <= 8) the order-3 terms were ~25,000 products of 6 FMA-rate instructions;
-// here they are 5,500 products of 4, and 16,000 coefficient FMA pairs.  At 256k
-// atoms orders 1-4 took 36.4 ms as one visit per (family, factor position)
-// with 3/4 of the instructions address, descriptor and product work; k_q3 takes
-// 18.2 ms and k_q4 1.5 ms.
+// per SIMD.  Per (atom, radial index) of the order-4 benchmark model (l <= 8) the
+// order-3 terms were ~25,000 products of 6 FMA-rate instructions; here they are
+// 5,500 products of 4, and 16,000 coefficient FMA pairs.  At 256k atoms orders 1-4
+// took 36.4 ms as one visit per (family, factor position) with 3/4 of the
+// instructions address, descriptor and product work; k_q3 takes 15.6 ms and k_q4
+// 1.5 ms.  Of a workgroup's 220 thousand cycles 15 go to the tile (the
+// workgroups of a launch keep in step, so all read HBM at once), 165 to the
+// records, 13 to the rows above the tile and 10 to the divided segments; with the
+// factors' addresses formed from m in each step and the divided rows read and
+// written one by one it was 18.2 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -51,24 +56,34 @@ __device__ __forceinline__ double flip(double v, unsigned mask) {
     return __hiloint2double(static_cast<int>(__double2hiint(v) ^ mask), __double2loint(v));
 }
 
-// One step's operands: both species' factors and the coefficients.
+// One step's operands: both species' factors, the coefficients and the next
+// step's factors (Rec3).
 template <int NT, int N>
 struct Step {
     double2 x[NT], y[NT];
     double c[N];
-    __device__ __forceinline__ void load(const double2* As, int ss, int xa, int yb, int ma, int mb, cptr<double> cp) {
-        const int ix = xa - abs(ma) * kBlock, iy = yb - abs(mb) * kBlock;
+    unsigned fx, fy;   // sign masks
+    unsigned nx, ny;   // next step's factors
+    __device__ __forceinline__ void load(const double2* As, int ss, unsigned dx, unsigned dy, cptr<double> cp) {
+        const char* base = reinterpret_cast<const char*>(As);
+        const double2* px = reinterpret_cast<const double2*>(base + (dx & ~kQ3Conj));
+        const double2* py = reinterpret_cast<const double2*>(base + (dy & ~kQ3Conj));
 #pragma unroll
         for (int s = 0; s < NT; ++s) {
-            x[s] = As[ix + s * ss];
-            y[s] = As[iy + s * ss];
+            x[s] = px[s * ss];
+            y[s] = py[s * ss];
         }
+        fx = dx & kQ3Conj;
+        fy = dy & kQ3Conj;
+        const uint64_t code = reinterpret_cast<cptr<uint64_t>>(cp)[0];
+        nx = static_cast<unsigned>(code);
+        ny = static_cast<unsigned>(code >> 32);
 #pragma unroll
-        for (int j = 0; j < N; ++j) c[j] = cp[j];
+        for (int j = 0; j < N; ++j) c[j] = cp[1 + j];
     }
-    template <int V>
-    __device__ __forceinline__ void use(int ma, int mb, double (&tr)[N][V], double (&ti)[N][V]) {
-        const unsigned fx = ma > 0 ? 0x80000000u : 0u, fy = mb > 0 ? 0x80000000u : 0u;
+    // FIRST: the sums start here
+    template <int V, bool FIRST = false>
+    __device__ __forceinline__ void use(double (&tr)[N][V], double (&ti)[N][V]) {
 #pragma unroll
         for (int s = 0; s < NT; ++s) {
             x[s].y = flip(x[s].y, fx);
@@ -82,8 +97,8 @@ struct Step {
             const double pi = fma(x[sa].x, y[sb].y, x[sa].y * y[sb].x);
 #pragma unroll
             for (int j = 0; j < N; ++j) {
-                tr[j][v] = fma(c[j], pr, tr[j][v]);
-                ti[j][v] = fma(c[j], pi, ti[j][v]);
+                tr[j][v] = FIRST ? c[j] * pr : fma(c[j], pr, tr[j][v]);
+                ti[j][v] = FIRST ? c[j] * pi : fma(c[j], pi, ti[j][v]);
             }
         }
     }
@@ -111,33 +126,23 @@ __device__ __forceinline__ void fold(cptr<double> w, const double (&tr)[N][V], c
 // One record: all ma with |k - ma| <= lb, the next step's operands requested
 // while this one is used (the loop is unrolled by two, so no copies).
 template <int NT, int LI, int N, bool SYM>
-__device__ __forceinline__ void record(const double2* As, int ss, int k, int la, int lb, int i0, cptr<double> c,
-                                       cptr<double> w, double (&gr)[NT][LI], double (&gi)[NT][LI]) {
+__device__ __forceinline__ void record(const double2* As, int ss, unsigned x0, unsigned y0, int left, int i0,
+                                       cptr<double> c, cptr<double> w, double (&gr)[NT][LI], double (&gi)[NT][LI]) {
     constexpr int V = NT == 1 ? 1 : SYM ? 3 : 4;
     double tr[N][V], ti[N][V];
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-#pragma unroll
-        for (int v = 0; v < V; ++v) tr[j][v] = ti[j][v] = 0.0;
-    // entry of a_{l,-|m|}: l (l + 1) / 2 + l - |m|, 64 lanes apart
-    const int xa = (la * (la + 1) / 2 + la) * kBlock, yb = (lb * (lb + 1) / 2 + lb) * kBlock;
-    int ma = max(-la, k - lb);
-    const int end = min(la, k + lb);
     Step<NT, N> cur, nxt;
-    cur.load(As, ss, xa, yb, ma, k - ma, c);
-    for (;;) {
-        const int m1 = min(ma + 1, end);
-        c += m1 > ma ? N : 0;
-        nxt.load(As, ss, xa, yb, m1, k - m1, c);
-        cur.template use<V>(ma, k - ma, tr, ti);
-        if (m1 == ma) break;
-        ma = m1;
-        const int m2 = min(ma + 1, end);
-        c += m2 > ma ? N : 0;
-        cur.load(As, ss, xa, yb, m2, k - m2, c);
-        nxt.template use<V>(ma, k - ma, tr, ti);
-        if (m2 == ma) break;
-        ma = m2;
+    cur.load(As, ss, x0, y0, c);
+    c += N + 1;
+    nxt.load(As, ss, cur.nx, cur.ny, c);
+    cur.template use<V, true>(tr, ti);
+    while (--left > 0) {
+        c += N + 1;
+        cur.load(As, ss, nxt.nx, nxt.ny, c);
+        nxt.template use<V>(tr, ti);
+        if (--left == 0) break;
+        c += N + 1;
+        nxt.load(As, ss, cur.nx, cur.ny, c);
+        cur.template use<V>(tr, ti);
     }
     switch (i0) {
         case 0: fold<NT, LI, N, V, 0>(w, tr, ti, gr, gi); break;
@@ -161,36 +166,52 @@ struct Row12 {
     }
 };
 
-// Adds the order-1/2 families of row (s, L) at output m = -k: order 2
-// G_{s,L,-k} += H C_k a_{s',L,+k}, order 1 G_{s,0,0} += H C; a0 holds both
-// species' a_{.,L,-k}.  Returns the energy of families outside the polynomial
-// (Euler: 1 / order of Re(G a)).
+// The order-1/2 families of the rows (s, L): their sources, and their part of
+// output m = -k: order 2 G_{s,L,-k} += H C_k a_{s',L,+k}, order 1 G_{s,0,0} += H C;
+// a0 holds both species' a_{.,L,-k}.  add() returns the energy of families outside
+// the polynomial (Euler: 1 / order of Re(G a)).
+template <int NT>
+struct Sources12 {
+    int src[NT + 1], coef[NT + 1];
+    double h[NT + 1];
+    __device__ __forceinline__ void load(const Row12& R, int t, int s, int L) {
+        cptr<int32_t> q = as_const(R.M.q12r) + uniform(((t * 2 + s) * (kMaxLQ12 + 1) + L) * 6);
+#pragma unroll
+        for (int i = 0; i <= NT; ++i) {
+            const int at = i < NT ? 2 * i : 4;
+            src[i] = i < NT || L == 0 ? q[at] : kNoSource;
+            coef[i] = q[at + 1];
+            h[i] = src[i] != kNoSource ? R.value(src[i]) : 0.0;
+        }
+    }
+    __device__ __forceinline__ double add(const Row12& R, int s, int L, int k, const double2 (&a0)[NT], double& gr,
+                                          double& gi) const {
+        cptr<double> c = as_const(R.M.coef);
+        double e = 0.0;
+        const double wk = k == 0 ? 0.5 : 1.0, sg = (k & 1) ? -1.0 : 1.0;
+#pragma unroll
+        for (int sp = 0; sp < NT; ++sp) {
+            if (src[sp] == kNoSource) continue;
+            const double hc = h[sp] * (sg * c[coef[sp] + k]);
+            gr = fma(hc, a0[sp].x, gr);
+            gi = fma(-hc, a0[sp].y, gi);
+            if (src[sp] < 0) e = fma(wk * hc, a0[sp].x * a0[s].x + a0[sp].y * a0[s].y, e);
+        }
+        if (src[NT] != kNoSource) {
+            const double v = h[NT] * c[coef[NT]];
+            gr += v;
+            if (src[NT] < 0) e = fma(v, a0[s].x, e);
+        }
+        return e;
+    }
+};
+
 template <int NT>
 __device__ __forceinline__ double add12(const Row12& R, int t, int s, int L, int k, const double2 (&a0)[NT],
                                         double& gr, double& gi) {
-    const DevModel& M = R.M;
-    cptr<int32_t> q = as_const(M.q12r) + uniform(((t * 2 + s) * (kMaxLQ12 + 1) + L) * 6);
-    cptr<double> coef = as_const(M.coef);
-    double e = 0.0;
-    const double wk = k == 0 ? 0.5 : 1.0, sg = (k & 1) ? -1.0 : 1.0;
-#pragma unroll
-    for (int sp = 0; sp < NT; ++sp) {
-        const int src = q[2 * sp];
-        if (src == kNoSource) continue;
-        const double hc = R.value(src) * (sg * coef[q[2 * sp + 1] + k]);
-        gr = fma(hc, a0[sp].x, gr);
-        gi = fma(-hc, a0[sp].y, gi);
-        if (src < 0) e = fma(wk * hc, a0[sp].x * a0[s].x + a0[sp].y * a0[s].y, e);
-    }
-    if (L == 0) {
-        const int src = q[4];
-        if (src != kNoSource) {
-            const double h = R.value(src) * coef[q[5]];
-            gr += h;
-            if (src < 0) e = fma(h, a0[s].x, e);
-        }
-    }
-    return e;
+    Sources12<NT> q;
+    q.load(R, t, s, L);
+    return q.add(R, s, L, k, a0, gr, gi);
 }
 
 template <int NT, int LI>
@@ -199,21 +220,46 @@ __global__ __launch_bounds__(kQ3Threads) void k_q3(DevModel M, DevSystem S, int 
     const int blk = blockIdx.x, n = blockIdx.y;
     const int t = uniform(S.block_type[blk]);
     const int per_s = n_lmh_of(M.lmaxq3) * kBlock;  // entries per species
-    for (int s = 0; s < NT; ++s) {
-        const double* src = S.A + a_index(M, blk, n, s, 0, 0, 0);
-        for (int k = threadIdx.x; k < per_s; k += kQ3Threads) {
-            const int lm = k / kBlock, ln = k % kBlock;
-            q3_tile[s * per_s + k] = double2{src[2 * lm * kBlock + ln], src[(2 * lm + 1) * kBlock + ln]};
-        }
-    }
+    const int wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int hw = M.prange[t][1] - M.prange[t][0];
     const double* hseg = S.H + static_cast<size_t>(blk) * kBlock * M.n_pr + static_cast<size_t>(n) * hw;
     double* hs = reinterpret_cast<double*>(q3_tile + NT * per_s);
-    if (stage)
-        for (int e = threadIdx.x; e < kBlock * hw; e += kQ3Threads)
+    {
+        // everything read from HBM before the first task is in flight together: the
+        // tile (a thread's entries are kWavesPerWg values of lm apart) and H
+        constexpr int kHold = (n_lmh_of(LI == 5 ? 8 : 10) + kWavesPerWg - 1) / kWavesPerWg, kHoldH = 4;
+        const int top = per_s / kBlock - 1;
+        double2 v[NT][kHold];
+        double hv[kHoldH];
+#pragma unroll
+        for (int s = 0; s < NT; ++s) {
+            const double* src = S.A + a_index(M, blk, n, s, 0, 0, lane);
+#pragma unroll
+            for (int i = 0; i < kHold; ++i) {
+                const int lm = min(wave + i * kWavesPerWg, top);
+                v[s][i] = double2{src[2 * lm * kBlock], src[(2 * lm + 1) * kBlock]};
+            }
+        }
+        const int hn = stage ? kBlock * hw : 0;
+#pragma unroll
+        for (int i = 0; i < kHoldH; ++i) {
+            const int e = min(static_cast<int>(threadIdx.x) + i * kQ3Threads, hn - 1);
+            hv[i] = hn > 0 ? hseg[static_cast<size_t>(e / hw) * M.n_pr + e % hw] : 0.0;
+        }
+#pragma unroll
+        for (int s = 0; s < NT; ++s)
+#pragma unroll
+            for (int i = 0; i < kHold; ++i)
+                if (wave + i * kWavesPerWg <= top) q3_tile[s * per_s + i * kQ3Threads + threadIdx.x] = v[s][i];
+#pragma unroll
+        for (int i = 0; i < kHoldH; ++i) {
+            const int e = threadIdx.x + i * kQ3Threads;
+            if (e < hn) hs[(e % hw) * kHPitch + e / hw] = hv[i];
+        }
+        for (int e = threadIdx.x + kHoldH * kQ3Threads; e < hn; e += kQ3Threads)
             hs[(e % hw) * kHPitch + e / hw] = hseg[static_cast<size_t>(e / hw) * M.n_pr + e % hw];
+    }
     __syncthreads();
-    const int wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const double2* As = q3_tile + lane;
     cptr<Task3> tasks = as_const(M.t3);
     cptr<Rec3> recs = as_const(M.r3);
@@ -241,20 +287,21 @@ __global__ __launch_bounds__(kQ3Threads) void k_q3(DevModel M, DevSystem S, int 
             const Rec3 cur = nxt;
             if (ri + 1 < re) nxt = recs[ri + 1];
             const int sig = uniform(cur.sig);
-            const int la = sig & 15, lb = (sig >> 4) & 15, i0 = (sig >> 12) & 15;
+            const int i0 = (sig >> 12) & 15, steps = sig >> 16;
+            const unsigned x0 = uniform(static_cast<int>(cur.x)), y0 = uniform(static_cast<int>(cur.y));
             cptr<double> c = coef + uniform(cur.coef);
             cptr<double> w = wts + uniform(cur.went) * 8;
             // N, and whether la = lb (one product for the two orders of a
             // species pair)
             switch ((sig >> 8) & 15) {
-                case 1: record<NT, LI, 1, false>(As, per_s, k, la, lb, i0, c, w, gr, gi); break;
-                case 2: record<NT, LI, 2, false>(As, per_s, k, la, lb, i0, c, w, gr, gi); break;
-                case 3: record<NT, LI, 3, false>(As, per_s, k, la, lb, i0, c, w, gr, gi); break;
-                case 4: record<NT, LI, 4, false>(As, per_s, k, la, lb, i0, c, w, gr, gi); break;
-                case 9: record<NT, LI, 1, true>(As, per_s, k, la, lb, i0, c, w, gr, gi); break;
-                case 10: record<NT, LI, 2, true>(As, per_s, k, la, lb, i0, c, w, gr, gi); break;
-                case 11: record<NT, LI, 3, true>(As, per_s, k, la, lb, i0, c, w, gr, gi); break;
-                default: record<NT, LI, 4, true>(As, per_s, k, la, lb, i0, c, w, gr, gi); break;
+                case 1: record<NT, LI, 1, false>(As, per_s, x0, y0, steps, i0, c, w, gr, gi); break;
+                case 2: record<NT, LI, 2, false>(As, per_s, x0, y0, steps, i0, c, w, gr, gi); break;
+                case 3: record<NT, LI, 3, false>(As, per_s, x0, y0, steps, i0, c, w, gr, gi); break;
+                case 4: record<NT, LI, 4, false>(As, per_s, x0, y0, steps, i0, c, w, gr, gi); break;
+                case 9: record<NT, LI, 1, true>(As, per_s, x0, y0, steps, i0, c, w, gr, gi); break;
+                case 10: record<NT, LI, 2, true>(As, per_s, x0, y0, steps, i0, c, w, gr, gi); break;
+                case 11: record<NT, LI, 3, true>(As, per_s, x0, y0, steps, i0, c, w, gr, gi); break;
+                default: record<NT, LI, 4, true>(As, per_s, x0, y0, steps, i0, c, w, gr, gi); break;
             }
         }
         pend = uniform(T.mode);
@@ -286,41 +333,60 @@ __global__ __launch_bounds__(kQ3Threads) void k_q3(DevModel M, DevSystem S, int 
         }
         eacc = fma(k == 0 ? 1.0 / 3.0 : 2.0 / 3.0, e3, eacc);
     }
-    // rows above the tile, order-1/2 families only: (L, k) entries dealt over
-    // the waves, a_nlm read from HBM
-    const int lhi = min(M.maxl, kMaxLQ12);
-    for (int e = n_lmh_of(M.lmaxq3) + wave; e < n_lmh_of(lhi); e += kWavesPerWg) {
-        int L = M.lmaxq3 + 1;
-        while (n_lmh_of(L) <= e) ++L;
-        const int kk = L * (L + 1) / 2 + L - e;
-        double2 a[NT];
+    // rows above the tile, order-1/2 families only: each L's m = -kk dealt over
+    // `share` waves, a_nlm read from HBM an entry ahead
+    const int nhi = min(M.maxl, kMaxLQ12) - M.lmaxq3, share = nhi > 0 ? (kWavesPerWg + nhi - 1) / nhi : 1;
+    for (int it = wave; it < nhi * share; it += kWavesPerWg) {
+        const int L = M.lmaxq3 + 1 + it / share;
+        const double* src = S.A + a_index(M, blk, n, 0, L * (L + 1) / 2 + L, 0, lane);
+        const int sp = M.n_lmh * 2 * kBlock;
+        double2 an[NT];
+        int kk = it % share;
 #pragma unroll
-        for (int s = 0; s < NT; ++s) {
-            const double* p = S.A + a_index(M, blk, n, s, e, 0, lane);
-            a[s] = double2{p[0], p[kBlock]};
-        }
+        for (int s = 0; s < NT; ++s) an[s] = double2{src[s * sp - 2 * kk * kBlock], src[s * sp - (2 * kk - 1) * kBlock]};
+        Sources12<NT> q12[NT];
 #pragma unroll
-        for (int s = 0; s < NT; ++s) {
-            double hr = 0.0, hi = 0.0;
-            eacc += add12<NT>(rows, t, s, L, kk, a, hr, hi);
-            double* g = G + static_cast<size_t>((s * M.n_lmh + e) * 2) * kBlock;
-            g[0] = hr;
-            g[kBlock] = hi;
+        for (int s = 0; s < NT; ++s) q12[s].load(rows, t, s, L);
+        for (; kk <= L; kk += share) {
+            double2 a[NT];
+            const int kn = min(kk + share, L);
+#pragma unroll
+            for (int s = 0; s < NT; ++s) {
+                a[s] = an[s];
+                an[s] = double2{src[s * sp - 2 * kn * kBlock], src[s * sp - (2 * kn - 1) * kBlock]};
+            }
+#pragma unroll
+            for (int s = 0; s < NT; ++s) {
+                double hr = 0.0, hi = 0.0;
+                eacc += q12[s].add(rows, s, L, kk, a, hr, hi);
+                double* g = G + static_cast<size_t>((s * M.n_lmh + L * (L + 1) / 2 + L - kk) * 2) * kBlock;
+                g[0] = hr;
+                g[kBlock] = hi;
+            }
         }
     }
     // parts of divided segments: the last task of a wave
     for (int r = 1; r <= M.q3_rounds; ++r) {
         __syncthreads();
         if (pend != r) continue;
+        // all rows read, then all written: one latency, not one per row
+        double* g[NT][LI];
+        double2 v[NT][LI];
+#pragma unroll
+        for (int s = 0; s < NT; ++s)
+#pragma unroll
+            for (int i = 0; i < LI; ++i) {
+                const int L = L0 + 2 * min(i, nL - 1);
+                g[s][i] = G + static_cast<size_t>((s * M.n_lmh + L * (L + 1) / 2 + L - k) * 2) * kBlock;
+                v[s][i] = double2{g[s][i][0], g[s][i][kBlock]};
+            }
 #pragma unroll
         for (int s = 0; s < NT; ++s)
 #pragma unroll
             for (int i = 0; i < LI; ++i) {
                 if (i >= nL) continue;
-                const int L = L0 + 2 * i;
-                double* g = G + static_cast<size_t>((s * M.n_lmh + L * (L + 1) / 2 + L - k) * 2) * kBlock;
-                g[0] += gr[s][i];
-                g[kBlock] += gi[s][i];
+                g[s][i][0] = v[s][i].x + gr[s][i];
+                g[s][i][kBlock] = v[s][i].y + gi[s][i];
             }
     }
     S.Eq34[(((size_t)blk * M.n_fn + n) * kWavesPerWg + wave) * kBlock + lane] = eacc;
