@@ -235,38 +235,61 @@ __global__ __launch_bounds__(64) void k_q12(DevModel M, DevSystem S, int stage) 
 }
 
 // ---------------------------------------------------------------- polynomial
-// One wave per slot: lanes stride the polynomial features.
 //   H_a = lin_a + (W d)_a + sum_{cubic} w d_b d_c
 //   E_P = sum_a d_a (lin_a + Hq_a / 2 + H3_a / 3)   (Euler, homogeneous parts)
-__global__ __launch_bounds__(256) void k_poly(DevModel M, DevSystem S) {
-    const int slot = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    __shared__ double red[4][64];
+// A workgroup per slot with the slot's d in LDS, kPolyLanes lanes per feature:
+// they take its cubic terms in turn, their sums go through a fixed butterfly.
+// Bound: the latency of the term lists (read by every slot, from the caches).  A
+// wave per slot with a feature per lane walked each list serially with d in HBM:
+// cubic model, 32 atoms, 59 us; now 8.7.
+constexpr int kPolyLanes = 16;
+constexpr int kPolyThreads = 256;
+
+// STAGE: the slot's row fits the 64 KB of LDS a launch has by default (8,192
+// features); else it is read from HBM
+template <bool STAGE>
+__global__ __launch_bounds__(kPolyThreads) void k_poly(DevModel M, DevSystem S) {
+    extern __shared__ double poly_d[];
+    __shared__ double red[kPolyThreads / 64];
+    const int slot = blockIdx.x;
+    if (S.atom_of_slot[slot] < 0) return;  // (nothing reads an empty slot's row or energy)
+    // the compact row of the slot's species (features it does not see are zero
+    // and have no column)
+    const int t = S.block_type[slot / kBlock];
+    const double* d = S.D + static_cast<size_t>(slot) * M.n_pr;
+    const double* hq = S.Hq + static_cast<size_t>(slot) * M.n_pr;
+    double* h = S.H + static_cast<size_t>(slot) * M.n_pr;
+    const int w = M.n_fn * (M.prange[t][1] - M.prange[t][0]);
+    const int32_t* c3o = M.c3_off + t * (M.n_pr + 1);
+    const double* lin = M.lin_p + static_cast<size_t>(t) * M.n_pr;
+    if (STAGE) {
+        for (int k = threadIdx.x; k < w; k += kPolyThreads) poly_d[k] = d[k];
+        __syncthreads();
+    }
+    auto dv = [&](int k) { return STAGE ? poly_d[k] : d[k]; };
+    const int u = threadIdx.x % kPolyLanes;
     double e = 0.0;
-    if (slot < S.nblocks * kBlock) {
-        // the compact row of the slot's species (features it does not see
-        // are zero and have no column)
-        const int t = S.block_type[slot / kBlock];
-        const double* d = S.D + (size_t)slot * M.n_pr;
-        const double* hq = S.Hq + (size_t)slot * M.n_pr;
-        double* h = S.H + (size_t)slot * M.n_pr;
-        const int w = M.n_fn * (M.prange[t][1] - M.prange[t][0]);
-        const int32_t* c3o = M.c3_off + t * (M.n_pr + 1);
-        const double* lin = M.lin_p + (size_t)t * M.n_pr;
-        for (int a = lane; a < w; a += 64) {
-            double h3 = 0.0;
-            for (int k = c3o[a]; k < c3o[a + 1]; ++k)
-                h3 = fma(M.c3_w[k], d[M.c3_bc[2 * k]] * d[M.c3_bc[2 * k + 1]], h3);
-            const double la = lin[a];
-            h[a] = la + hq[a] + h3;
-            e = fma(d[a], la + 0.5 * hq[a] + h3 / 3.0, e);
+    for (int a = threadIdx.x / kPolyLanes; a < w; a += kPolyThreads / kPolyLanes) {
+        double h3 = 0.0;
+        const int k1 = c3o[a + 1];
+#pragma unroll 4
+        for (int k = c3o[a] + u; k < k1; k += kPolyLanes)
+            h3 = fma(M.c3_w[k], dv(M.c3_bc[2 * k]) * dv(M.c3_bc[2 * k + 1]), h3);
+#pragma unroll
+        for (int off = kPolyLanes / 2; off > 0; off >>= 1) h3 += __shfl_xor(h3, off);
+        if (u == 0) {
+            const double la = lin[a], q = hq[a];
+            h[a] = la + q + h3;
+            e = fma(dv(a), la + 0.5 * q + h3 / 3.0, e);
         }
     }
-    red[threadIdx.x >> 6][lane] = e;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
+    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = e;
     __syncthreads();
-    if (lane == 0 && slot < S.nblocks * kBlock) {
+    if (threadIdx.x == 0) {
         double s = 0.0;
-        for (int k = 0; k < 64; ++k) s += red[threadIdx.x >> 6][k];
+        for (int k = 0; k < kPolyThreads / 64; ++k) s += red[k];
         S.Ep[slot] = s;
     }
 }
@@ -535,7 +558,11 @@ hipError_t launch_poly(const DevModel& m, const DevSystem& s, hipStream_t st) {
     const int nslot = s.nblocks * kBlock;
     if (nslot == 0 || m.n_p == 0) return hipSuccess;
     if (m.poly_fused) return launch_poly_sum(m, s, st);  // H and the partials came from the GEMM
-    hipLaunchKernelGGL(k_poly, dim3((nslot + 3) / 4), dim3(256), 0, st, m, s);
+    const size_t lds = sizeof(double) * m.n_pr;
+    if (lds + sizeof(double) * (kPolyThreads / 64) <= 64 * 1024)
+        hipLaunchKernelGGL(k_poly<true>, dim3(nslot), dim3(kPolyThreads), lds, st, m, s);
+    else
+        hipLaunchKernelGGL(k_poly<false>, dim3(nslot), dim3(kPolyThreads), 0, st, m, s);
     return launched();
 }
 
