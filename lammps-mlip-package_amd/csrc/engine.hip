@@ -711,7 +711,7 @@ struct Scope {
 
 namespace mlip {
 
-bool run_pipeline(mlip_ctx* c) {
+bool run_pipeline(mlip_ctx* c, const std::function<bool()>& before_gather) {
     const DevModel& m = c->dm;
     const DevSystem& s = c->ds;
     const Model& mm = c->model;
@@ -733,6 +733,7 @@ bool run_pipeline(mlip_ctx* c) {
         run("pair_features", [&] { return launch_pair_features(m, s, st); });
         run("pair_poly", [&] { return launch_pair_poly(m, s, st); });
         run("force", [&] { return launch_pair_force(m, s, st); });
+        if (ok && before_gather && !before_gather()) return false;
         run("gather", [&] { return launch_gather(m, s, st); });
         run("energy_virial", [&] { return launch_energy_virial(m, s, c->total_reduce, st); });
         if (c->nstruct > 0)
@@ -759,6 +760,7 @@ bool run_pipeline(mlip_ctx* c) {
     if (mm.has_order34) run("q34_adj", [&] { return launch_q34_adj(m, s, st); });
     if (mm.has_hi) run("qhigh_adj", [&] { return launch_qhigh(m, s, false, st); });
     run("force", [&] { return launch_force(m, s, c->precision, c->force_threads, st); });
+    if (ok && before_gather && !before_gather()) return false;
     run("gather", [&] { return launch_gather(m, s, st); });
     run("energy_virial", [&] { return launch_energy_virial(m, s, c->total_reduce, st); });
     if (c->nstruct > 0)
@@ -877,16 +879,31 @@ int lammps_compute(mlip_ctx* c, int nlocal, int nghost, const double* x, const i
                    double* eng, double* virial, double* eatom, double* vatom) {
     (void)eflag;
     (void)vflag;
-    LammpsLists L;
+    LammpsLists& L = c->lists;
     const int rc = lammps_lists(c, nlocal, nghost, x, type, tag, inum, ilist, numneigh, firstneigh, neigh_off,
                                 neigh_idx, neigh_full, L);
     if (rc != MLIP_OK) return rc;
     c->resident = false;
     c->nstruct = 0;
-    if (!setup_system(c, L.nall, inum, L.npairs, L.x, L.elem, L.elem_own, L.poff, L.pnbr, &L.pcen, nullptr, L.gof,
-                      L.gen))
+    // the gather lists are formed while the device works on what does not need
+    // them (864 atoms: 0.25 ms on the host, as long as the kernels up to there)
+    if (!upload(c, c->x, L.x.data(), L.x.size(), "positions") ||
+        !upload(c, c->elem, L.elem.data(), L.elem.size(), "elements") ||
+        !upload(c, c->poff, L.poff.data(), L.poff.size(), "pair offsets") ||
+        !upload(c, c->pnbr, L.pnbr.data(), L.pnbr.size(), "pair neighbors") ||
+        !upload(c, c->pcen, L.pcen.data(), L.pcen.size(), "pair centres"))
         return MLIP_ERR_DEVICE;
-    if (!run_pipeline(c)) return MLIP_ERR_DEVICE;
+    if (!c->goff.ensure(static_cast<size_t>(L.nall) + 1) || !c->gent.ensure(2 * static_cast<size_t>(L.npairs))) {
+        c->err = "device allocation failed for gather lists";
+        return MLIP_ERR_DEVICE;
+    }
+    if (!setup_layout(c, L.nall, inum, L.npairs, L.elem_own, true, false)) return MLIP_ERR_DEVICE;
+    auto gather = [&] {
+        lammps_gather(L);
+        return upload(c, c->goff, L.gof.data(), L.gof.size(), "gather offsets") &&
+               upload(c, c->gent, L.gen.data(), L.gen.size(), "gather entries");
+    };
+    if (!run_pipeline(c, gather)) return MLIP_ERR_DEVICE;
     double* epv = nullptr;
     double* evat = nullptr;
     if ((eatom || vatom) && c->atom_mode == MLIP_ATOM_PAIR_SPLIT) {
@@ -924,7 +941,8 @@ int lammps_lists(mlip_ctx* c, int nlocal, int nghost, const double* x, const int
         L.elem[k] = c->elem_of_type[t - 1];
     }
     // owners: ilist order; half lists need the owner of each ghost (by tag)
-    std::vector<int> owner_of_local(nlocal, -1);
+    std::vector<int32_t>& owner_of_local = L.owner_of_local;
+    owner_of_local.assign(nlocal, -1);
     for (int ii = 0; ii < inum; ++ii) {
         if (ilist[ii] < 0 || ilist[ii] >= nlocal) {
             c->err = "ilist entry out of range";
@@ -932,25 +950,51 @@ int lammps_lists(mlip_ctx* c, int nlocal, int nghost, const double* x, const int
         }
         owner_of_local[ilist[ii]] = ii;
     }
-    std::unordered_map<int64_t, int> local_of_tag;
+    // tags to local atoms: a table where the tags are as dense as LAMMPS makes
+    // them (1 .. natoms), a map otherwise
+    std::unordered_map<int64_t, int> local_of_far_tag;
+    const int64_t span = 4 * static_cast<int64_t>(nlocal) + 1024;
+    bool dense = true;
     if (!neigh_full) {
         if (!tag) {
             c->err = "half neighbor lists need atom tags (newton on, single rank)";
             return MLIP_ERR_ARG;
         }
-        local_of_tag.reserve(nlocal * 2);
-        for (int i = 0; i < nlocal; ++i) local_of_tag[tag[i]] = i;
+        for (int i = 0; i < nlocal && dense; ++i) dense = tag[i] >= 0 && tag[i] < span;
+        if (dense) {
+            L.local_of_tag.assign(static_cast<size_t>(span), -1);
+            for (int i = 0; i < nlocal; ++i) L.local_of_tag[tag[i]] = i;
+        } else {
+            local_of_far_tag.reserve(nlocal * 2);
+            for (int i = 0; i < nlocal; ++i) local_of_far_tag[tag[i]] = i;
+        }
     }
+    // owner of position j's atom, or -1
+    auto owner_of = [&](int j) {
+        int i = -1;
+        if (dense) {
+            if (tag[j] >= 0 && tag[j] < span) i = L.local_of_tag[tag[j]];
+        } else {
+            const auto it = local_of_far_tag.find(tag[j]);
+            if (it != local_of_far_tag.end()) i = it->second;
+        }
+        return i < 0 ? -1 : owner_of_local[i];
+    };
     auto list_of = [&](int ii, int& n) -> const int* {
         const int i = ilist[ii];
         n = numneigh[i];
         return firstneigh ? firstneigh[i] : neigh_idx + neigh_off[ii];
     };
-    std::vector<std::vector<std::pair<int32_t, int32_t>>> per(inum);  // (centre pos, neighbor pos)
+    // pairs per owner, then the pairs in the same order (for a half list each entry
+    // gives its centre's owner a pair and its neighbor's owner the reverse)
+    int64_t total = 0;
+    for (int ii = 0; ii < inum; ++ii) total += std::max(0, numneigh[ilist[ii]]);
+    if (!neigh_full) total *= 2;
+    const bool big = total > (INT32_MAX - 1) / 2;  // refused below, after the entries' own errors
+    L.poff.assign(static_cast<size_t>(inum) + 1, 0);
     for (int ii = 0; ii < inum; ++ii) {
         int n = 0;
         const int* js = list_of(ii, n);
-        const int i = ilist[ii];
         if (n < 0 || (n > 0 && !js)) {
             c->err = "bad neighbor count or list";
             return MLIP_ERR_ARG;
@@ -961,39 +1005,70 @@ int lammps_lists(mlip_ctx* c, int nlocal, int nghost, const double* x, const int
                 c->err = "neighbor index out of range";
                 return MLIP_ERR_ARG;
             }
-            per[ii].push_back({i, j});
             if (!neigh_full) {
-                auto it = local_of_tag.find(tag[j]);
-                if (it == local_of_tag.end() || owner_of_local[it->second] < 0) {
+                const int o = owner_of(j);
+                if (o < 0) {
                     c->err = "neighbor tag without a local owner (half lists are single-rank)";
                     return MLIP_ERR_ARG;
                 }
-                per[owner_of_local[it->second]].push_back({j, i});
+                if (!big) ++L.poff[o + 1];
             }
         }
+        if (!big) L.poff[ii + 1] += n;
     }
-    L.poff.assign(inum + 1, 0);
-    L.pnbr.clear();
-    L.pcen.clear();
-    for (int ii = 0; ii < inum; ++ii) {
-        L.poff[ii + 1] = L.poff[ii] + static_cast<int32_t>(per[ii].size());
-        for (const auto& e : per[ii]) {
-            L.pcen.push_back(e.first);
-            L.pnbr.push_back(e.second);
-        }
-    }
-    L.npairs = static_cast<int64_t>(L.pnbr.size());
-    if (L.npairs > (INT32_MAX - 1) / 2) {
+    if (big) {
         c->err = "more than 2^30 pairs";  // gather offsets reach 2 * npairs
         return MLIP_ERR_ARG;
+    }
+    for (int ii = 0; ii < inum; ++ii) L.poff[ii + 1] += L.poff[ii];
+    L.npairs = total;
+    L.pnbr.resize(static_cast<size_t>(total));
+    L.pcen.resize(static_cast<size_t>(total));
+    if (neigh_full) {
+        for (int ii = 0; ii < inum; ++ii) {
+            int n = 0;
+            const int* js = list_of(ii, n);
+            std::copy(js, js + n, L.pnbr.begin() + L.poff[ii]);
+            std::fill_n(L.pcen.begin() + L.poff[ii], n, ilist[ii]);
+        }
+    } else {
+        L.fill.assign(L.poff.begin(), L.poff.end() - 1);
+        auto put = [&](int owner, int cen, int nbr) {
+            const int at = L.fill[owner]++;
+            L.pcen[at] = cen;
+            L.pnbr[at] = nbr;
+        };
+        for (int ii = 0; ii < inum; ++ii) {
+            int n = 0;
+            const int* js = list_of(ii, n);
+            for (int jj = 0; jj < n; ++jj) {
+                put(ii, ilist[ii], js[jj]);
+                put(owner_of(js[jj]), js[jj], ilist[ii]);
+            }
+        }
     }
     // owners are numbered by ilist position; centre and neighbor positions
     // keep their LAMMPS indices through pcen / pnbr
     L.x.assign(x, x + 3 * static_cast<size_t>(nall));
     L.elem_own.assign(inum, 0);
     for (int ii = 0; ii < inum; ++ii) L.elem_own[ii] = L.elem[ilist[ii]];
-    build_gather(nall, L.poff, L.pnbr, &L.pcen, L.gof, L.gen);
     return MLIP_OK;
+}
+
+void lammps_gather(LammpsLists& L) {
+    const size_t np = L.pnbr.size();
+    L.gof.assign(static_cast<size_t>(L.nall) + 1, 0);
+    for (size_t p = 0; p < np; ++p) {
+        ++L.gof[L.pcen[p] + 1];
+        ++L.gof[L.pnbr[p] + 1];
+    }
+    for (int k = 0; k < L.nall; ++k) L.gof[k + 1] += L.gof[k];
+    L.gen.resize(2 * np);
+    L.fill.assign(L.gof.begin(), L.gof.end() - 1);
+    for (size_t p = 0; p < np; ++p) {
+        L.gen[L.fill[L.pcen[p]]++] = -static_cast<int32_t>(p + 1);
+        L.gen[L.fill[L.pnbr[p]]++] = static_cast<int32_t>(p + 1);
+    }
 }
 
 int lammps_results(mlip_ctx* c, int nall, int inum, const int* ilist, double* f, double* eng, double* virial,

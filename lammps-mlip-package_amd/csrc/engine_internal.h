@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -49,7 +50,19 @@ struct TrainWork;  // training-feature tables and outputs (train.hip)
 
 }  // namespace mlip
 
+// A LAMMPS-shaped neighbor list as the engine's pair and gather lists.  Kept in
+// the context from call to call for its memory: fresh vectors of a few megabytes
+// are page faults on every call.
+struct LammpsLists {
+    int nall = 0;
+    int64_t npairs = 0;
+    std::vector<double> x;
+    std::vector<int32_t> elem, elem_own, poff, pnbr, pcen, gof, gen;
+    std::vector<int32_t> owner_of_local, local_of_tag, fill;  // work space
+};
+
 struct mlip_ctx {
+    LammpsLists lists;
     mlip::Model model;
     std::vector<int> elem_of_type;  // LAMMPS type-1 -> element (or -1)
     int precision = mlip::kFP64;
@@ -166,21 +179,19 @@ bool upload(mlip_ctx* c, DBuf<T>& b, const T* h, size_t n, const char* what) {
 }
 
 void drop_graph(mlip_ctx* c);
-bool run_pipeline(mlip_ctx* c);
+// before_gather (when given) runs on the host when everything up to the pair forces
+// is enqueued: it uploads the gather lists
+bool run_pipeline(mlip_ctx* c, const std::function<bool()>& before_gather = nullptr);
 bool run_eval(mlip_ctx* c);
 bool run_atom_split(mlip_ctx* c, double* epv, double* evat);
 // LAMMPS-shaped input (mlip_compute / mlip_compute_flat) turned into the
 // engine's directed-pair lists: both directions of every pair, centre
 // positions kept (pcen), owners in ilist order, force gather lists.
-struct LammpsLists {
-    int nall = 0;
-    int64_t npairs = 0;
-    std::vector<double> x;
-    std::vector<int32_t> elem, elem_own, poff, pnbr, pcen, gof, gen;
-};
 int lammps_lists(mlip_ctx* c, int nlocal, int nghost, const double* x, const int* type, const int64_t* tag, int inum,
                  const int* ilist, const int* numneigh, const int* const* firstneigh, const int* neigh_off,
                  const int* neigh_idx, int neigh_full, LammpsLists& L);
+// gof, gen of such lists
+void lammps_gather(LammpsLists& L);
 // After an evaluation of such lists: adds forces, energy and virial into the
 // caller's arrays and fills eatom / vatom (epv, evat: device scratch of
 // 7 npairs and 7 nall doubles for the pair split, unused in site mode).

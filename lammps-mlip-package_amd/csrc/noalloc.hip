@@ -136,7 +136,7 @@ extern "C" int mlip_compute_flat_noalloc(mlip_ctx* c, int nlocal, int nghost, co
         c->err = "no scratch array on this device: " + serr;
         return MLIP_ERR_DEVICE;
     }
-    LammpsLists L;
+    LammpsLists& L = c->lists;
     int rc = lammps_lists(c, nlocal, nghost, x, type, tag, inum, ilist, numneigh, nullptr, neigh_off, neigh_idx,
                           neigh_full, L);
     if (rc != MLIP_OK) return rc;
@@ -168,13 +168,16 @@ extern "C" int mlip_compute_flat_noalloc(mlip_ctx* c, int nlocal, int nghost, co
         !up(P.b.elem, L.elem.data(), na * sizeof(int32_t), "elements") ||
         !up(P.b.poff, L.poff.data(), L.poff.size() * sizeof(int32_t), "pair offsets") ||
         !up(P.b.pnbr, L.pnbr.data(), np * sizeof(int32_t), "pair neighbors") ||
-        !up(P.b.pcen, L.pcen.data(), np * sizeof(int32_t), "pair centres") ||
-        !up(P.b.goff, L.gof.data(), L.gof.size() * sizeof(int32_t), "gather offsets") ||
-        !up(P.b.gent, L.gen.data(), L.gen.size() * sizeof(int32_t), "gather entries"))
+        !up(P.b.pcen, L.pcen.data(), np * sizeof(int32_t), "pair centres"))
         return MLIP_ERR_DEVICE;
     c->resident = false;
     c->nstruct = 0;
     if (!bind_system(c, L.nall, inum, L.npairs, L.elem_own, aos, sos, bt, P.b)) return MLIP_ERR_DEVICE;
-    if (!run_pipeline(c)) return MLIP_ERR_DEVICE;
+    auto gather = [&] {
+        lammps_gather(L);
+        return up(P.b.goff, L.gof.data(), L.gof.size() * sizeof(int32_t), "gather offsets") &&
+               up(P.b.gent, L.gen.data(), L.gen.size() * sizeof(int32_t), "gather entries");
+    };
+    if (!run_pipeline(c, gather)) return MLIP_ERR_DEVICE;
     return lammps_results(c, L.nall, inum, ilist, f, eng, virial, eatom, vatom, P.epv, P.evat);
 }
