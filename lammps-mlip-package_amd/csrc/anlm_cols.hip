@@ -19,8 +19,9 @@
 // Bound: the FP64 pipe, which matrix and vector instructions share on this
 // device (69 and 50 TFLOP/s alone, 56-67 together): per step of four neighbors
 // 13 products of 64 cycles and ~90 vector instructions.  256k atoms (137 neighbors,
-// l_max 12, 12 functions): 9.4 ms with the order-1/2 features (7.0 without;
-// the pipe is 73% busy), 3,991 atoms 198 us.  Before: a workgroup of four waves
+// l_max 12, 12 functions): 8.2 ms with the order-1/2 features (7.0 without),
+// 3,991 atoms 177 us (features from tables in HBM, four barriers a round: 9.4 ms,
+// 198 us).  Before: a workgroup of four waves
 // with chunks of 16 mixed neighbors, a column per thread through LDS and two
 // barriers per chunk, 11.9 ms, and a feature pass that re-read a_nlm, 2.6 ms
 // (3,991 atoms: 250 + 62 us).  Also tried: columns formed a lane per neighbor
@@ -45,6 +46,7 @@ typedef double dbl4 __attribute__((ext_vector_type(4)));
 
 constexpr double kPiRef = 3.141592653589793;  // mlip_basis_function.cpp:26
 constexpr int kBatch = 64;  // neighbors per batch
+constexpr int kColsFeat = 48;  // order-1/2 features per species (41 for two species and l_max 12)
 
 // T: type of z and the start powers (FP32 in the mixed mode; g, the recursion,
 // products and sums are FP64)
@@ -58,13 +60,14 @@ struct Lds {
         };
         double buf[kColsBuf];         // a round of the epilogue
     };
+    double fw[kColsFeat][kQ12Weights];  // order-1/2 features of the centre's species: weights,
+    uint32_t fd[kColsFeat];             // order | L | s0 | s1 in 4 bits each, column above
 };
 
 template <typename T, int LT, int NS>
 __global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(3))) void k_anlm_cols(DevModel M, DevSystem S,
                                                                                               int feat) {
     __shared__ Lds<T, LT> L;
-    static_assert(sizeof(Lds<T, LT>) == sizeof(L.buf));
     const int slot = xcd_slot(blockIdx.x, S.nblocks);
     if (slot < 0) return;
     const int atom = S.atom_of_slot[slot];
@@ -85,6 +88,17 @@ __global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(3))) vo
     dbl4 acc[LT];
 #pragma unroll
     for (int t = 0; t < LT; ++t) acc[t] = dbl4{0.0, 0.0, 0.0, 0.0};
+    // The features' tables, here because a read behind the stores of a_nlm waits for
+    // them
+    const int blk = slot / kBlock, slane = slot % kBlock;
+    const int ty = S.block_type[blk];
+    const int f0 = M.fq12_off[ty], nfe = feat ? M.fq12_off[ty + 1] - f0 : 0;
+    for (int k = tid; k < nfe * kQ12Weights; k += 64 * NS)
+        L.fw[k / kQ12Weights][k % kQ12Weights] = M.fq12w[static_cast<size_t>(f0) * kQ12Weights + k];
+    for (int k = tid; k < nfe; k += 64 * NS) {
+        const FeatQ12 f = M.fq12[f0 + k];
+        L.fd[k] = f.order | f.L << 4 | f.s0 << 8 | f.s1 << 12 | f.col << 16;
+    }
     const int p0 = S.poff[atom], p1 = S.pend[atom];
     const double pir = kPiRef / M.cutoff;
     for (int b0 = p0; b0 < p1; b0 += kBatch) {
@@ -158,19 +172,22 @@ __global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(3))) vo
             }
         }
     }
-    const int blk = slot / kBlock, slane = slot % kBlock;
-    // norms, then a_nlm to HBM: result r of lane (lq, li) is radial index lq + 4 r
+    // norms, then a_nlm to HBM: result r of lane (lq, li) is radial index lq + 4 r.
+    // Each step's table reads wait for the stores before them, which paces these
+    // 8-byte stores so that the L2 gathers the lines of neighboring slots: all
+    // tables first, then all stores, took 9.4 ms instead of 8.2.
     double* ab = S.A + a_index(M, blk, 0, wave, 0, 0, slane);
     const uint32_t np = static_cast<uint32_t>(NS * nlmh) * 2 * kBlock;  // stride of a radial index
+    int lmc[LT];
 #pragma unroll
     for (int t = 0; t < LT; ++t) {
-        const int lmc = M.cols->lmc[t][li];
         const double nrm = M.cols->norm[t][li];
-        const uint32_t at = lq * np + static_cast<uint32_t>(lmc) * kBlock;
+        lmc[t] = M.cols->lmc[t][li];
+        const uint32_t at = lq * np + static_cast<uint32_t>(lmc[t]) * kBlock;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             acc[t][r] *= nrm;
-            if (lmc >= 0 && lq + 4 * r < nfn) (ab + 4 * r * np)[at] = acc[t][r];
+            if (lmc[t] >= 0 && lq + 4 * r < nfn) (ab + 4 * r * np)[at] = acc[t][r];
         }
     }
     if (!feat) return;
@@ -179,43 +196,52 @@ __global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(3))) vo
     // as [n][s][lm](re, im), thread per (feature, n) with n fastest (the
     // features are listed by L, so a wave's items have nearly equal lengths),
     // the round's row segment (zero where no order-1/2 family writes) stored as
-    // one run of the slot's compact row.
-    const int ty = S.block_type[blk];
-    const int lo = M.prange[ty][0], w = M.prange[ty][1] - lo;
-    const int f0 = M.fq12_off[ty], nfe = M.fq12_off[ty + 1] - f0;
+    // one run of the slot's compact row.  Two barriers a round: the segment
+    // alternates between two places, so that it is stored while the next round
+    // begins.
+    const int w = M.prange[ty][1] - M.prange[ty][0];
     double* as = L.buf;                        // [n][s][lm] (re, im)
-    double* seg = as + 4 * NS * nlmh * 2;      // [n][rank - lo]
+    double* segs = as + 4 * NS * nlmh * 2;     // two of [n][rank - lo]
+    __syncthreads();
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int r0 = 4 * r, rn = min(4, nfn - r0);
         if (rn <= 0) break;
-        __syncthreads();
+        double* seg = segs + (r & 1) * 4 * w;
 #pragma unroll
-        for (int t = 0; t < LT; ++t) {
-            const int lmc = M.cols->lmc[t][li];
-            if (lmc >= 0 && lq < rn) as[((lq * NS + wave) * nlmh) * 2 + lmc] = acc[t][r];
-        }
+        for (int t = 0; t < LT; ++t)
+            if (lmc[t] >= 0 && lq < rn) as[((lq * NS + wave) * nlmh) * 2 + lmc[t]] = acc[t][r];
         for (int e = tid; e < rn * w; e += 64 * NS) seg[e] = 0.0;
         __syncthreads();
         for (int it = tid; it < nfe * rn; it += 64 * NS) {
             const int fi = it / rn, nl = it - fi * rn;
-            const FeatQ12 f = M.fq12[f0 + fi];
-            const double* wt = M.fq12w + static_cast<size_t>(f0 + fi) * kQ12Weights;
-            const double2* x = reinterpret_cast<const double2*>(as) + (nl * NS + f.s0) * nlmh;
+            const uint32_t f = L.fd[fi];
+            const double* wt = L.fw[fi];
+            const double2* x = reinterpret_cast<const double2*>(as) + (nl * NS + (f >> 8 & 15)) * nlmh;
             double d;
-            if (f.order == 1) {
+            if ((f & 15) == 1) {
                 d = wt[0] * x[0].x;
             } else {
-                // the order-1/2 pass's pair-summed form, same order of terms
-                const double2* y = reinterpret_cast<const double2*>(as) + (nl * NS + f.s1) * nlmh;
-                const int fl = f.L, b = fl * (fl + 1) / 2 + fl;  // lmh(L, 0); lmh(L, -k) = b - k
+                // the order-1/2 pass's pair-summed form, same order of terms;
+                // four at a time (weights past L are zero), their reads together
+                const double2* y = reinterpret_cast<const double2*>(as) + (nl * NS + (f >> 12 & 15)) * nlmh;
+                const int fl = f >> 4 & 15, b = fl * (fl + 1) / 2 + fl;  // lmh(L, 0); lmh(L, -k) = b - k
                 d = 0.0;
-                for (int k = 0; k <= fl; ++k) {
-                    const double2 xv = x[b - k], yv = y[b - k];
-                    d = fma(wt[k], xv.x * yv.x + xv.y * yv.y, d);
+                for (int k = 0; k <= fl; k += 4) {
+                    double2 xv[4], yv[4];
+                    double wv[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int at = b - min(k + j, fl);
+                        xv[j] = x[at];
+                        yv[j] = y[at];
+                        wv[j] = wt[k + j];
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) d = fma(wv[j], xv[j].x * yv[j].x + xv[j].y * yv[j].y, d);
                 }
             }
-            seg[nl * w + f.col] = d;
+            seg[nl * w + (f >> 16)] = d;
         }
         __syncthreads();
         double* drow = S.D + static_cast<size_t>(slot) * M.n_pr + static_cast<size_t>(r0) * w;
@@ -262,10 +288,10 @@ void build_cols_tables(int maxl, ColsTab& t) {
 
 bool anlm_cols_fits(const DevModel& m) { return m.cols != nullptr && m.maxl <= kColsMaxL && m.n_fn <= 16 && m.n_type <= 2; }
 
-// a round's a_nlm and row segment fit the LDS buffer
+// the features' tables, a round's a_nlm and two row segments fit the LDS
 bool anlm_cols_features(const DevModel& m) {
     for (int t = 0; t < m.n_type; ++t)
-        if (4 * (2 * m.n_type * m.n_lmh + (m.prange[t][1] - m.prange[t][0])) > kColsBuf) return false;
+        if (m.fq12_off[t + 1] - m.fq12_off[t] > kColsFeat || m.prange[t][1] - m.prange[t][0] > 65535 || 4 * (2 * m.n_type * m.n_lmh + 2 * (m.prange[t][1] - m.prange[t][0])) > kColsBuf) return false;
     return true;
 }
 

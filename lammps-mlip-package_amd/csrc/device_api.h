@@ -48,8 +48,8 @@ struct ForceTab {
     int32_t row[(kForceEntries + 1) / 2][16];
 };
 // weights of an order-1/2 feature's terms m = 0 .. L (L <= 12): the coefficients
-// of +m and -m summed, with the sign (-1)^m
-constexpr int kQ12Weights = 14;
+// of +m and -m summed, with the sign (-1)^m; zero from L + 1
+constexpr int kQ12Weights = 16;
 
 struct DevModel {
     int n_type, n_fn, n_gtinv, n_lmh, maxl, lmax3, n_pitc, n_p;
