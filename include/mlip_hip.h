@@ -186,9 +186,9 @@ int mlip_graph_mode(mlip_ctx* ctx, int on);
 int mlip_autotune(mlip_ctx* ctx, int reps, int* chosen);
 
 /* a_nlm kernel: 0 = thread per lm column with FP64 register accumulators,
- * 1 = chunk products on the matrix cores (FP64 MFMA; the default, used when
- * the model has l_max <= 12, two species and at most 32 radial functions,
- * else kernel 0 runs).  Both give the same sums up to rounding order. */
+ * 1 = products on the matrix cores (FP64 MFMA; the default, used when the
+ * model has l_max <= 12, at most two species and 32 radial functions, else
+ * kernel 0 runs).  Both give the same sums up to rounding order. */
 int mlip_set_anlm_kernel(mlip_ctx* ctx, int kind);
 int mlip_get_anlm_kernel(const mlip_ctx* ctx);
 
@@ -207,7 +207,8 @@ int mlip_autotune_q34(mlip_ctx* ctx, int reps, int* plan3);
 int mlip_set_q34_plan(mlip_ctx* ctx, int region_cost, int visit_cost, int pair_lmax);
 
 /* Sets the force kernel's launch shape directly (64, 128, 192 or 256
- * threads per workgroup; 192 by default).  Results do not depend on it
+ * threads per workgroup; 256 by default), for models with l_max <= 12 and at
+ * most 16 radial functions; others have one shape.  Results do not depend on it
  * beyond the summation order of the per-atom virial. */
 int mlip_set_force_threads(mlip_ctx* ctx, int threads);
 

@@ -207,10 +207,10 @@ size_t lds_limit();
 hipError_t launched(size_t lds_bytes = 0);
 
 // a_nlm kernels: kAnlmValu (k_anlm, thread per lm column, FP64 registers) or
-// kAnlmMfma (k_anlm_mfma, chunk products on the matrix cores) where the
-// model fits it (anlm_has_mfma), k_anlm otherwise
+// kAnlmMfma (matrix cores: k_anlm_cols up to 16 radial functions, k_anlm_mfma up
+// to 32) where the model fits one (anlm_has_mfma), k_anlm otherwise
 enum AnlmKind : int { kAnlmValu = 0, kAnlmMfma = 1 };
-// feat: the register kernel also forms the order-1/2 polynomial features
+// feat: k_anlm and k_anlm_cols also form the order-1/2 polynomial features
 // (what k_q12<true> does) from the a_nlm it holds; only where
 // anlm_forms_features says the launch can
 hipError_t launch_anlm(const DevModel& m, const DevSystem& s, int precision, hipStream_t st, int kind = kAnlmValu,

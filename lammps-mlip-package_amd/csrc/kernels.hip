@@ -2,14 +2,17 @@
 //
 // Pipeline for one evaluation (reference: PairMLIPGtinv::compute,
 // src/USER-MLIP/pair_mlip_gtinv.cpp:63-125, and docs/formulation.md):
-//   k_anlm   a_{i,s,n,lm} = sum_j g_n(r_ij) Y_lm(r_ij)          (:349-447, pair_kernels.hip)
-//   k_q12    order-1/2 invariants: polynomial features or adjoint G
-//   k_q34    order-3/4 invariants: polynomial features or adjoint G,
-//            a_nlm tile of 64 same-species centres resident in LDS
-//   k_gemm_rows  Hq = D W (quadratic form of the polynomial model, FP64 MFMA; gemm.hip),
-//                or, without cubic terms, H and the polynomial energy in its epilogue
+//   k_anlm_cols  a_{i,s,n,lm} = sum_j g_n(r_ij) Y_lm(r_ij) and the order-1/2
+//                features (:349-447, anlm_cols.hip; larger models pair_kernels.hip)
+//   k_q12    order-1/2 invariants where no other kernel forms them
+//   k_gemm_rows, k_gemm_small  Hq = D W (quadratic form of the polynomial model, FP64
+//                MFMA; gemm.hip), or, without cubic terms, H and the polynomial energy
 //   k_poly   E_i polynomial part and H = dE_i/dd                 (:321-343,481-521)
-//   k_force  per-pair dE_i/d(del) from G and dphi/d(del)          (:161-256, pair_kernels.hip)
+//   k_q3, k_q4  order-3/4 adjoint of families outside the polynomial (q3.hip)
+//   k_q34    order-3/4 invariants in the polynomial: features and adjoint,
+//            a_nlm tile of 64 same-species centres resident in LDS
+//   k_force_cols  per-pair dE_i/d(del) from G and dphi/d(del)     (:161-256,
+//                force_cols.hip; larger models pair_kernels.hip)
 //   k_gather atomics-free per-position force sums, deterministic
 //   k_energy, k_totals  per-centre energies and virial, fixed-order reductions
 //

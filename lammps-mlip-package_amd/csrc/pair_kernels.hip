@@ -1,4 +1,6 @@
-// Per-pair kernels of the gtinv path: a_nlm accumulation and pair forces,
+// Per-pair kernels of the gtinv path for models beyond the matrix-core kernels
+// of anlm_cols.hip and force_cols.hip (l_max above 12, or more than 16 radial
+// functions), and the register a_nlm kernel: a_nlm accumulation and pair forces,
 // each in FP64 and in the mixed mode (FP32 per-pair geometry, radial
 // functions, Y_lm and their gradients; FP64 accumulation of a_nlm, FP64
 // pair forces out of the kernel, FP64 virial).
@@ -369,7 +371,8 @@ __global__ __launch_bounds__(NTH) void k_anlm(DevModel M, DevSystem S, int ngrou
 }
 
 // ---------------------------------------------------------------- a_nlm on the matrix cores
-// The same sum as a product per chunk of 16 neighbors:
+// For 17 to 32 radial functions.  The same sum as a product per chunk of 16
+// neighbors:
 //   a_s[n][(lm, re/im)] += sum_k At[k][n] Y[k][(lm, re/im)],
 // k = the chunk's neighbors with species s, on v_mfma_f64_16x16x4f64 (A[i][k]
 // from lane 16 k + i, B[k][j] from lane 16 k + j, result register r of lane
