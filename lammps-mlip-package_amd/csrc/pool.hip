@@ -123,6 +123,14 @@ __global__ __launch_bounds__(256) void k_disp_next(const NveDesc* d, const int32
     if (threadIdx.x == 0) out[blockIdx.x] = sqrt(sh[0]);
 }
 
+// A released request's atoms own no pairs and no gather entries: one launch for
+// the four ranges (as four memsets, 24 requests spent 0.5 ms of 11.5 on them)
+__global__ __launch_bounds__(256) void k_release(int32_t* pbeg, int32_t* pend, int32_t* gbeg, int32_t* gend, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    pbeg[i] = pend[i] = gbeg[i] = gend[i] = 0;
+}
+
 __global__ void k_scatter_slots(const int32_t* atom_of_slot, int nslot, int32_t* slot_of_atom) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nslot) return;
@@ -662,11 +670,11 @@ int admit_device(mlip_ctx* c, Pool* p, int count, const int* natoms, const int64
 // any more).
 bool release_request(mlip_ctx* c, Pool* p, Request& r) {
     const size_t a0 = static_cast<size_t>(r.a0), n = static_cast<size_t>(r.natoms);
-    if (!hip_ok(c, hipMemsetAsync(p->pbeg.p + a0, 0, n * 4, c->stream), "pool release") ||
-        !hip_ok(c, hipMemsetAsync(p->pend.p + a0, 0, n * 4, c->stream), "pool release") ||
-        !hip_ok(c, hipMemsetAsync(p->gbeg.p + a0, 0, n * 4, c->stream), "pool release") ||
-        !hip_ok(c, hipMemsetAsync(p->gend.p + a0, 0, n * 4, c->stream), "pool release"))
-        return false;
+    if (n > 0) {
+        hipLaunchKernelGGL(k_release, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, c->stream,
+                           p->pbeg.p + a0, p->pend.p + a0, p->gbeg.p + a0, p->gend.p + a0, static_cast<int>(n));
+        if (!hip_ok(c, hipGetLastError(), "pool release")) return false;
+    }
     p->atoms.give(r.a0, r.natoms);
     p->pairs.give(r.p0, std::max<int64_t>(r.np, 1));
     return true;
