@@ -39,6 +39,7 @@
 
 #include "device_api.h"
 #include "device_common.h"
+#include "q3_rows.h"
 #include "q4_terms.h"
 
 namespace mlip {
@@ -335,13 +336,13 @@ __global__ __launch_bounds__(kQ3Threads) void k_q3(DevModel M, DevSystem S, int 
     }
     // rows above the tile, order-1/2 families only: each L's m = -kk dealt over
     // `share` waves, a_nlm read from HBM an entry ahead
-    const int nhi = min(M.maxl, kMaxLQ12) - M.lmaxq3, share = nhi > 0 ? (kWavesPerWg + nhi - 1) / nhi : 1;
+    const int nhi = q3_rows_above(M.lmaxq3, M.maxl), share = q3_row_share(M.lmaxq3, nhi);
     for (int it = wave; it < nhi * share; it += kWavesPerWg) {
-        const int L = M.lmaxq3 + 1 + it / share;
+        const int L = q3_row_level(it, share, M.lmaxq3);
         const double* src = S.A + a_index(M, blk, n, 0, L * (L + 1) / 2 + L, 0, lane);
         const int sp = M.n_lmh * 2 * kBlock;
         double2 an[NT];
-        int kk = it % share;
+        int kk = q3_row_first(it, share);  // (<= L)
 #pragma unroll
         for (int s = 0; s < NT; ++s) an[s] = double2{src[s * sp - 2 * kk * kBlock], src[s * sp - (2 * kk - 1) * kBlock]};
         Sources12<NT> q12[NT];
