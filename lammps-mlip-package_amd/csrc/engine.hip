@@ -830,14 +830,15 @@ bool run_atom_split(mlip_ctx* c, double* epv, double* evat) {
         se.H = se.Hq;
         if (me.poly_fused) {
             // without cubic terms He = lin / q + D W' with W'_ab = W_ab / (q_a +
-            // q_b): the quadratic-form product with split weights (its energy
-            // partials go to the old H, which this pass no longer reads); one
-            // wave per centre over W took 982 us at 864 atoms of the order-4 model
+            // q_b): the quadratic-form product with split weights, into Hq and
+            // without energy partials (the evaluation's H stays); one wave per
+            // centre over W took 982 us at 864 atoms of the order-4 model
             DevModel mg = me;
             DevSystem sg = c->ds;
             mg.wmat = me.wmat_e;
             mg.lin_p = me.lin_e;
-            std::swap(sg.H, sg.Hq);
+            sg.H = sg.Hq;
+            sg.Hq = nullptr;
             run("poly_split", launch_poly_gemm(mg, sg, c->nblk_type, st));
         } else if (me.n_p > 0) {
             run("poly_split", launch_poly_split(me, se, st));

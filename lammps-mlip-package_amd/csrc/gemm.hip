@@ -28,7 +28,8 @@ namespace {
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 
 // Per species: its rows of D, its form (w x w), the output rows, and for the
-// fused polynomial step linear weights and energy partials; ld = row pitch.
+// fused polynomial step linear weights and energy partials (null: not wanted);
+// ld = row pitch.
 struct GemmArgs {
     const double* A[2];
     const double* B[2];
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(kGThreads) __attribute__((amdgpu_waves_per_eu(4))) 
                 if ((lane & 15) == 0) esum[wc][rt] = e;
             }
         __syncthreads();
-        if (tid < kGM) epart[static_cast<size_t>(m0 + tid) * ldep + nt] = esum[0][tid] + esum[1][tid];
+        if (epart && tid < kGM) epart[static_cast<size_t>(m0 + tid) * ldep + nt] = esum[0][tid] + esum[1][tid];
         return;
     }
 #pragma unroll
@@ -251,7 +252,7 @@ __global__ __launch_bounds__(kSThreads) void k_gemm_small(GemmArgs G) {
 #pragma unroll
         for (int o = 1; o < 16; o <<= 1) e += __shfl_xor(e, o);
         const double other = __shfl_xor(e, 16);
-        if ((threadIdx.x & 31) == 0) G.epart[t][static_cast<size_t>(mt * kSM + row) * ld + nt] = e + other;
+        if (G.epart[t] && (threadIdx.x & 31) == 0) G.epart[t][static_cast<size_t>(mt * kSM + row) * ld + nt] = e + other;
     }
 }
 
@@ -299,7 +300,7 @@ hipError_t launch_poly_gemm(const DevModel& m, const DevSystem& s, const int* nb
         g.B[t] = m.wmat + m.wofs[t];
         g.C[t] = (m.poly_fused ? s.H : s.Hq) + r0;
         g.lin[t] = m.lin_p + static_cast<size_t>(t) * m.n_pr;
-        g.epart[t] = s.Hq + r0;
+        g.epart[t] = s.Hq ? s.Hq + r0 : nullptr;
         g.w[t] = w;
         if (small) {
             lds = std::max(lds, small_lds(w));
