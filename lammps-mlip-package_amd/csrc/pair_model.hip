@@ -109,6 +109,12 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_feat(DevModel M, DevSyste
 // Bound: the row loop's latency.  One thread per centre over the derivative
 // lists (66k entries, dependent loads) took 12.3 ms at 2,048 atoms of the
 // 20-function cubic model whatever the atom count up to one wave per CU.
+// Rounding: the products reach 1e5 against energies of a few eV, so the order of
+// the additions decides what is lost.  rms force error against 80 bits (500 and
+// 2,048 atoms of that model, of the rms force): one chain per derivative over the
+// lists 2.9e-13 .. 3.2e-13; four plain chains per column, as the split alone gives,
+// 6.1e-13 .. 6.5e-13; with the additions of eight rows each compensated (Kahan)
+// 2.4e-13 (224 us a step of the 2,048 atoms; the plain four chains 227 us).
 constexpr int kPolySplit = 4;
 
 __global__ __launch_bounds__(1024) void k_pair_poly_dense(DevModel M, DevSystem S) {
@@ -131,16 +137,27 @@ __global__ __launch_bounds__(1024) void k_pair_poly_dense(DevModel M, DevSystem 
     const int wave = uniform(threadIdx.x >> 6), tile = wave % ntile, split = wave / ntile;
     const double* w = M.pd_w + static_cast<size_t>(t) * (M.pd_k2 + M.pd_k3) * M.pd_cols + tile * 16 + (lane & 15);
     const double* di = d + (lane & 15) * pitch;
+    // two steps' products by the instruction, added with the rounding of each
+    // addition carried into the next (see above)
     auto sum = [&](int k0, int k1) {
-        dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-        for (int k = k0; k < k1; k += 4) {
+        const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
+        auto step = [&](int k, dbl4 acc) __attribute__((always_inline)) {
             const int kk = k + (lane >> 4);
             const int bc = M.pd_bc[kk];
             const double a = di[bc & 0xffff] * di[bc >> 16];
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, w[static_cast<size_t>(kk) * M.pd_cols], acc, 0, 0, 0);
-        }
-        return acc;
+            return __builtin_amdgcn_mfma_f64_16x16x4f64(a, w[static_cast<size_t>(kk) * M.pd_cols], acc, 0, 0, 0);
+        };
+        dbl4 acc = zero, over = zero;
+        auto add = [&](dbl4 p) __attribute__((always_inline)) {
+            const dbl4 y = p - over, t = acc + y;
+            over = (t - acc) - y;
+            acc = t;
+        };
+        int k = k0;
+#pragma unroll 4
+        for (; k + 4 < k1; k += 8) add(step(k + 4, step(k, zero)));
+        if (k < k1) add(step(k, zero));
+        return acc - over;
     };
     // row ranges of the split, in steps of 4
     const int q2 = M.pd_k2 / 4, q3 = M.pd_k3 / 4;
