@@ -14,8 +14,11 @@ namespace mlip {
 constexpr int kBlock = kBlockLanes;  // atoms per slot block (one wavefront of lanes)
 
 
-// doubles of DevSystem::red: partial energies, then partial virials
-constexpr int kRedDoubles = 4096;
+// DevSystem::red: partial energies, then partial virials of six components.  The
+// fixed scratch of mlip_compute_flat_noalloc holds it beside the structure, so
+// it stays small.
+constexpr int kEnergyParts = 512, kVirialParts = 64;
+constexpr int kRedDoubles = kEnergyParts + 6 * kVirialParts;
 
 enum Precision : int { kFP64 = 0, kMixed = 1 };
 

@@ -452,6 +452,7 @@ __global__ __launch_bounds__(kEnergyThreads) void k_energy(DevModel M, DevSystem
     const int part = blockIdx.x - eparts;
     double v = 0.0;
     if (tid < 6 * kVirRows)
+#pragma unroll 4
         for (int64_t i = static_cast<int64_t>(part) * kVirRows + tid / 6; i < S.nown;
              i += static_cast<int64_t>(vparts) * kVirRows)
             v += S.vown[6 * i + tid % 6];
@@ -460,7 +461,7 @@ __global__ __launch_bounds__(kEnergyThreads) void k_energy(DevModel M, DevSystem
     if (tid < 6) {
         double s = 0.0;
         for (int k = 0; k < kVirRows; ++k) s += sh[6 * k + tid];
-        S.red[kRedDoubles / 2 + part * 6 + tid] = s;
+        S.red[kEnergyParts + part * 6 + tid] = s;
     }
 }
 
@@ -471,7 +472,7 @@ __global__ __launch_bounds__(64 * 7) void k_totals(DevSystem S, int eparts, int 
     if (c == 0) {
         for (int i = lane; i < eparts; i += 64) s += S.red[i];
     } else {
-        for (int i = lane; i < vparts; i += 64) s += S.red[kRedDoubles / 2 + i * 6 + c - 1];
+        for (int i = lane; i < vparts; i += 64) s += S.red[kEnergyParts + i * 6 + c - 1];
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
@@ -613,8 +614,8 @@ hipError_t launch_struct_reduce(const DevSystem& s, const int32_t* sbeg, const i
 }
 
 hipError_t launch_energy_virial(const DevModel& m, const DevSystem& s, bool totals, hipStream_t st) {
-    const int eparts = std::min(s.nblocks, kRedDoubles / 2);
-    const int vparts = totals ? std::min(kRedDoubles / 2 / 6, (s.nown + kVirRows - 1) / kVirRows) : 0;
+    const int eparts = std::min(s.nblocks, kEnergyParts);
+    const int vparts = totals ? std::min(kVirialParts, (s.nown + kVirRows - 1) / kVirRows) : 0;
     if (eparts + vparts > 0)
         hipLaunchKernelGGL(k_energy, dim3(eparts + vparts), dim3(kEnergyThreads), 0, st, m, s, eparts, vparts);
     const hipError_t e = launched();
