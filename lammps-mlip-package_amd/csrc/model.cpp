@@ -749,8 +749,25 @@ void extract_order4(Model& m, int t) {
     tt.plan_adj.swap(rest);
 }
 
+// One order-1/2 family per row species, l and factor species, as TypeTables::q12r
+// holds them.
+bool single_order12(const Model& m) {
+    std::map<std::array<int, 4>, int> seen;  // (centre type, S, L, factor species or 2) -> family
+    for (int t = 0; t < m.n_type; ++t)
+        for (int i = 0; i < m.n_gtinv; ++i) {
+            const Itc& it = m.itcs[i];
+            if (it.order > 2 || !((it.type_mask >> t) & 1u)) continue;
+            for (int p = 0; p < it.order; ++p) {
+                const int S = m.tcp_other[it.tc[p]][t], other = it.order == 2 ? m.tcp_other[it.tc[1 - p]][t] : 2;
+                const auto at = seen.insert({{t, S, m.irreps[it.irrep].l[0], other}, i}).first;
+                if (at->second != i) return false;
+            }
+        }
+    return true;
+}
+
 // Order-1/2 families of centre type t by adjoint row (TypeTables::q12r).
-bool rows_order12(Model& m, int t, const std::vector<std::map<std::vector<int>, double>>& cmap) {
+void rows_order12(Model& m, int t, const std::vector<std::map<std::vector<int>, double>>& cmap) {
     std::vector<int32_t>& r = m.types[t].q12r;
     r.assign(2 * (kMaxLQ12 + 1) * 6, kNoSource);
     for (int i = 0; i < m.n_gtinv; ++i) {
@@ -764,9 +781,7 @@ bool rows_order12(Model& m, int t, const std::vector<std::map<std::vector<int>, 
             // C(k, -k) (p = 1); order 1: C
             const int S = m.tcp_other[it.tc[p]][t], other = q == 2 ? m.tcp_other[it.tc[1 - p]][t] : 2;
             int32_t* e = &r[(S * (kMaxLQ12 + 1) + L) * 6 + 2 * other];
-            if (e[0] != kNoSource && e[0] != src) return false;
-            const bool fresh = e[0] == kNoSource;
-            if (fresh) {
+            if (e[0] == kNoSource) {
                 e[0] = src;
                 e[1] = static_cast<int32_t>(m.coef.size());
                 m.coef.resize(m.coef.size() + L + 1, 0.0);
@@ -776,11 +791,11 @@ bool rows_order12(Model& m, int t, const std::vector<std::map<std::vector<int>, 
                                            : lookup(cm, p == 0 ? std::vector<int>{-k, k} : std::vector<int>{k, -k});
         }
     }
-    return true;
 }
 
-// Builds the flattened visit tables for centre type t.
-void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<int>, double>>& cmap,
+// Builds the flattened visit tables for centre type t; by_output: order-3 linear
+// families go to the order-3 kernel's entries.
+void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<int>, double>>& cmap, bool by_output,
                        std::vector<Entry3>& entries) {
     TypeTables tt;
     std::vector<std::vector<VisitQ12>> by_l(m.maxl + 1);
@@ -1004,7 +1019,7 @@ void build_type_tables(Model& m, int t, const std::vector<std::map<std::vector<i
         }
         adj.swap(merged);
     }
-    extract_order3(m, adj, entries);
+    if (by_output) extract_order3(m, adj, entries);
     tt.plan_adj = std::move(adj);
     tt.plan_feat = std::move(feat);
     m.types[t] = std::move(tt);
@@ -1488,7 +1503,10 @@ bool load_model(const std::string& path, const GtinvTable& table, Model& m, std:
     m.types.assign(m.n_type, TypeTables());
     m.c3q.clear();
     std::vector<std::vector<Entry3>> entries(m.n_type);
-    for (int t = 0; t < m.n_type; ++t) build_type_tables(m, t, cmap, entries[t]);
+    // (families the rows of the order-3 kernel cannot hold stay the order-3/4 and
+    // order-1/2 kernels', which add any number to a row)
+    const bool by_output = single_order12(m);
+    for (int t = 0; t < m.n_type; ++t) build_type_tables(m, t, cmap, by_output, entries[t]);
     m.lmaxq3 = -1;
     for (int t = 0; t < m.n_type; ++t)
         for (const Entry3& e : entries[t]) m.lmaxq3 = std::max({m.lmaxq3, e.L, e.lb});
@@ -1497,10 +1515,7 @@ bool load_model(const std::string& path, const GtinvTable& table, Model& m, std:
         for (int t = 0; t < m.n_type; ++t) {
             plan_order3(m, m.types[t], entries[t]);
             extract_order4(m, t);
-            if (!rows_order12(m, t, cmap)) {
-                err = "internal: two order-1/2 families of one species pair and l";
-                return false;
-            }
+            rows_order12(m, t, cmap);
         }
     // tile of the order-3/4 adjoint kernel: the visits it keeps
     m.lmax_t = 0;
