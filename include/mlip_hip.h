@@ -77,7 +77,11 @@ int mlip_set_atom_mode(mlip_ctx* ctx, int mode);
  * Accumulates into f[nall][3] (ghost entries are left for LAMMPS reverse
  * communication); adds to *eng_vdwl and virial6 (xx, yy, zz, xy, xz, yz).
  * eatom[nall] and vatom6[nall][6] (nullable) are accumulated as
- * mlip_set_atom_mode selects. */
+ * mlip_set_atom_mode selects.
+ * The context keeps the host memory of a call's lists (16 bytes per directed
+ * pair, 64 per position) for the next one: at most four times what the last
+ * call used (3 MB aside), nothing once it holds a resident structure, a batch
+ * or a pool. */
 int mlip_compute(mlip_ctx* ctx, int nlocal, int nghost, const double* x, const int* type,
                  const int64_t* tag, int inum, const int* ilist, const int* numneigh,
                  const int* const* firstneigh, int neigh_full, int eflag, int vflag, double* f,

@@ -567,6 +567,7 @@ int finish_batch(mlip_ctx* c, int nstruct, const std::vector<int32_t>& soff, int
     if (!upload(c, c->soff, soff.data(), soff.size(), "structure offsets") || !c->sout.ensure(7 * nstruct))
         return MLIP_ERR_DEVICE;
     if (!hip_ok(c, hipStreamSynchronize(c->stream), "batch upload")) return MLIP_ERR_DEVICE;
+    c->lists = LammpsLists{};
     c->nstruct = nstruct;
     c->sbeg = c->soff.p;
     c->send = c->soff.p + 1;
@@ -916,7 +917,9 @@ int lammps_compute(mlip_ctx* c, int nlocal, int nghost, const double* x, const i
         epv = c->epv.p;
         evat = c->evat.p;
     }
-    return lammps_results(c, L.nall, inum, ilist, f, eng, virial, eatom, vatom, epv, evat);
+    const int rr = lammps_results(c, L.nall, inum, ilist, f, eng, virial, eatom, vatom, epv, evat);
+    L.trim();
+    return rr;
 }
 
 }  // namespace
@@ -951,6 +954,7 @@ int lammps_lists(mlip_ctx* c, int nlocal, int nghost, const double* x, const int
         }
         owner_of_local[ilist[ii]] = ii;
     }
+    L.local_of_tag.clear();
     // tags to local atoms: a table where the tags are as dense as LAMMPS makes
     // them (1 .. natoms), a map otherwise
     std::unordered_map<int64_t, int> local_of_far_tag;
@@ -1317,6 +1321,7 @@ int mlip_resident_set(mlip_ctx* c, int natoms, const double* x, const int* type,
                       gen))
         return MLIP_ERR_DEVICE;
     if (!hip_ok(c, hipStreamSynchronize(c->stream), "resident upload")) return MLIP_ERR_DEVICE;
+    c->lists = LammpsLists{};
     c->resident = true;
     c->resident_natoms = natoms;
     return MLIP_OK;
@@ -1469,6 +1474,7 @@ int mlip_resident_set_cell(mlip_ctx* c, int natoms, const double* cell9, const d
     const int rc = setup_cells_device(c, 1, &na, cell9, x, elem);
     if (rc != MLIP_OK) return rc;
     if (!hip_ok(c, hipStreamSynchronize(c->stream), "resident build")) return MLIP_ERR_DEVICE;
+    c->lists = LammpsLists{};
     c->resident = true;
     c->resident_natoms = natoms;
     return MLIP_OK;

@@ -11,6 +11,7 @@
 
 #include "../../include/mlip_hip.h"
 #include "device_api.h"
+#include "lammps_lists.h"
 #include "model.h"
 
 namespace mlip {
@@ -49,17 +50,6 @@ struct NbWork;  // device neighbor-build scratch (nbuild.hip)
 struct TrainWork;  // training-feature tables and outputs (train.hip)
 
 }  // namespace mlip
-
-// A LAMMPS-shaped neighbor list as the engine's pair and gather lists.  Kept in
-// the context from call to call for its memory: fresh vectors of a few megabytes
-// are page faults on every call.
-struct LammpsLists {
-    int nall = 0;
-    int64_t npairs = 0;
-    std::vector<double> x;
-    std::vector<int32_t> elem, elem_own, poff, pnbr, pcen, gof, gen;
-    std::vector<int32_t> owner_of_local, local_of_tag, fill;  // work space
-};
 
 struct mlip_ctx {
     LammpsLists lists;

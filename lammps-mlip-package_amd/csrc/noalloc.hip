@@ -179,5 +179,7 @@ extern "C" int mlip_compute_flat_noalloc(mlip_ctx* c, int nlocal, int nghost, co
                up(P.b.gent, L.gen.data(), L.gen.size() * sizeof(int32_t), "gather entries");
     };
     if (!run_pipeline(c, gather)) return MLIP_ERR_DEVICE;
-    return lammps_results(c, L.nall, inum, ilist, f, eng, virial, eatom, vatom, P.epv, P.evat);
+    rc = lammps_results(c, L.nall, inum, ilist, f, eng, virial, eatom, vatom, P.epv, P.evat);
+    L.trim();
+    return rc;
 }

@@ -474,6 +474,8 @@ int mlip_pool_init(mlip_ctx* c, int64_t max_atoms, int64_t max_pairs, int max_re
         return MLIP_ERR_ARG;
     pool_free(c);
     drop_graph(c);
+    (void)hipStreamSynchronize(c->stream);
+    c->lists = LammpsLists{};
     auto* p = new Pool();
     c->pool = p;
     const Model& m = c->model;
