@@ -203,7 +203,9 @@ int mlip_get_anlm_kernel(const mlip_ctx* ctx);
  * `reps` times on the current resident structure or batch with each, and
  * keeps the fastest; plan3 receives its two constants and the pairing limit
  * (-1: no paired rows).  Results do not depend on the plan beyond the
- * summation order of split rows and of the paired rows' products. */
+ * summation order of split rows and of the paired rows' products.  A model that
+ * gives this kernel no visits (order-3/4 families all outside the polynomial, or
+ * none) keeps its plan, and nothing is timed. */
 int mlip_autotune_q34(mlip_ctx* ctx, int reps, int* plan3);
 
 /* Sets the order-3/4 workgroup plan directly (the three values

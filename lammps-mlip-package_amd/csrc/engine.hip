@@ -1650,7 +1650,12 @@ int mlip_autotune_q34(mlip_ctx* c, int reps, int* plan2) {
         return MLIP_ERR_STATE;
     }
     Model& m = c->model;
-    if (!m.has_order34 || m.pair_model) {
+    // nothing to time where the order-3/4 kernel has no visits: models without
+    // those orders, and those whose families are all the order-3 and order-4
+    // products' (q3.hip)
+    bool visits = false;
+    for (const TypeTables& tt : m.types) visits = visits || !tt.plan_adj.empty();
+    if (!visits || !m.has_order34 || m.pair_model) {
         if (plan2) plan2[0] = m.plan_region, plan2[1] = m.plan_visit, plan2[2] = m.plan_pair;
         return MLIP_OK;
     }
