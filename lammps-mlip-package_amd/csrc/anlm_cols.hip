@@ -33,6 +33,8 @@
 // Reference: PairMLIPGtinv::compute_anlm (src/USER-MLIP/pair_mlip_gtinv.cpp:349-447).
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
+
 #include "device_api.h"
 #include "device_common.h"
 
@@ -58,7 +60,7 @@ struct Lds {
             T z[kBatch];
             T w[kBatch][2 * LT + 1];  // (-conj(u))^m, m < LT; odd pitch
         };
-        double buf[kColsBuf];         // a round of the epilogue
+        alignas(16) double buf[kColsBuf];  // a round of the epilogue, read as double2
     };
     double fw[kColsFeat][kQ12Weights];  // order-1/2 features of the centre's species: weights,
     uint32_t fd[kColsFeat];             // order | L | s0 | s1 in 4 bits each, column above
@@ -68,6 +70,8 @@ template <typename T, int LT, int NS>
 __global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(3))) void k_anlm_cols(DevModel M, DevSystem S,
                                                                                               int feat) {
     __shared__ Lds<T, LT> L;
+    using Shared = Lds<T, LT>;
+    static_assert(alignof(Shared) >= sizeof(double2) && offsetof(Shared, buf) == 0, "16-byte reads of buf");
     const int slot = xcd_slot(blockIdx.x, S.nblocks);
     if (slot < 0) return;
     const int atom = S.atom_of_slot[slot];
