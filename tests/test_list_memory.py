@@ -1,6 +1,6 @@
 """The host memory that a context keeps between LAMMPS calls follows the calls, and a
 context that goes on with a resident structure, a batch or a pool gives it back."""
-import os
+import ctypes
 
 import numpy as np
 import pytest
@@ -15,16 +15,23 @@ def test_kept_lists_follow_the_calls(tmp_path):
     host_checks.run(tmp_path, "lists_kept")
 
 
-def resident_bytes():
-    with open("/proc/self/statm") as f:
-        return int(f.read().split()[1]) * os.sysconf("SC_PAGE_SIZE")
+class _MallInfo(ctypes.Structure):
+    _fields_ = [(k, ctypes.c_size_t) for k in ("arena", "ordblks", "smblks", "hblks", "hblkhd", "usmblks", "fsmblks",
+                                               "uordblks", "fordblks", "keepcost")]
+
+
+def allocated_bytes():
+    """Bytes of the C library's heap in use (freed ones may stay in the process)."""
+    f = ctypes.CDLL(None).mallinfo2
+    f.restype = _MallInfo
+    m = f()
+    return m.uordblks + m.hblkhd
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("then", ["smaller call", "resident", "batch", "pool"])
 def test_memory_given_back(then):
-    # 12 million directed pairs (all but a few beyond the cutoff): 192 MB of lists,
-    # in arrays beyond what the C library keeps in its heap (32 MB)
+    # 12 million directed pairs (all but a few beyond the cutoff): 192 MB of lists
     n, per = 60000, 200
     k = np.arange(n, dtype=np.int32)
     x = np.zeros((n, 3))
@@ -39,7 +46,7 @@ def test_memory_given_back(then):
     small = W.build_neighbor_list(s, p.init_one(), full=True)
     p.compute(small, small.types)
     p.compute(nl, nl.types)
-    before = resident_bytes()
+    before = allocated_bytes()
     if then == "smaller call":
         p.compute(small, small.types)
     elif then == "resident":
@@ -48,6 +55,6 @@ def test_memory_given_back(then):
         BatchSystem(p, [s]).compute()
     else:
         RequestPool(p, 256, 65536, 1)
-    given = before - resident_bytes()
+    given = before - allocated_bytes()
     print("%s: %.0f MB given back" % (then, given / 1e6), flush=True)
     assert given >= 100e6
