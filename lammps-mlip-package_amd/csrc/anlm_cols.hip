@@ -294,8 +294,10 @@ bool anlm_cols_fits(const DevModel& m) { return m.cols != nullptr && m.maxl <= k
 
 // the features' tables, a round's a_nlm and two row segments fit the LDS
 bool anlm_cols_features(const DevModel& m) {
-    for (int t = 0; t < m.n_type; ++t)
-        if (m.fq12_off[t + 1] - m.fq12_off[t] > kColsFeat || m.prange[t][1] - m.prange[t][0] > 65535 || 4 * (2 * m.n_type * m.n_lmh + 2 * (m.prange[t][1] - m.prange[t][0])) > kColsBuf) return false;
+    for (int t = 0; t < m.n_type; ++t) {
+        const int features = m.fq12_off[t + 1] - m.fq12_off[t], w = m.prange[t][1] - m.prange[t][0];
+        if (features > kColsFeat || w > 65535 || 4 * (2 * m.n_type * m.n_lmh + 2 * w) > kColsBuf) return false;
+    }
     return true;
 }
 

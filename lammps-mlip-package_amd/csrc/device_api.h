@@ -59,7 +59,7 @@ struct DevModel {
     int lmax_t;             // largest l of the order-3/4 adjoint kernel's tile (lmax3: the feature kernel's)
     int has_q34;            // order-3/4 invariants present (k_q34 runs)
     int q12_fuse;           // order-1/2 adjoint rows L <= q12_fuse are the order-3/4 kernel's (-1: none)
-    int q12_fuse_hi;        // ... and the rows lmax3 < L <= q12_fuse_hi (a_nlm from HBM)
+    int q12_fuse_hi;        // ... and the rows lmax_t < L <= q12_fuse_hi (a_nlm from HBM)
     int q12_adj_levels;     // 1 if some level is left to the order-1/2 adjoint kernel (else it
                             // is not launched and its energies Eq12 are not read)
     double cutoff;

@@ -80,11 +80,5 @@ __device__ __forceinline__ PairDel pair_del(const DevModel& M, const DevSystem& 
     return g;
 }
 
-// compile-time constants as arguments
-template <int N>
-struct Const {
-    static constexpr int value = N;
-};
-
 }  // namespace dev
 }  // namespace mlip

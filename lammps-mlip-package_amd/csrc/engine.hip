@@ -519,8 +519,7 @@ bool setup_layout(mlip_ctx* c, int nall, int nown, int64_t npairs, const std::ve
 // Upload a structure with host-built lists and lay it out.
 bool setup_system(mlip_ctx* c, int nall, int nown, int64_t npairs, const std::vector<double>& x,
                   const std::vector<int32_t>& elem, const std::vector<int32_t>& elem_own,
-                  const std::vector<int32_t>& poff,
-                  const std::vector<int32_t>& pnbr, const std::vector<int32_t>* pcen,
+                  const std::vector<int32_t>& poff, const std::vector<int32_t>& pnbr,
                   const std::vector<double>* pshift, const std::vector<int32_t>& goff,
                   const std::vector<int32_t>& gent) {
     bool ok = upload(c, c->x, x.data(), x.size(), "positions") &&
@@ -530,9 +529,8 @@ bool setup_system(mlip_ctx* c, int nall, int nown, int64_t npairs, const std::ve
               upload(c, c->goff, goff.data(), goff.size(), "gather offsets") &&
               upload(c, c->gent, gent.data(), gent.size(), "gather entries");
     if (!ok) return false;
-    if (pcen && !upload(c, c->pcen, pcen->data(), pcen->size(), "pair centres")) return false;
     if (pshift && !upload(c, c->pshift, pshift->data(), pshift->size(), "pair shifts")) return false;
-    return setup_layout(c, nall, nown, npairs, elem_own, pcen != nullptr, pshift != nullptr);
+    return setup_layout(c, nall, nown, npairs, elem_own, false, pshift != nullptr);
 }
 
 // Structures from periodic cells with their lists built on the device
@@ -582,27 +580,33 @@ int finish_batch(mlip_ctx* c, int nstruct, const std::vector<int32_t>& soff, int
 namespace mlip {
 
 // Force gather lists: for every position k, the pairs whose centre (-) or
-// neighbor (+) is k, in increasing pair order.
-void build_gather(int nall, const std::vector<int32_t>& poff, const std::vector<int32_t>& pnbr,
-                  const std::vector<int32_t>* pcen, std::vector<int32_t>& goff, std::vector<int32_t>& gent) {
-    const int nown = static_cast<int>(poff.size()) - 1;
+// neighbor (+) is k, in increasing pair order (a self-image pair's centre entry
+// first).  cen(p): centre of pair p; fill: work space.
+template <typename F>
+void gather_lists(int nall, const std::vector<int32_t>& pnbr, F cen, std::vector<int32_t>& goff,
+                  std::vector<int32_t>& gent, std::vector<int32_t>& fill) {
     const size_t np = pnbr.size();
-    std::vector<int32_t> cnt(nall + 1, 0);
-    std::vector<int32_t> cen(np);
-    for (int o = 0; o < nown; ++o)
-        for (int p = poff[o]; p < poff[o + 1]; ++p) cen[p] = pcen ? (*pcen)[p] : o;
+    goff.assign(static_cast<size_t>(nall) + 1, 0);
     for (size_t p = 0; p < np; ++p) {
-        ++cnt[cen[p] + 1];
-        ++cnt[pnbr[p] + 1];
+        ++goff[cen(p) + 1];
+        ++goff[pnbr[p] + 1];
     }
-    goff.assign(nall + 1, 0);
-    for (int k = 0; k < nall; ++k) goff[k + 1] = goff[k] + cnt[k + 1];
-    gent.assign(goff[nall], 0);
-    std::vector<int32_t> fill(goff.begin(), goff.end() - 1);
+    for (int k = 0; k < nall; ++k) goff[k + 1] += goff[k];
+    gent.resize(2 * np);
+    fill.assign(goff.begin(), goff.end() - 1);
     for (size_t p = 0; p < np; ++p) {
-        gent[fill[cen[p]]++] = -static_cast<int32_t>(p + 1);
+        gent[fill[cen(p)]++] = -static_cast<int32_t>(p + 1);
         gent[fill[pnbr[p]]++] = static_cast<int32_t>(p + 1);
     }
+}
+
+// ... of lists without ghosts, pairs in centre order
+void build_gather(int nall, const std::vector<int32_t>& poff, const std::vector<int32_t>& pnbr,
+                  std::vector<int32_t>& goff, std::vector<int32_t>& gent) {
+    std::vector<int32_t> cen(pnbr.size()), fill;
+    for (size_t o = 0; o + 1 < poff.size(); ++o)
+        for (int p = poff[o]; p < poff[o + 1]; ++p) cen[p] = static_cast<int32_t>(o);
+    gather_lists(nall, pnbr, [&](size_t p) { return cen[p]; }, goff, gent, fill);
 }
 
 WorkSizes work_sizes(const Model& m, int nall, int nown, int64_t npairs, int nblocks) {
@@ -1061,19 +1065,7 @@ int lammps_lists(mlip_ctx* c, int nlocal, int nghost, const double* x, const int
 }
 
 void lammps_gather(LammpsLists& L) {
-    const size_t np = L.pnbr.size();
-    L.gof.assign(static_cast<size_t>(L.nall) + 1, 0);
-    for (size_t p = 0; p < np; ++p) {
-        ++L.gof[L.pcen[p] + 1];
-        ++L.gof[L.pnbr[p] + 1];
-    }
-    for (int k = 0; k < L.nall; ++k) L.gof[k + 1] += L.gof[k];
-    L.gen.resize(2 * np);
-    L.fill.assign(L.gof.begin(), L.gof.end() - 1);
-    for (size_t p = 0; p < np; ++p) {
-        L.gen[L.fill[L.pcen[p]]++] = -static_cast<int32_t>(p + 1);
-        L.gen[L.fill[L.pnbr[p]]++] = static_cast<int32_t>(p + 1);
-    }
+    gather_lists(L.nall, L.pnbr, [&](size_t p) { return L.pcen[p]; }, L.gof, L.gen, L.fill);
 }
 
 int lammps_results(mlip_ctx* c, int nall, int inum, const int* ilist, double* f, double* eng, double* virial,
@@ -1312,13 +1304,12 @@ int mlip_resident_set(mlip_ctx* c, int natoms, const double* x, const int* type,
             return MLIP_ERR_ARG;
         }
     std::vector<int32_t> gof, gen;
-    build_gather(natoms, poff, pnbr, nullptr, gof, gen);
+    build_gather(natoms, poff, pnbr, gof, gen);
     std::vector<double> xv(x, x + 3 * static_cast<size_t>(natoms));
     std::vector<double> sh;
     if (nbr_shift) sh.assign(nbr_shift, nbr_shift + 3 * npairs);
     c->nstruct = 0;
-    if (!setup_system(c, natoms, natoms, npairs, xv, elem, elem, poff, pnbr, nullptr, nbr_shift ? &sh : nullptr, gof,
-                      gen))
+    if (!setup_system(c, natoms, natoms, npairs, xv, elem, elem, poff, pnbr, nbr_shift ? &sh : nullptr, gof, gen))
         return MLIP_ERR_DEVICE;
     if (!hip_ok(c, hipStreamSynchronize(c->stream), "resident upload")) return MLIP_ERR_DEVICE;
     c->lists = LammpsLists{};
@@ -1439,9 +1430,9 @@ int mlip_batch_set(mlip_ctx* c, int nstruct, const int* natoms, const double* ce
         }
     }
     std::vector<int32_t> gof, gen;
-    build_gather(n, poff, pnbr, nullptr, gof, gen);
+    build_gather(n, poff, pnbr, gof, gen);
     std::vector<double> xv(x, x + 3 * static_cast<size_t>(n));
-    if (!setup_system(c, n, n, static_cast<int64_t>(pnbr.size()), xv, elem, elem, poff, pnbr, nullptr, &sh, gof, gen))
+    if (!setup_system(c, n, n, static_cast<int64_t>(pnbr.size()), xv, elem, elem, poff, pnbr, &sh, gof, gen))
         return MLIP_ERR_DEVICE;
     return finish_batch(c, nstruct, soff, n);
 }

@@ -189,7 +189,7 @@ int lammps_results(mlip_ctx* c, int nall, int inum, const int* ilist, double* f,
                    double* eatom, double* vatom, double* epv, double* evat);
 void collect_profile(mlip_ctx* c);
 void build_gather(int nall, const std::vector<int32_t>& poff, const std::vector<int32_t>& pnbr,
-                  const std::vector<int32_t>* pcen, std::vector<int32_t>& goff, std::vector<int32_t>& gent);
+                  std::vector<int32_t>& goff, std::vector<int32_t>& gent);
 void pool_free(mlip_ctx* c);
 // Full periodic lists (0 < r < rc, self-images, image shifts) of nstruct
 // structures whose positions (concatenated, natoms[s] each) are already in

@@ -248,7 +248,7 @@ __global__ __launch_bounds__(64) void k_q12(DevModel M, DevSystem S, int stage) 
 constexpr int kPolyLanes = 16;
 constexpr int kPolyThreads = 256;
 
-// STAGE: the slot's row fits the 64 KB of LDS a launch has by default (8,192
+// STAGE: the slot's row fits the 64 KB of LDS a launch has by default (8,188
 // features); else it is read from HBM
 template <bool STAGE>
 __global__ __launch_bounds__(kPolyThreads) void k_poly(DevModel M, DevSystem S) {

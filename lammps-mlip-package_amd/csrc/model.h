@@ -282,8 +282,8 @@ struct Model {
     // the same derivatives as one dense product per centre species t where
     // the lists fill it: columns a = s n_fn + n (its features by neighbor
     // species s, nf = n_type n_fn of them, padded to 16), rows = the factors
-    // d_b (kd2 rows, the quadratic terms), then the products d_b d_c, b <= c
-    // (the cubic ones), each part padded to 4 rows; pd_bc holds b | c << 16
+    // d_b (pd_k2 rows, the quadratic terms), then the products d_b d_c, b <= c
+    // (pd_k3, the cubic ones), each part padded to 4 rows; pd_bc holds b | c << 16
     // per row (index nf: the factor 1)
     int pd_k2 = 0, pd_k3 = 0, pd_cols = 0;         // pd_cols = 0: lists only
     std::vector<int32_t> pd_bc;

@@ -381,18 +381,19 @@ __global__ __launch_bounds__(NTH) void k_anlm(DevModel M, DevSystem S, int ngrou
 // species' accumulators (two for the step that straddles the boundary, with
 // the other species' columns masked to zero) and no lane branches on species.
 // One workgroup of four waves per centre; wave w owns the column tiles
-// w, w + 4, ... and both species' accumulators for them (MT tiles of 16 radial
-// indices each).  Per-pair geometry, g_n and Y_lm are computed as in k_anlm
+// w, w + 4, ... and both species' accumulators for them (kAmRows tiles of 16
+// radial indices each).  Per-pair geometry, g_n and Y_lm are computed as in k_anlm
 // (radial functions in FP64, Y_lm in T); the product and its accumulation
 // are FP64.
 constexpr int kAmThreads = 256;
 constexpr int kAmJ = 16;
+constexpr int kAmRows = 2;
 
-template <typename T, int MT, int NTW>
+template <typename T, int NTW>
 struct AmLds {
     static constexpr int kCols = 64 * NTW;      // 4 waves x NTW tiles x 16 columns
     static constexpr int kYPitch = kCols + 2;   // doubles; offsets the rows' banks
-    static constexpr int kAPitch = 16 * MT + 2;
+    static constexpr int kAPitch = 16 * kAmRows + 2;
     T diag[kSmallL1 + 1];
     T alm[kSmallL1][kSmallL1];
     T ainv[kSmallL1][kSmallL1];
@@ -404,9 +405,9 @@ struct AmLds {
     alignas(16) double Y[kAmJ][kYPitch];    // [sorted neighbor][(lm, re/im)]
 };
 
-template <typename T, int MT, int NTW>
+template <typename T, int NTW>
 __global__ __launch_bounds__(kAmThreads) void k_anlm_mfma(DevModel M, DevSystem S) {
-    using L_t = AmLds<T, MT, NTW>;
+    using L_t = AmLds<T, NTW>;
     constexpr int kCols = L_t::kCols;
     __shared__ L_t L;
     const int slot = xcd_slot(blockIdx.x, S.nblocks);
@@ -431,11 +432,11 @@ __global__ __launch_bounds__(kAmThreads) void k_anlm_mfma(DevModel M, DevSystem 
         for (int k = tid; k < kAmJ * kCols; k += kAmThreads) L.Y[k / kCols][k % kCols] = 0.0;
     }
     typedef double dbl4 __attribute__((ext_vector_type(4)));
-    dbl4 acc[2][MT][NTW];
+    dbl4 acc[2][kAmRows][NTW];
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+        for (int i = 0; i < kAmRows; ++i)
 #pragma unroll
             for (int t = 0; t < NTW; ++t) acc[s][i][t] = dbl4{0.0, 0.0, 0.0, 0.0};
     const int p0 = S.poff[atom], p1 = S.pend[atom];
@@ -476,7 +477,7 @@ __global__ __launch_bounds__(kAmThreads) void k_anlm_mfma(DevModel M, DevSystem 
                 const int k = sp == 0 ? __popcll(m0 & below) : (sp == 1 ? n0 + __popcll(m1 & below) : -1);
                 if (k >= 0) {
                     const double r = L.rr[q], fcq = L.fc[q];
-                    for (int n = part; n < 16 * MT; n += 16) {
+                    for (int n = part; n < 16 * kAmRows; n += 16) {
                         const double d = n < nfn ? r - L.mu[n] : 0.0;
                         L.At[k][n] = n < nfn ? exp(-L.beta[n] * (d * d)) * fcq : 0.0;
                     }
@@ -511,8 +512,8 @@ __global__ __launch_bounds__(kAmThreads) void k_anlm_mfma(DevModel M, DevSystem 
                     }
                 }
                 // rows past the chunk's valid neighbors are zero
-                for (int e = tid; e < (kAmJ - nval) * 16 * MT; e += kAmThreads)
-                    L.At[nval + e / (16 * MT)][e % (16 * MT)] = 0.0;
+                for (int e = tid; e < (kAmJ - nval) * 16 * kAmRows; e += kAmThreads)
+                    L.At[nval + e / (16 * kAmRows)][e % (16 * kAmRows)] = 0.0;
                 for (int e = tid; e < (kAmJ - nval) * 2 * nlmh; e += kAmThreads)
                     L.Y[nval + e / (2 * nlmh)][e % (2 * nlmh)] = 0.0;
             }
@@ -523,9 +524,9 @@ __global__ __launch_bounds__(kAmThreads) void k_anlm_mfma(DevModel M, DevSystem 
                 if (kb >= nval) break;
                 const int kr = kb + (lane >> 4);
                 const bool s0 = kb < n0, s1 = kb + 3 >= n0;  // species present in the step
-                double a0[MT], a1[MT];
+                double a0[kAmRows], a1[kAmRows];
 #pragma unroll
-                for (int i = 0; i < MT; ++i) {
+                for (int i = 0; i < kAmRows; ++i) {
                     const double a = L.At[kr][16 * i + (lane & 15)];
                     a0[i] = kr < n0 ? a : 0.0;
                     a1[i] = kr < n0 ? 0.0 : a;
@@ -534,7 +535,7 @@ __global__ __launch_bounds__(kAmThreads) void k_anlm_mfma(DevModel M, DevSystem 
                 for (int t = 0; t < NTW; ++t) {
                     const double b = L.Y[kr][(wave * NTW + t) * 16 + (lane & 15)];
 #pragma unroll
-                    for (int i = 0; i < MT; ++i) {
+                    for (int i = 0; i < kAmRows; ++i) {
                         if (s0) acc[0][i][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[i], b, acc[0][i][t], 0, 0, 0);
                         if (s1) acc[1][i][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[i], b, acc[1][i][t], 0, 0, 0);
                     }
@@ -548,7 +549,7 @@ __global__ __launch_bounds__(kAmThreads) void k_anlm_mfma(DevModel M, DevSystem 
     for (int s = 0; s < 2; ++s) {
         if (s >= M.n_type) break;
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+        for (int i = 0; i < kAmRows; ++i)
 #pragma unroll
             for (int t = 0; t < NTW; ++t) {
                 const int col = (wave * NTW + t) * 16 + (lane & 15);
@@ -575,13 +576,13 @@ __global__ __launch_bounds__(kAmThreads) void k_anlm_mfma(DevModel M, DevSystem 
 //   singular terms cancel to c Q' (z x, z y, -(1-z^2)).
 constexpr int kForceThreads = 128;
 
-template <typename T, int KL1>
+template <typename T>
 struct ForceLds {
     double beta[kMaxFn], mu[kMaxFn];
-    T diag[KL1 + 1];
-    T alm[KL1][KL1];
-    T ainv[KL1][KL1];
-    T grad[KL1][KL1];
+    T diag[kL1 + 1];
+    T alm[kL1][kL1];
+    T ainv[kL1][kL1];
+    T grad[kL1][kL1];
     double trig[kTrigN + 1];  // sin / cos series coefficients, then pi / r_c
 };
 
@@ -592,12 +593,12 @@ struct ForceLds {
 // from HBM instead (GL = false; every thread of the workgroup reads the same
 // entries, served by the caches), and models with more than 16 radial functions
 // keep the register arrays they need (no occupancy cap).
-template <int NF, int NT, typename T, bool GL, int KL1>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NF > 16 ? 1 : (sizeof(T) == 4 ? 4 : 3)))) void k_force(DevModel M, DevSystem S) {
+template <int NF, typename T, bool GL>
+__global__ __launch_bounds__(kForceThreads) __attribute__((amdgpu_waves_per_eu(NF > 16 ? 1 : (sizeof(T) == 4 ? 4 : 3)))) void k_force(DevModel M, DevSystem S) {
     extern __shared__ __attribute__((aligned(16))) unsigned char force_dyn[];
     T* Gs = reinterpret_cast<T*>(force_dyn);  // [ns][n_lmh][NF][2]
-    __shared__ ForceLds<T, KL1> C;
-    __shared__ double vred[6][NT / 64];
+    __shared__ ForceLds<T> C;
+    __shared__ double vred[6][kForceThreads / 64];
     const int slot = xcd_slot(blockIdx.x, S.nblocks);
     if (slot < 0) return;
     const int atom = S.atom_of_slot[slot];
@@ -608,7 +609,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NF > 16 ? 1 
     // n >= n_fn read an in-range entry and store zero), so that their HBM /
     // L2 reads are in flight together
 #pragma unroll 4
-    for (int k = threadIdx.x; GL && k < ns * nlmh * NF; k += NT) {
+    for (int k = threadIdx.x; GL && k < ns * nlmh * NF; k += kForceThreads) {
         const int n = k % NF;
         const int lm = (k / NF) % nlmh;
         const int s = k / (NF * nlmh);
@@ -620,13 +621,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NF > 16 ? 1 
     }
     {
         const YTab<T>* yt = ytab_of<T>(M);
-        for (int k = threadIdx.x; k < KL1 * KL1; k += NT) {
-            const int l = k / KL1, mm = k % KL1;
+        for (int k = threadIdx.x; k < kL1 * kL1; k += kForceThreads) {
+            const int l = k / kL1, mm = k % kL1;
             C.alm[l][mm] = yt->alm[l][mm];
             C.ainv[l][mm] = yt->ainv[l][mm];
             C.grad[l][mm] = yt->grad[l][mm];
         }
-        if (threadIdx.x <= KL1) C.diag[threadIdx.x] = yt->diag[threadIdx.x];
+        if (threadIdx.x <= kL1) C.diag[threadIdx.x] = yt->diag[threadIdx.x];
         if (threadIdx.x < kTrigN) C.trig[threadIdx.x] = trig_coef(threadIdx.x);
         if (threadIdx.x == kTrigN) C.trig[kTrigN] = kPiRef / M.cutoff;
         if (threadIdx.x < kMaxFn) {
@@ -637,7 +638,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NF > 16 ? 1 
     __syncthreads();
     const int p0 = S.poff[atom], p1 = S.pend[atom];
     double v0 = 0, v1 = 0, v2 = 0, v3 = 0, v4 = 0, v5 = 0;
-    for (int64_t p = p0 + threadIdx.x; p < p1; p += NT) {
+    for (int64_t p = p0 + threadIdx.x; p < p1; p += kForceThreads) {
         const PairDel pg = pair_del(M, S, atom, p);
         double fx = 0.0, fy = 0.0, fz = 0.0;
         double ex = pg.dx, ey = pg.dy, ez = pg.dz;  // del for the virial
@@ -836,7 +837,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NF > 16 ? 1 
     __syncthreads();
     if (threadIdx.x < 6) {
         double s = 0.0;
-        for (int k = 0; k < NT / 64; ++k) s += vred[threadIdx.x][k];
+        for (int k = 0; k < kForceThreads / 64; ++k) s += vred[threadIdx.x][k];
         S.vown[6 * atom + threadIdx.x] = s;
     }
 }
@@ -972,10 +973,10 @@ hipError_t launch_anlm_nth(const DevModel& m, const DevSystem& s, int npt, int n
     return launched();
 }
 
-template <typename T, int MT, int NTW>
+template <typename T, int NTW>
 hipError_t launch_anlm_mfma_k(const DevModel& m, const DevSystem& s, hipStream_t st) {
-    if (sizeof(AmLds<T, MT, NTW>) > lds_limit()) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((k_anlm_mfma<T, MT, NTW>), dim3(slot_grid(s)), dim3(kAmThreads), 0, st, m, s);
+    if (sizeof(AmLds<T, NTW>) > lds_limit()) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL((k_anlm_mfma<T, NTW>), dim3(slot_grid(s)), dim3(kAmThreads), 0, st, m, s);
     return launched();
 }
 
@@ -990,9 +991,9 @@ bool anlm_mfma_fits(const DevModel& m) {
 template <typename T>
 hipError_t launch_anlm_mfma_t(const DevModel& m, const DevSystem& s, hipStream_t st) {
     const int ntw = ((2 * m.n_lmh + 15) / 16 + 3) / 4;
-    if (ntw == 1) return launch_anlm_mfma_k<T, 2, 1>(m, s, st);
-    if (ntw == 2) return launch_anlm_mfma_k<T, 2, 2>(m, s, st);
-    return launch_anlm_mfma_k<T, 2, 3>(m, s, st);
+    if (ntw == 1) return launch_anlm_mfma_k<T, 1>(m, s, st);
+    if (ntw == 2) return launch_anlm_mfma_k<T, 2>(m, s, st);
+    return launch_anlm_mfma_k<T, 3>(m, s, st);
 }
 
 template <typename T>
@@ -1007,43 +1008,42 @@ hipError_t launch_anlm_t(const DevModel& m, const DevSystem& s, int feat, hipStr
     return launch_anlm_nth<256, T, kL1, kLargeGW>(m, s, npt, ngroup, passes, feat, st);
 }
 
-template <int NF, int NT, typename T, bool GL, int KL1>
+template <int NF, typename T, bool GL>
 hipError_t launch_force_k(const DevModel& m, const DevSystem& s, hipStream_t st) {
     const size_t lds = GL ? sizeof(T) * 2 * m.n_type * m.n_lmh * NF : 0;
-    if (lds + sizeof(ForceLds<T, KL1>) + sizeof(double) * 6 * (NT / 64) > lds_limit())
+    if (lds + sizeof(ForceLds<T>) + sizeof(double) * 6 * (kForceThreads / 64) > lds_limit())
         return hipErrorInvalidConfiguration;
     if (GL) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_force<NF, NT, T, GL, KL1>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_force<NF, T, GL>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((k_force<NF, NT, T, GL, KL1>), dim3(slot_grid(s)), dim3(NT), lds, st, m, s);
+    hipLaunchKernelGGL((k_force<NF, T, GL>), dim3(slot_grid(s)), dim3(kForceThreads), lds, st, m, s);
     return launched();
 }
 
 // G tile staged in LDS when it fits beside the kernel's static LDS
-template <typename T, int KL1>
-bool force_tile_fits(const DevModel& m, int nf, int nt) {
+template <typename T>
+bool force_tile_fits(const DevModel& m, int nf) {
     const size_t lds = sizeof(T) * 2 * m.n_type * m.n_lmh * nf;
-    return lds + sizeof(ForceLds<T, KL1>) + sizeof(double) * 6 * (nt / 64) <= lds_limit();
+    return lds + sizeof(ForceLds<T>) + sizeof(double) * 6 * (kForceThreads / 64) <= lds_limit();
 }
 
 // G staged in LDS where it fits (GL)
 template <typename T, bool GL>
 hipError_t launch_force_gl(const DevModel& m, const DevSystem& s, hipStream_t st) {
-    if (m.n_fn <= 4) return launch_force_k<4, kForceThreads, T, GL, kL1>(m, s, st);
-    if (m.n_fn <= 8) return launch_force_k<8, kForceThreads, T, GL, kL1>(m, s, st);
-    if (m.n_fn <= 12) return launch_force_k<12, kForceThreads, T, GL, kL1>(m, s, st);
-    if (m.n_fn <= 16) return launch_force_k<16, kForceThreads, T, GL, kL1>(m, s, st);
-    if (m.n_fn <= 24) return launch_force_k<24, kForceThreads, T, GL, kL1>(m, s, st);
-    return launch_force_k<32, kForceThreads, T, GL, kL1>(m, s, st);
+    if (m.n_fn <= 4) return launch_force_k<4, T, GL>(m, s, st);
+    if (m.n_fn <= 8) return launch_force_k<8, T, GL>(m, s, st);
+    if (m.n_fn <= 12) return launch_force_k<12, T, GL>(m, s, st);
+    if (m.n_fn <= 16) return launch_force_k<16, T, GL>(m, s, st);
+    if (m.n_fn <= 24) return launch_force_k<24, T, GL>(m, s, st);
+    return launch_force_k<32, T, GL>(m, s, st);
 }
 
 template <typename T>
 hipError_t launch_force_t(const DevModel& m, const DevSystem& s, hipStream_t st) {
     const int nf = m.n_fn <= 16 ? (m.n_fn + 3) / 4 * 4 : m.n_fn <= 24 ? 24 : 32;
-    return force_tile_fits<T, kL1>(m, nf, kForceThreads) ? launch_force_gl<T, true>(m, s, st)
-                                                        : launch_force_gl<T, false>(m, s, st);
+    return force_tile_fits<T>(m, nf) ? launch_force_gl<T, true>(m, s, st) : launch_force_gl<T, false>(m, s, st);
 }
 
 }  // namespace

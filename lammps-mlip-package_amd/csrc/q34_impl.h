@@ -2,7 +2,8 @@
 // (FEAT = true) or the adjoint G = dE/da (FEAT = false).
 //
 // Workgroup = kWavesPerWg waves on one (block of 64 same-type centres,
-// radial index n).  The a_nlm tile (l <= lmax3, both species) sits in LDS as
+// radial index n).  The a_nlm tile (both species, l <= lmax3 for the features,
+// l <= lmax_t, the visits left to this kernel, for the adjoint) sits in LDS as
 // [s][lm][lane](re, im); each wave owns (S, L) output groups (or balanced
 // parts of heavy ones) and keeps G_{S,L,m<=0} in registers.  For L <=
 // kPairMaxL the rows of both species form one group, whose visits common

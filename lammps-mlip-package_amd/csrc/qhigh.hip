@@ -67,8 +67,9 @@ __global__ __launch_bounds__(64) void k_qhigh(DevModel M, DevSystem S) {
 #pragma unroll
         for (int k = 0; k <= kMaxLHi; ++k) gr[k] = gi[k] = 0.0;
         // the factors' (species, l) of the visit in one scalar: indexed in the record
-        // they are a read of scratch memory per term and factor (864 atoms, all 1,090
-        // order-5/6 visits in the polynomial: 51.4 + 7.8 ms, now 38.8 + 6.1)
+        // they are a read of scratch memory per term and factor (864 atoms, two
+        // species, orders 5 and 6 to l = 1 in the polynomial, 2 functions: adjoint
+        // 51.4 and features 7.8 ms, now 38.8 and 6.1)
         static_assert(kMaxOrderGpu - 1 <= 5, "twelve bits each");
         uint64_t factors = 0;
 #pragma unroll

@@ -392,7 +392,9 @@ __global__ __launch_bounds__(kTrThreads) void k_tr_dirj(DevModel M, DevSystem S,
 
 // LDS bytes of a launch shape, and the shape for a model: 128 features and 16
 // pairs per workgroup where the tables leave two workgroups per CU, fewer as
-// l_max grows (B takes n_type kp 8 bytes per feature, a pair 32 kp).
+// l_max grows (B takes n_type kp 8 bytes per feature, a pair 32 kp), down to 16
+// and 4, which is taken even where only one workgroup then fits (two species at
+// l_max 12).
 size_t tr_lds(const DevModel& m, const TrShape& h) {
     return sizeof(double) * (static_cast<size_t>(2) * h.nrow * m.n_type * m.n_lmh +
                              static_cast<size_t>(m.n_type) * h.kp * h.F + static_cast<size_t>(h.pairs) * 4 * h.ypitch());
