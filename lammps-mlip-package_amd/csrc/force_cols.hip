@@ -23,7 +23,8 @@
 //
 // Bound: the FP64 pipe (vector and matrix instructions share it; 84 products of
 // 64 cycles and ~700 vector instructions per tile at l_max 12 and 12 functions).
-// 256k atoms (137 neighbors, l_max 12, 12 functions): 11.2 ms, the pipe 89% busy;
+// 256k atoms (137 neighbors, l_max 12, 12 functions): 11.2 ms, matrix instructions
+// busy 50 % and vector issue 33 % of the SIMD cycles;
 // 3,991 atoms 202 us; mixed, 31k atoms: 0.96 ms.  Before: a thread per pair with G
 // read as LDS broadcasts (bound by them: one 16-byte read per four FMAs), 14.9 ms,
 // 293 us and 1.29 ms.  No spill is affordable here: with 464 bytes of scratch per

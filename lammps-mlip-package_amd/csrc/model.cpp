@@ -653,8 +653,7 @@ void plan_order3(Model& m, TypeTables& tt, const std::vector<Entry3>& en) {
         }
     // Cut the sequence of records into twelve ranges.  The three waves of a SIMD
     // issue oldest first, so with ranges of equal cost they end one after the other
-    // (119-132, 137-156 and 163-185 thousand cycles) and the last runs alone;
-    // shares of 112 : 104 : 84 took the order-3/4 pass of 256k atoms from 18.2 to
+    // and the last runs alone; shares of 112 : 104 : 84 took the order-3/4 pass of 256k atoms from 18.2 to
     // 17.1 ms (115 : 100 : 85 the same, 125 : 100 : 75 18.3).
     static_assert(kWavesPerWg == 12, "three waves a SIMD");
     constexpr long kShare[3] = {112, 104, 84};

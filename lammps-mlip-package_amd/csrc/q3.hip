@@ -28,10 +28,8 @@
 // 5,500 products of 4, and 16,000 coefficient FMA pairs.  At 256k atoms orders 1-4
 // took 36.4 ms as one visit per (family, factor position) with 3/4 of the
 // instructions address, descriptor and product work; k_q3 takes 15.6 ms and k_q4
-// 1.5 ms.  Of a workgroup's 220 thousand cycles 15 go to the tile (the
-// workgroups of a launch keep in step, so all read HBM at once), 165 to the
-// records, 13 to the rows above the tile and 10 to the divided segments; with the
-// factors' addresses formed from m in each step and the divided rows read and
+// 1.5 ms (vector issue 57 % of the SIMD cycles, the waves wait half of theirs); with
+// the factors' addresses formed from m in each step and the divided rows read and
 // written one by one it was 18.2 ms.
 #include <hip/hip_runtime.h>
 
